@@ -67,6 +67,7 @@ PER_FILE_FLAGS = {
     "hs_prefill_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true",
                             "-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],
     "hs_decode_gqa.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
+    "hs_prefill_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
     "hs_decode_splitmm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
 }
 

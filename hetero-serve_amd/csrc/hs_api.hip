@@ -587,6 +587,9 @@ static int prefill_common(const float* q, const int32_t* cu_q, int S, int max_ro
   a.splits = 1;
   a.P = 1;
   a.qscale = scale * kLog2e;
+  int dev = 0;
+  if (rows_prefill_serves(a, kv_dtype, D) && hipGetDevice(&dev) == hipSuccess)
+    return launch_rows_prefill(a, kv_dtype, D, std::max(1, device_cu_count(dev)), st);
   return launch_row_attn(a, kv_dtype, D, st);
 }
 

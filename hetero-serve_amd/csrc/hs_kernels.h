@@ -150,6 +150,14 @@ int launch_kv_append(void* k_cache, void* v_cache, int kv_dtype, int NB, int BS,
                      const int32_t* seq_ids, int64_t n, const void* k_src, const void* v_src,
                      int src_dtype, int64_t src_row_stride, hipStream_t stream);
 
+// Causal prefill in fp32 arithmetic on the fp32 matrix cores
+// (hs_prefill_rows.hip): a.S rows per sequence, or with a.cu_q ragged rows, at
+// most a.S per sequence, on a device of `cus` CUs.  `serves` is false for sizes
+// that its 32-bit offsets and positions cannot hold (a cache of 256 GiB, a table
+// of 2^30 tokens); launch_row_attn's one wave per row takes those.
+bool rows_prefill_serves(const RowAttnArgs& a, int kv_dtype, int D);
+int launch_rows_prefill(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream);
+
 // Matrix-core causal prefill (hs_prefill_mfma.hip).  cu_q null: S rows per
 // sequence, q/out [B, S, H, D]; else ragged rows as in hs_prefill_varlen.
 int launch_prefill_mfma(const float* q, const int32_t* cu_q, int S, int max_rows_per_seq,

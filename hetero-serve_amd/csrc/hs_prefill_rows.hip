@@ -1,0 +1,504 @@
+// Causal chunked prefill in fp32 arithmetic on gfx950's fp32 matrix cores.
+//
+// Reference: paged_attention_prefill_kernel,
+// heteroserve/model/paged_attn_prefill.py:72-157 (query s of a chunk sits at
+// position ctx - S + s and attends to keys [0, that position]; rows at
+// negative positions are zero).  This is hs_prefill*'s use_mfma = 0 path: any
+// cache dtype, any block size, head dims 32 to 256, nothing rounded below
+// fp32 anywhere.
+//
+// What bounds it.  The products run on v_mfma_f32_16x16x4_f32 (64 FLOPs a
+// cycle and SIMD, 157 TFLOP/s over the device at 2.4 GHz), whose 32 cycles
+// each leave room for everything else: the softmax, the LDS reads and the
+// loads of a 16-key tile take a fraction of its products' time.  The row
+// kernel that this one replaced gave every (query, head) a wave of its own,
+// which read all the keys of its row again and reduced every score over 16
+// lanes.
+//
+// Work decomposition.  A workgroup owns 16 * NT rows of one (sequence, KV
+// head), a row being a (query, head of the group) pair with the queries
+// outermost, so a short chunk of grouped heads still fills the tiles.  Its W
+// waves take the 16-key tiles in turn and combine their softmax states
+// through LDS at the end: the key split, and not a second query tile, is what
+// gives a small chunk enough waves.  Per tile and wave:
+//   S^T = K . Q^T    K staged in the wave's own LDS as fp32 (coalesced loads,
+//                    one tile ahead), lane (row j = l % 16, group g = l / 16)
+//                    reading dims g D/4 .. of key j; Q^T from LDS the same way
+//   O^T += V^T . P^T V^T straight from global memory: lane (j, g) loads the
+//                    D/16 values of key 4 g + i that are rows j of the
+//                    output tiles, 16 lanes a whole head row, and the S^T
+//                    accumulator is P^T's operand layout as it stands
+// The waves share nothing in the loop, so it has no barriers.  Rows of one
+// (sequence, KV head) are dealt heaviest first.
+//
+// Masked keys.  A score that a row does not see is -inf and its probability
+// 0, but 0 times an infinite or NaN value is NaN in a matrix product, and a
+// row must not see values past its own position.  Tiles in which some row
+// masks some key therefore look at their V values, and one with a non-finite
+// value adds its keys one by one, to the rows that see them.
+#include "hs_kernels.h"
+
+namespace hs {
+
+namespace {
+
+typedef float float4x __attribute__((ext_vector_type(4)));
+
+constexpr int kKeys = 16;            // keys of a tile (MFMA M), and rows of a row tile (MFMA N)
+constexpr float kRowsSlack = 8.0f;   // lazy raise of the running max, log2 units
+
+struct RowsArgs {
+  RowAttnArgs a;
+  int n_tiles;    // row tiles per (sequence, KV head) in the grid
+  int bs_shift;   // log2(BS), or -1
+  int reversed;   // the first workgroups, taken in reverse
+};
+
+// N 32-bit words of consecutive bytes, loaded at once.
+template <int N>
+struct Words {
+  uint32_t w[N];
+};
+
+template <int N>
+__device__ inline Words<N> load_words(const void* p) {
+  typedef unsigned int vec __attribute__((ext_vector_type(N)));
+  typedef vec vec_u __attribute__((aligned(4)));
+  const vec x = *reinterpret_cast<const vec_u*>(p);
+  Words<N> r;
+#pragma unroll
+  for (int i = 0; i < N; ++i) r.w[i] = x[i];
+  return r;
+}
+
+template <>
+__device__ inline Words<1> load_words<1>(const void* p) {
+  return Words<1>{{*reinterpret_cast<const uint32_t*>(p)}};
+}
+
+// Element e of the words, widened to fp32 (exact).
+template <typename T, int N>
+__device__ inline float word_elem(const Words<N>& x, int e) {
+  if constexpr (sizeof(T) == 4) {
+    return __uint_as_float(x.w[e]);
+  } else {
+    float f[2];
+    Elem<T>::pair(x.w[e >> 1], f);
+    return f[e & 1];
+  }
+}
+
+__device__ inline float max_over_groups(float x) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+__device__ inline float sum_over_groups(float x) {
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Orders a wave's LDS writes before its later LDS reads for the compiler (the
+// hardware keeps a wave's LDS operations in order).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The rows of row tile `tile` of (sequence b, KV head kvh); every thread of the
+// workgroup calls it (it holds barriers).
+template <typename T, int D, int NT, int W>
+__device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
+  const RowAttnArgs& a = ra.a;
+  constexpr int kRows = kKeys * NT;
+  constexpr int kRow = D + 4;                    // floats of a staged row: 16-byte reads of 16
+                                                 // rows fall on 16 different bank quads
+  constexpr int kVec = Elem<T>::kVec;            // elements of a 16-byte load
+  constexpr int kLpr = D / kVec;                 // K loads: lanes per token
+  constexpr int kTpl = 64 / kLpr;                // tokens per load
+  constexpr int kLi = kKeys / kTpl;              // loads per tile
+  constexpr int kDT = D / 16;                    // output tiles, and V values per lane and key
+  constexpr int kVE = kDT < kVec ? kDT : kVec;   // V values of one load
+  constexpr int kNV = kDT / kVE;                 // V loads per key
+  constexpr int kVW = kVE * (int)sizeof(T) / 4;  // words of one V load
+  static_assert(kLi >= 1 && kTpl * kLi == kKeys && kVW >= 1, "head_dim");
+
+  __shared__ __align__(16) float ks[W][kKeys][kRow];
+  __shared__ __align__(16) float qs[kRows][kRow];
+  __shared__ float wave_m[W][kRows], wave_l[W][kRows], inv_l[kKeys];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar: the tile loop is too
+  const int j = lane & 15;
+  const int g = lane >> 4;
+
+  // ---- the rows of this workgroup (everything here is workgroup-uniform) ----
+  const int G = a.H / a.Hkv;
+  const int row0 = a.cu_q ? a.cu_q[b] : b * a.S;
+  const int S_b = a.cu_q ? a.cu_q[b + 1] - row0 : a.S;
+  const int n_rows = S_b * G;                     // the launcher keeps S * G within 31 bits
+  const int r_first = tile * kRows;
+  const int64_t cap = (int64_t)a.MB * a.BS;
+  const int64_t base = (int64_t)a.ctx[b] - S_b;   // position of query 0
+  auto query_of = [&](int r) { return G == 1 ? r : (int)((uint32_t)r / (uint32_t)G); };
+  auto row_end = [&](int r) -> int {              // keys row r sees: [0, row_end)
+    const int64_t e = base + query_of(r) + 1;
+    return (int)max((int64_t)0, min(e, cap));
+  };
+  auto out_row = [&](int r) -> int64_t {          // element offset of row r in q and out
+    const int s = query_of(r);
+    return (((int64_t)row0 + s) * a.H + kvh * G + (r - s * G)) * D;
+  };
+  const int hi = row_end(min(r_first + kRows, n_rows) - 1);   // rows see more keys as r grows
+  const int seen_by_all = row_end(r_first);
+  if (hi <= 0) {
+    for (int i = tid; i < kRows * (D / 4); i += 64 * W) {
+      const int r = r_first + i / (D / 4);
+      if (r < n_rows)
+        *reinterpret_cast<float4*>(a.out + out_row(r) + 4 * (i % (D / 4))) =
+            make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    return;
+  }
+
+  // ---- the tiles of this wave: wv, wv + W, ... ------------------------------
+  const int n_kt = (hi + kKeys - 1) / kKeys;
+  const int32_t* bt = a.bt + (int64_t)b * a.MB;
+  const uint32_t tok_units = (uint32_t)(a.Hkv * (D * (int)sizeof(T) / 64));   // 64-byte units
+  const char* kbase = static_cast<const char*>(a.k) + (int64_t)kvh * D * (int)sizeof(T) +
+                      (lane % kLpr) * 16;
+  const char* vbase = static_cast<const char*>(a.v) +
+                      ((int64_t)kvh * D + kVE * j) * (int)sizeof(T);
+  // Where key 16 n + j lies in the cache, in 64-byte units (a key past the last
+  // is read as the last).  The launcher keeps the cache within 32 bits of them.
+  auto slot_of = [&](int n) -> uint32_t {
+    const int t = min(n * kKeys + j, hi - 1);
+    const int blk = ra.bs_shift >= 0 ? t >> ra.bs_shift : t / a.BS;
+    return ((uint32_t)safe_block(bt[blk], a.NB) * (uint32_t)a.BS + (uint32_t)(t - blk * a.BS)) *
+           tok_units;
+  };
+  uint4 kr[kLi];
+  Words<kVW> vr[4][kNV];
+  auto load_k = [&](uint32_t slots) {
+#pragma unroll
+    for (int u = 0; u < kLi; ++u) {
+      const uint32_t s = __shfl(slots, u * kTpl + lane / kLpr);
+      kr[u] = load16(kbase + ((uint64_t)s << 6));
+    }
+  };
+  auto load_v = [&](uint32_t slots) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t s = __shfl(slots, 4 * g + i);
+      const char* p = vbase + ((uint64_t)s << 6);
+#pragma unroll
+      for (int u = 0; u < kNV; ++u)
+        vr[i][u] = load_words<kVW>(p + u * 16 * kVE * (int)sizeof(T));
+    }
+  };
+
+  uint32_t next_slots = 0;
+  if (wv < n_kt) {
+    const uint32_t slots = slot_of(wv);
+    next_slots = slot_of(wv + W);
+    load_k(slots);
+    load_v(slots);
+  }
+
+  // ---- queries into LDS, scaled; rows past the last are zero ----------------
+  for (int i = tid; i < kRows * (D / 4); i += 64 * W) {
+    const int r = r_first + i / (D / 4);
+    float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (r < n_rows) {
+      x = *reinterpret_cast<const float4*>(a.q + out_row(r) + 4 * (i % (D / 4)));
+      x = make_float4(x.x * a.qscale, x.y * a.qscale, x.z * a.qscale, x.w * a.qscale);
+    }
+    *reinterpret_cast<float4*>(&qs[i / (D / 4)][4 * (i % (D / 4))]) = x;
+  }
+  int lim[NT];   // keys that row j of each row tile sees
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int r = r_first + t * kKeys + j;
+    lim[t] = r < n_rows ? row_end(r) : 0;
+  }
+  __syncthreads();
+
+  float m[NT], l[NT];
+  float4x o[NT][kDT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    m[t] = kNegBig;
+    l[t] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < kDT; ++d) o[t][d] = float4x{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+
+  for (int n = wv; n < n_kt; n += W) {
+#pragma unroll
+    for (int u = 0; u < kLi; ++u) {
+      float f[kVec];
+      Elem<T>::to_f32(kr[u], f);
+      float* dst = &ks[wv][u * kTpl + lane / kLpr][(lane % kLpr) * kVec];
+#pragma unroll
+      for (int e = 0; e < kVec; e += 4)
+        *reinterpret_cast<float4*>(dst + e) = make_float4(f[e], f[e + 1], f[e + 2], f[e + 3]);
+    }
+    wave_lds_fence();
+    // The slots two tiles ahead are asked for before the loads of the next
+    // tile, so that no later wait for them waits for those loads; and past
+    // the last tile the loads go on (one token's rows again), because a load
+    // under a condition makes the compiler wait for every load at the join.
+    const uint32_t slots = next_slots;
+    next_slots = slot_of(n + 2 * W);
+    load_k(slots);
+
+    // S^T: lane (j, g) gets keys 4 g + i of row j of each row tile.  kAcc
+    // accumulators per row tile, summed at the end: short chains of dependent
+    // products, and of roundings.
+    constexpr int kAcc = NT == 1 ? 4 : 2;
+    float4x sa[NT][kAcc];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int c = 0; c < kAcc; ++c) sa[t][c] = float4x{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int c = 0; c < D / 16; ++c) {
+      const float4 kf = *reinterpret_cast<const float4*>(&ks[wv][j][g * (D / 4) + 4 * c]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const float4 qf =
+            *reinterpret_cast<const float4*>(&qs[t * kKeys + j][g * (D / 4) + 4 * c]);
+        sa[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf.x, sa[t][0], 0, 0, 0);
+        sa[t][1 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf.y, sa[t][1 % kAcc], 0, 0, 0);
+        sa[t][2 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf.z, sa[t][2 % kAcc], 0, 0, 0);
+        sa[t][3 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf.w, sa[t][3 % kAcc], 0, 0, 0);
+      }
+    }
+    float4x s[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      s[t] = kAcc == 4 ? (sa[t][0] + sa[t][1]) + (sa[t][2] + sa[t][3 % kAcc])
+                       : sa[t][0] + sa[t][1];
+    wave_lds_fence();
+
+    const int t0 = n * kKeys;
+    const bool masked = t0 + kKeys > seen_by_all;   // wave-uniform
+    float p[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        x[i] = !masked || t0 + 4 * g + i < lim[t] ? s[t][i] : -INFINITY;
+      const float mx = max_over_groups(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])));
+      const float m_new = mx > m[t] + kRowsSlack ? mx : m[t];
+      if (__builtin_amdgcn_ballot_w64(m_new != m[t]) != 0) {
+        const float corr = fast_exp2(m[t] - m_new);
+        l[t] *= corr;
+#pragma unroll
+        for (int d = 0; d < kDT; ++d)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[t][d][i] *= corr;
+        m[t] = m_new;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[t][i] = fast_exp2(x[i] - m[t]);   // masked: exp2(-inf) = 0
+        l[t] += p[t][i];
+      }
+    }
+
+    bool one_by_one = false;
+    if (masked) {
+      float chk = 0.0f;   // 0 unless some V value is infinite or NaN
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int u = 0; u < kNV; ++u)
+#pragma unroll
+          for (int e = 0; e < kVE; ++e) chk = fmaf(word_elem<T>(vr[i][u], e), 0.0f, chk);
+      one_by_one = __builtin_amdgcn_ballot_w64(chk != 0.0f) != 0;   // NaN != 0
+    }
+    if (!one_by_one) {
+      // O^T += V^T . P^T: output tile (u, e) holds dims 16 kVE u + kVE row + e
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int u = 0; u < kNV; ++u)
+#pragma unroll
+          for (int e = 0; e < kVE; ++e) {
+            const float vf = word_elem<T>(vr[i][u], e);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              o[t][u * kVE + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf, p[t][i],
+                                                                      o[t][u * kVE + e], 0, 0, 0);
+          }
+    } else {
+#pragma unroll 1
+      for (int gk = 0; gk < 4; ++gk) {   // keys 4 gk + i, the other groups' values zero
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int u = 0; u < kNV; ++u)
+#pragma unroll
+            for (int e = 0; e < kVE; ++e) {
+              const float vf = g == gk ? word_elem<T>(vr[i][u], e) : 0.0f;
+#pragma unroll
+              for (int t = 0; t < NT; ++t) {
+                const float4x with = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                    vf, p[t][i], o[t][u * kVE + e], 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                  if (t0 + 4 * gk + i < lim[t]) o[t][u * kVE + e][r] = with[r];
+              }
+              __builtin_amdgcn_sched_barrier(0);   // one product at a time: registers
+            }
+      }
+    }
+    load_v(slots);
+  }
+
+  // ---- combine the waves' states and write the rows -------------------------
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    l[t] = sum_over_groups(l[t]);
+    if (g == 0) {
+      wave_m[wv][t * kKeys + j] = m[t];
+      wave_l[wv][t * kKeys + j] = l[t];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    float mm = wave_m[0][t * kKeys + j];
+#pragma unroll
+    for (int w = 1; w < W; ++w) mm = fmaxf(mm, wave_m[w][t * kKeys + j]);
+    float ll = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+      ll += wave_l[w][t * kKeys + j] * fast_exp2(wave_m[w][t * kKeys + j] - mm);
+    const float sc = fast_exp2(m[t] - mm);
+    const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
+    // row j of the tile, this wave's part; its K rows are no longer needed
+#pragma unroll
+    for (int u = 0; u < kNV; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < kVE; ++e)
+          ks[wv][j][16 * kVE * u + kVE * (4 * g + i) + e] = o[t][u * kVE + e][i] * sc;
+    if (wv == 0 && g == 0) inv_l[j] = inv;
+    __syncthreads();
+    for (int i = tid; i < kKeys * (D / 4); i += 64 * W) {
+      const int rr = i / (D / 4), c = 4 * (i % (D / 4));
+      float4 x = *reinterpret_cast<const float4*>(&ks[0][rr][c]);
+#pragma unroll
+      for (int w = 1; w < W; ++w) {
+        const float4 y = *reinterpret_cast<const float4*>(&ks[w][rr][c]);
+        x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
+      }
+      const float f = inv_l[rr];
+      const int r = r_first + t * kKeys + rr;
+      if (r < n_rows)
+        *reinterpret_cast<float4*>(a.out + out_row(r) + c) =
+            make_float4(x.x * f, x.y * f, x.z * f, x.w * f);
+    }
+    __syncthreads();
+  }
+}
+
+template <typename T, int D, int NT, int W>
+__global__ __launch_bounds__(64 * W) void rows_prefill_kernel(RowsArgs ra) {
+  const RowAttnArgs& a = ra.a;
+  const int n_pairs = a.B * a.Hkv;
+  const int wg = (int)blockIdx.x < ra.reversed ? ra.reversed - 1 - (int)blockIdx.x : (int)blockIdx.x;
+  const int pair = wg % n_pairs;
+  const int b = pair / a.Hkv;
+  const int kvh = pair - b * a.Hkv;
+  const int rows = (a.cu_q ? a.cu_q[b + 1] - a.cu_q[b] : a.S) * (a.H / a.Hkv);
+  // heaviest first; the step is for a ragged sequence of more than a.S rows
+  for (int tile = ra.n_tiles - 1 - wg / n_pairs; tile * kKeys * NT < rows; tile += ra.n_tiles)
+    rows_tile<T, D, NT, W>(ra, b, kvh, tile);
+}
+
+// ---------------------------------------------------------------------------
+// host launch
+// ---------------------------------------------------------------------------
+
+template <typename T, int D, int NT, int W>
+void launch_shape(const RowAttnArgs& a, int64_t rows_per_pair, int cus, hipStream_t stream) {
+  RowsArgs ra;
+  ra.a = a;
+  ra.n_tiles = (int)ceil_div(rows_per_pair, kKeys * NT);
+  ra.bs_shift = (a.BS & (a.BS - 1)) == 0 ? __builtin_ctz((unsigned)a.BS) : -1;
+  const int64_t n_wg = (int64_t)ra.n_tiles * a.B * a.Hkv;
+  // More than one workgroup per CU but not two: the hardware deals the first
+  // round out to all CUs and the second to the first of them again, so with
+  // the first round reversed those hold its lightest workgroups (and not its
+  // heaviest) beside the second's.  Only where two workgroups fit a CU
+  // together (their registers, up to head dim 64).  GPT-2's 512-token chunk,
+  // 384 workgroups: 26.4 -> 23.7 us.
+  ra.reversed = D <= 64 && n_wg > cus && n_wg <= 2 * (int64_t)cus ? cus : 0;
+  const dim3 grid((unsigned)n_wg), block(64 * W);
+  hipLaunchKernelGGL((rows_prefill_kernel<T, D, NT, W>), grid, block, 0, stream, ra);
+}
+
+// The workgroup's shape.  Measured on MI355X (us, rows x waves 16 x 4 / 16 x 8
+// / 32 x 8; one sequence unless said):
+//   12 heads, D 64, fp32, 512 rows on 512 tokens     27 / 24 / 26
+//   the same, 16 rows on 1000                         20 / 17 / 25
+//   32 heads, D 128, fp32, 512 rows on 512            89 / 90 / 86
+//   32 / 8 heads, D 128, bf16, 256 rows on 512        38 / 39 / 37
+//   32 / 8 heads, D 128, fp16, 9 rows on 3000         87 / 72 / 121
+//   8 / 4 heads, D 256, fp32, 700 rows on 1000        142 / 170 / -
+// (the row kernel before: 117, 59, 766, 109, 442, 803).  So 8 waves of 16
+// rows; 32 rows, which read K and V half as often, once they still give every
+// CU two workgroups; and 4 waves at head dim 256, where the registers hold
+// one wave a SIMD.
+template <typename T, int D>
+void launch_d(const RowAttnArgs& a, int64_t rows_per_pair, int cus, hipStream_t stream) {
+  if constexpr (D == 256) {
+    launch_shape<T, D, 1, 4>(a, rows_per_pair, cus, stream);
+  } else {
+    const int64_t wide = sat_mul(ceil_div(rows_per_pair, 2 * kKeys), a.B, a.Hkv);
+    if (wide >= 2 * (int64_t)cus) launch_shape<T, D, 2, 8>(a, rows_per_pair, cus, stream);
+    else launch_shape<T, D, 1, 8>(a, rows_per_pair, cus, stream);
+  }
+}
+
+template <typename T>
+void launch_t(const RowAttnArgs& a, int D, int64_t rows_per_pair, int cus, hipStream_t stream) {
+  switch (D) {
+    case 32: launch_d<T, 32>(a, rows_per_pair, cus, stream); break;
+    case 64: launch_d<T, 64>(a, rows_per_pair, cus, stream); break;
+    case 128: launch_d<T, 128>(a, rows_per_pair, cus, stream); break;
+    default: launch_d<T, 256>(a, rows_per_pair, cus, stream); break;
+  }
+}
+
+}  // namespace
+
+bool rows_prefill_serves(const RowAttnArgs& a, int kv_dtype, int D) {
+  const int elem = kv_dtype == HS_DTYPE_F32 ? 4 : 2;
+  const int64_t tiles = sat_mul(ceil_div(sat_mul(a.S, a.H / a.Hkv), kKeys), a.B, a.Hkv);
+  return tiles > 0 && tiles <= 0x7fffffffLL && sat_mul(a.S, a.H / a.Hkv) <= (1LL << 30) &&
+         sat_mul(a.NB, a.BS, (int64_t)a.Hkv * (D * elem / 64)) <= 0xffffffffLL &&
+         sat_mul(a.MB, a.BS) <= (1LL << 30);
+}
+
+int launch_rows_prefill(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream) {
+  const int64_t rows_per_pair = (int64_t)a.S * (a.H / a.Hkv);
+  profile_begin(stream);
+  if (kv_dtype == HS_DTYPE_F32) launch_t<float>(a, D, rows_per_pair, cus, stream);
+  else if (kv_dtype == HS_DTYPE_F16) launch_t<_Float16>(a, D, rows_per_pair, cus, stream);
+  else launch_t<Bf16>(a, D, rows_per_pair, cus, stream);
+  profile_end(stream);
+  return check_launch("paged prefill");
+}
+
+}  // namespace hs

@@ -9,8 +9,8 @@ build_error :258, paged_attention_prefill :263-278).
                     (padding) are zero
     ->              [B, S, H, D] float32
 
-Runs libhsattn's row kernel (one online-softmax pass per query row and head,
-fp32 arithmetic, any KV dtype).  Difference from the reference: no torch
+Runs libhsattn's fp32 prefill (tiles of query rows on the fp32 matrix cores,
+any KV dtype and block size).  Difference from the reference: no torch
 fallback -- RuntimeError when the library is unavailable.  The binding that
 goes into the reference tree keeps the reference's torch branch
 (``paged_attention_prefill_torch``) for hosts without the library, which the
@@ -43,7 +43,7 @@ def paged_attention_prefill_varlen(q, cu_seqlens_q, max_seqlen_q, k_cache, v_cac
 
     q [total, H, D]; sequence b owns rows cu_seqlens_q[b]:cu_seqlens_q[b+1],
     which are the trailing tokens of its context.  use_mfma selects the
-    matrix-core kernel (fp16/bf16 KV, block_size 16) or the fp32 row kernel.
+    matrix-core kernel (fp16/bf16 KV, block_size 16) or the fp32 one.
     """
     _hip.lib("prefill kernel")
     return _hip.prefill_varlen(q, cu_seqlens_q, max_seqlen_q, k_cache, v_cache,

@@ -229,7 +229,8 @@ size_t hs_prefill_workspace_bytes(int B, int max_seqlen_q, int H, int D, int use
  * Replaces:
  *   use_mfma = 0: paged_attention_prefill,
  *                 heteroserve/model/paged_attn_prefill.py:159-214
- *                 (fp32 VALU arithmetic, any KV dtype, D in {32,64,128,256})
+ *                 (fp32 arithmetic on the fp32 matrix cores, any KV dtype and
+ *                 block size, D in {32,64,128,256})
  *   use_mfma = 1: paged_attention_prefill_wmma,
  *                 heteroserve/model/paged_attn_wmma.py:256-318
  *                 (fp16 matrix-core operands with fp32 accumulation; KV dtype

@@ -1,0 +1,144 @@
+"""The fp32 prefill (use_mfma = 0) on the fp32 matrix cores, at the sizes where
+its tiles can go wrong: row tiles of 16 and 32, key tiles of 16, waves that
+get no tile, block sizes that are no power of two, grouped heads that share a
+row tile, ragged and padded rows, and values that a row must not see.
+
+Tolerance.  Nothing is rounded below fp32, so the error is that of fp32 sums:
+a random walk of at most max(D, n / 8) = 256 roundings of 2^-24 relative to the
+result, 16 * 6e-8 = 1e-6 in the 2-norm against fp64.
+"""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from oracle.attention import prefill_one  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+REL = 1e-6
+
+
+def _case(chunks, ctxs, H, Hkv, D, BS, dtype, seed=0):
+    rng = np.random.default_rng(seed)
+    need = [max(1, -(-max(n, 1) // BS)) for n in ctxs]
+    ids = rng.permutation(sum(need) + 3)
+    bt = np.full((len(ctxs), max(need) + 1), -1, dtype=np.int32)
+    at = 0
+    for i, k in enumerate(need):
+        bt[i, :k] = ids[at:at + k]
+        at += k
+    gen = torch.Generator().manual_seed(seed)
+    k, v = (torch.randn((sum(need) + 3, BS, Hkv, D), generator=gen).to(dtype) for _ in range(2))
+    q = torch.randn((sum(chunks), H, D), generator=gen)
+    return q, k, v, torch.from_numpy(bt), torch.tensor(ctxs, dtype=torch.int32)
+
+
+def _run(q, k, v, bt, ctx, chunks, longest=None):
+    from heteroserve.model.paged_attn_prefill import paged_attention_prefill_varlen
+
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(chunks)]), dtype=torch.int32)
+    got = paged_attention_prefill_varlen(
+        q.to(DEV), cu.to(DEV), longest or max(chunks), k.to(DEV), v.to(DEV), bt.to(DEV),
+        ctx.to(DEV), 1.0 / math.sqrt(q.shape[2]), use_mfma=False)
+    return got.cpu()
+
+
+def _want(q, k, v, bt, ctx, chunks):
+    """prefill_one in fp64: same function, doubled operands."""
+    out, row = [], 0
+    for b, n in enumerate(chunks):
+        S, H, D = n, q.shape[1], q.shape[2]
+        m = min(int(ctx[b]), bt.shape[1] * k.shape[1])
+        res = torch.zeros((S, H, D), dtype=torch.float64)
+        if S and m > 0:
+            pages = bt[b, :-(-m // k.shape[1])].long().clamp(min=0)
+            g = H // k.shape[2]
+            kk, vv = (x[pages].reshape(-1, *x.shape[2:])[:m].double().repeat_interleave(g, 1)
+                      for x in (k, v))
+            s = torch.einsum("shd,nhd->shn", q[row:row + S].double(), kk) / math.sqrt(D)
+            pos = int(ctx[b]) - S + torch.arange(S)
+            s = s.masked_fill((torch.arange(m)[None] > pos[:, None])[:, None], -math.inf)
+            res = torch.einsum("shn,nhd->shd", torch.nan_to_num(torch.softmax(s, -1)), vv)
+        out.append(res)
+        row += n
+    return torch.cat(out)
+
+
+def _rel(got, want):
+    return ((got.double() - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+@pytest.mark.parametrize("H,Hkv,BS", [(4, 4, 16), (6, 2, 5), (16, 1, 32), (3, 3, 1)])
+def test_edges_of_tiles(dtype, D, H, Hkv, BS):
+    """Chunks and contexts on both sides of 16, 32 and 8 x 16, in one ragged call."""
+    chunks = [1, 15, 16, 17, 33, 0, 64]
+    ctxs = [1, 15, 129, 200, 33, 40, 321]
+    args = _case(chunks, ctxs, H, Hkv, D, BS, dtype)
+    got = _run(*args, chunks)
+    assert _rel(got, _want(*args, chunks)) <= REL
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_wide_row_tiles(D):
+    """Enough rows for the 32-row tiles (2 workgroups a CU), a remainder of 9."""
+    chunks, ctxs = [521, 300], [521, 333]
+    args = _case(chunks, ctxs, 32, 32, D, 16, torch.float32, seed=1)
+    assert _rel(_run(*args, chunks), _want(*args, chunks)) <= REL
+
+
+def test_one_to_two_workgroups_per_cu():
+    """The reversed first round: 12 heads x 25 row tiles = 300 workgroups."""
+    chunks, ctxs = [400], [500]
+    args = _case(chunks, ctxs, 12, 12, 64, 16, torch.float32, seed=2)
+    assert _rel(_run(*args, chunks), _want(*args, chunks)) <= REL
+
+
+def test_short_context_rows_and_understated_maximum():
+    """Rows at negative positions are zero, contexts past the table are cut at
+    its end, and rows past max_seqlen_q are still served."""
+    chunks, ctxs = [40, 50], [10, 96]
+    args = _case(chunks, ctxs, 4, 2, 64, 16, torch.float16, seed=3)
+    got = _run(*args, chunks)
+    assert torch.all(got[:30] == 0)
+    assert _rel(got, _want(*args, chunks)) <= REL
+    assert torch.equal(_run(*args, chunks, longest=20), got)
+    q, k, v, bt, ctx = args
+    long_ctx = ctx.clone()
+    long_ctx[1] = 500      # the table holds 112 tokens
+    want = torch.cat([prefill_one(q[:40], k, v, bt[0], 10, 0.125),
+                      prefill_one(q[40:], k, v, bt[1], 500, 0.125)])
+    assert _rel(_run(q, k, v, bt, long_ctx, chunks), want.double()) <= REL
+
+
+@pytest.mark.parametrize("bad", [math.inf, -math.inf, math.nan])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D,H,Hkv", [(64, 2, 2), (128, 8, 2), (256, 2, 1)])
+def test_rows_do_not_see_later_values(bad, dtype, D, H, Hkv):
+    """A non-finite V value reaches the rows at or after its position, in its
+    own head and dim only; stale values after the context reach no row."""
+    chunks, ctxs = [50], [70]
+    q, k, v, bt, ctx = _case(chunks, ctxs, H, Hkv, D, 16, dtype, seed=4)
+    clean = _run(q, k, v, bt, ctx, chunks)
+    pos = 45
+    v[bt[0, pos // 16], pos % 16, 0, 7] = bad
+    v[bt[0, 4], 70 - 64:, :, :] = bad        # past the context, in its last page
+    k[bt[0, 4], 70 - 64:, :, :] = bad
+    got = _run(q, k, v, bt, ctx, chunks)
+    G = H // Hkv
+    first = pos - 20                         # row of that position
+    hit = torch.zeros_like(got, dtype=torch.bool)
+    hit[first:, :G, 7] = True
+    if math.isnan(bad):
+        assert torch.isnan(got[hit]).all()
+    else:
+        assert (got[hit] == bad).all()
+    # the others: the same values, up to the order of the sums in that tile
+    assert _rel(got[~hit], clean[~hit].double()) <= REL
