@@ -25,6 +25,12 @@ import threading
 from pathlib import Path
 from typing import Optional
 
+try:
+    import torch
+except ImportError as _exc:   # reported by _load()
+    torch = None
+    _torch_error = str(_exc)
+
 ABI_VERSION = 5
 DTYPE_F32, DTYPE_F16, DTYPE_BF16 = 0, 1, 2
 
@@ -104,10 +110,8 @@ def _load() -> None:
         if os.environ.get("HETEROSERVE_DISABLE_CUDA_KERNEL"):
             _state, _error = "unavailable", "disabled by HETEROSERVE_DISABLE_CUDA_KERNEL"
             return
-        try:
-            import torch
-        except ImportError as exc:
-            _state, _error = "unavailable", f"torch unavailable: {exc}"
+        if torch is None:
+            _state, _error = "unavailable", f"torch unavailable: {_torch_error}"
             return
         if not torch.cuda.is_available():
             _state, _error = "unavailable", "no HIP device"
@@ -142,6 +146,8 @@ def error() -> Optional[str]:
 
 def lib(what: str = "paged attention HIP kernel") -> ctypes.CDLL:
     """The loaded library, or RuntimeError naming why it is unavailable."""
+    if _state == "ready":
+        return _lib
     _load()
     if _state != "ready":
         raise RuntimeError(f"{what} unavailable: {_error}")
@@ -155,79 +161,118 @@ def check(rc: int) -> None:
 
 # ---------------------------------------------------------------------------
 # marshalling helpers
+#
+# A small decode step is a few microseconds on the GPU, so the calls below are
+# what such a step costs: they compare device indexes (an int from one C call)
+# instead of device objects, convert only what needs converting, ask torch for
+# the raw stream, and remember workspace sizes.  A decode call of 8 sequences
+# took 16.2 us of host time before.
 # ---------------------------------------------------------------------------
 
-def dtype_code(dt) -> int:
-    import torch
+_DTYPE_CODES = {} if torch is None else {
+    torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
+_raw_stream = getattr(getattr(torch, "_C", None), "_cuda_getCurrentRawStream", None)
 
-    codes = {torch.float32: DTYPE_F32, torch.float16: DTYPE_F16, torch.bfloat16: DTYPE_BF16}
-    if dt not in codes:
+
+def dtype_code(dt) -> int:
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
         raise RuntimeError(f"unsupported KV cache dtype {dt} (float32, float16 or bfloat16)")
-    return codes[dt]
+    return code
 
 
 def stream_of(device) -> int:
-    import torch
-
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device() if device.index is None else device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def _int32_on(t, device):
-    import torch
+def _stream_at(index: int) -> int:
+    """The current stream of device `index`."""
+    if _raw_stream is not None:
+        return _raw_stream(index)
+    return torch.cuda.current_stream(index).cuda_stream
 
+
+def _int32_on(t, device):
     if not torch.is_tensor(t):
         t = torch.as_tensor(t)
+    if t.dtype is torch.int32 and t.get_device() == device.index and t.is_contiguous():
+        return t
     return t.to(device=device, dtype=torch.int32).contiguous()
 
 
-def _check_device(q, k_cache, v_cache) -> None:
-    if not q.is_cuda:
+def _check_device(q, k_cache, v_cache) -> int:
+    """The device index that all three tensors are on."""
+    index = q.get_device()
+    if index < 0 or not q.is_cuda:
         raise RuntimeError("q must be on CUDA")
-    if not (k_cache.is_cuda and v_cache.is_cuda):
-        raise RuntimeError("kv cache must be on CUDA")
-    if k_cache.device != q.device or v_cache.device != q.device:
+    if k_cache.get_device() != index or v_cache.get_device() != index:
+        if not (k_cache.is_cuda and v_cache.is_cuda):
+            raise RuntimeError("kv cache must be on CUDA")
         raise RuntimeError("q and the kv cache must be on the same device")
+    return index
 
 
 def _check_q(q):
-    import torch
-
-    if q.dtype != torch.float32:
+    if q.dtype is not torch.float32:
         raise RuntimeError(f"q must be float32, got {q.dtype}")
     return q.contiguous()
 
 
 def _check_kv(k_cache, v_cache, D):
-    if k_cache.dim() != 4:
+    """(k_cache, v_cache) contiguous, and their shape."""
+    shape = k_cache.shape
+    if len(shape) != 4:
         raise RuntimeError("k_cache must be [NB, BS, H, D]")
-    if v_cache.shape != k_cache.shape:
+    if v_cache.shape != shape:
         raise RuntimeError("v_cache must have the shape of k_cache")
-    if k_cache.dtype != v_cache.dtype:
+    if k_cache.dtype is not v_cache.dtype:
         raise RuntimeError("k_cache and v_cache must have the same dtype")
-    if k_cache.shape[3] != D:
-        raise RuntimeError(f"head_dim mismatch: q has {D}, cache has {k_cache.shape[3]}")
-    return k_cache.contiguous(), v_cache.contiguous()
+    if shape[3] != D:
+        raise RuntimeError(f"head_dim mismatch: q has {D}, cache has {shape[3]}")
+    return k_cache.contiguous(), v_cache.contiguous(), shape
 
 
 class _DeviceGuard:
-    """Make `device` current for the duration of a library call."""
+    """Make device `index` current for the duration of a library call."""
 
-    def __init__(self, device):
-        import torch
+    __slots__ = ("_index", "_prev")
 
-        self._torch = torch
-        self._dev = device.index if device.index is not None else torch.cuda.current_device()
+    def __init__(self, index: int):
+        self._index = index
         self._prev = None
 
     def __enter__(self):
-        cur = self._torch.cuda.current_device()
-        if cur != self._dev:
+        cur = torch.cuda.current_device()
+        if cur != self._index:
             self._prev = cur
-            self._torch.cuda.set_device(self._dev)
+            torch.cuda.set_device(self._index)
 
     def __exit__(self, *exc):
         if self._prev is not None:
-            self._torch.cuda.set_device(self._prev)
+            torch.cuda.set_device(self._prev)
+
+
+# Workspace sizes of decode calls by their arguments and device.  The sizes are
+# fixed for a device and a library; the table is emptied when it grows past
+# what a server's batch sizes and table widths make.
+_WS_SIZES: dict = {}
+_WS_SIZES_MAX = 4096
+
+
+def _decode_workspace(query, index: int, *sizes: int) -> int:
+    """query(*sizes), with device `index` current (only sizes above 0 are kept:
+    0 may also be a failed query)."""
+    key = (query.__name__, index, sizes)
+    n = _WS_SIZES.get(key)
+    if n is None:
+        n = query(*sizes)
+        if n:
+            if len(_WS_SIZES) >= _WS_SIZES_MAX:
+                _WS_SIZES.clear()
+            _WS_SIZES[key] = n
+    return n
 
 
 def decode(q, k_cache, v_cache, block_tables, context_lens, scale: float,
@@ -237,56 +282,53 @@ def decode(q, k_cache, v_cache, block_tables, context_lens, scale: float,
     shared_pages=True (fixed partitions only, num_splits == 0) runs
     hs_decode_shared: partitions whose block ids several sequences share are
     read once for all of them."""
-    import torch
-
     L = lib()
-    _check_device(q, k_cache, v_cache)
+    index = _check_device(q, k_cache, v_cache)
     if q.dim() != 3:
         raise RuntimeError("q must be [B, H, D]")
     q = _check_q(q)
     B, H, D = q.shape
-    k_cache, v_cache = _check_kv(k_cache, v_cache, D)
-    NB, BS, Hkv, _ = k_cache.shape
-    bt = _int32_on(block_tables, q.device)
-    ctx = _int32_on(context_lens, q.device)
+    k_cache, v_cache, (NB, BS, Hkv, _) = _check_kv(k_cache, v_cache, D)
+    dev = q.device
+    bt = _int32_on(block_tables, dev)
+    ctx = _int32_on(context_lens, dev)
     if bt.dim() != 2 or bt.shape[0] != B:
         raise RuntimeError("block_tables must be [B, max_blocks]")
     if ctx.numel() != B:
         raise RuntimeError("context_lens must have one entry per sequence")
     MB = bt.shape[1]
-    out = torch.empty((B, H, D), dtype=torch.float32, device=q.device)
+    out = q.new_empty(q.shape)
     if B == 0:
         return out
-    if shared_pages and int(num_splits) != 0:
+    scale, num_splits, partition_tokens = float(scale), int(num_splits), int(partition_tokens)
+    if shared_pages and num_splits != 0:
         raise RuntimeError("shared_pages needs fixed partitions (num_splits == 0)")
-    if shared_pages:
-        ws_bytes = L.hs_decode_shared_workspace_bytes(B, H, Hkv, D, BS, max(MB, 1),
-                                                      int(partition_tokens))
-    else:
-        ws_bytes = L.hs_decode_workspace_bytes(B, H, Hkv, D, BS, max(MB, 1), int(num_splits),
-                                               int(partition_tokens))
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
-    wsp = ws.data_ptr() if ws is not None else None
-    with _DeviceGuard(q.device):
+    with _DeviceGuard(index):
         if shared_pages:
-            check(L.hs_decode_shared(
-                q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype),
-                NB, bt.data_ptr(), ctx.data_ptr(), out.data_ptr(), B, H, Hkv, D, BS, MB,
-                float(scale), int(partition_tokens), wsp, ws_bytes, stream_of(q.device)))
+            ws_bytes = _decode_workspace(L.hs_decode_shared_workspace_bytes, index, B, H, Hkv, D,
+                                         BS, max(MB, 1), partition_tokens)
         else:
-            check(L.hs_decode(
+            ws_bytes = _decode_workspace(L.hs_decode_workspace_bytes, index, B, H, Hkv, D, BS,
+                                         max(MB, 1), num_splits, partition_tokens)
+        ws = q.new_empty((ws_bytes + 3) // 4) if ws_bytes else None
+        wsp = ws.data_ptr() if ws is not None else None
+        if shared_pages:
+            rc = L.hs_decode_shared(
                 q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype),
                 NB, bt.data_ptr(), ctx.data_ptr(), out.data_ptr(), B, H, Hkv, D, BS, MB,
-                float(scale), int(num_splits), int(partition_tokens), wsp, ws_bytes,
-                stream_of(q.device)))
+                scale, partition_tokens, wsp, ws_bytes, _stream_at(index))
+        else:
+            rc = L.hs_decode(
+                q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype),
+                NB, bt.data_ptr(), ctx.data_ptr(), out.data_ptr(), B, H, Hkv, D, BS, MB,
+                scale, num_splits, partition_tokens, wsp, ws_bytes, _stream_at(index))
+        check(rc)
     return out
 
 
 def _prefill_workspace(L, B: int, rows: int, H: int, D: int, use_mfma: bool, split: bool,
                        device):
     """(tensor or None, bytes): the key-range split's scratch, when it applies."""
-    import torch
-
     nbytes = L.hs_prefill_workspace_bytes(B, rows, H, D, int(bool(use_mfma))) if split else 0
     if not nbytes:
         return None, 0
@@ -299,32 +341,29 @@ def prefill(q, k_cache, v_cache, block_tables, context_lens, scale: float, use_m
 
     split=False passes no workspace, so the matrix-core kernel runs without
     the key-range split (for tests of that launch shape)."""
-    import torch
-
     L = lib()
-    _check_device(q, k_cache, v_cache)
+    index = _check_device(q, k_cache, v_cache)
     if q.dim() != 4:
         raise RuntimeError("q must be [B, S, H, D]")
     q = _check_q(q)
     B, S, H, D = q.shape
-    k_cache, v_cache = _check_kv(k_cache, v_cache, D)
-    NB, BS, Hkv, _ = k_cache.shape
+    k_cache, v_cache, (NB, BS, Hkv, _) = _check_kv(k_cache, v_cache, D)
     bt = _int32_on(block_tables, q.device)
     ctx = _int32_on(context_lens, q.device)
     if bt.dim() != 2 or bt.shape[0] != B:
         raise RuntimeError("block_tables must be [B, max_blocks]")
     if ctx.numel() != B:
         raise RuntimeError("context_lens must have one entry per sequence")
-    out = torch.empty((B, S, H, D), dtype=torch.float32, device=q.device)
+    out = q.new_empty(q.shape)
     if B == 0 or S == 0:
         return out
-    with _DeviceGuard(q.device):
+    with _DeviceGuard(index):
         ws, ws_bytes = _prefill_workspace(L, B, S, H, D, use_mfma, split, q.device)
         check(L.hs_prefill(
             q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype),
             NB, bt.data_ptr(), ctx.data_ptr(), out.data_ptr(), B, S, H, Hkv, D, BS,
             bt.shape[1], float(scale), int(bool(use_mfma)),
-            ws.data_ptr() if ws is not None else None, ws_bytes, stream_of(q.device)))
+            ws.data_ptr() if ws is not None else None, ws_bytes, _stream_at(index)))
     return out
 
 
@@ -332,26 +371,23 @@ def prefill_varlen(q, cu_seqlens_q, max_seqlen_q: int, k_cache, v_cache, block_t
                    context_lens, scale: float, use_mfma: bool, split: bool = True):
     """out[T, H, D] fp32 for ragged chunks via hs_prefill_varlen (split as for
     prefill)."""
-    import torch
-
     L = lib()
-    _check_device(q, k_cache, v_cache)
+    index = _check_device(q, k_cache, v_cache)
     if q.dim() != 3:
         raise RuntimeError("q must be [total_tokens, H, D]")
     q = _check_q(q)
     T, H, D = q.shape
-    k_cache, v_cache = _check_kv(k_cache, v_cache, D)
-    NB, BS, Hkv, _ = k_cache.shape
+    k_cache, v_cache, (NB, BS, Hkv, _) = _check_kv(k_cache, v_cache, D)
     bt = _int32_on(block_tables, q.device)
     ctx = _int32_on(context_lens, q.device)
     cu = _int32_on(cu_seqlens_q, q.device)
     B = bt.shape[0]
     if cu.numel() != B + 1 or ctx.numel() != B:
         raise RuntimeError("cu_seqlens_q must be [B + 1] and context_lens [B]")
-    out = torch.empty((T, H, D), dtype=torch.float32, device=q.device)
+    out = q.new_empty(q.shape)
     if B == 0 or T == 0:
         return out
-    with _DeviceGuard(q.device):
+    with _DeviceGuard(index):
         ws, ws_bytes = _prefill_workspace(L, B, int(max_seqlen_q), H, D, use_mfma, split,
                                           q.device)
         check(L.hs_prefill_varlen(
@@ -359,7 +395,7 @@ def prefill_varlen(q, cu_seqlens_q, max_seqlen_q: int, k_cache, v_cache, block_t
             v_cache.data_ptr(), dtype_code(k_cache.dtype), NB, bt.data_ptr(), ctx.data_ptr(),
             out.data_ptr(), B, H, Hkv, D, BS, bt.shape[1], float(scale),
             int(bool(use_mfma)), ws.data_ptr() if ws is not None else None, ws_bytes,
-            stream_of(q.device)))
+            _stream_at(index)))
     return out
 
 
@@ -376,9 +412,9 @@ def kv_pack(pool, ids_dev, out) -> None:
     L = lib("KV pack HIP kernel")
     Ls, _, NB = pool.shape[:3]
     page = pool[0, 0, 0].numel() * pool.element_size()
-    with _DeviceGuard(pool.device):
+    with _DeviceGuard(pool.get_device()):
         check(L.hs_kv_pack(pool.data_ptr(), Ls, NB, page, ids_dev.data_ptr(), ids_dev.numel(),
-                           out.data_ptr(), stream_of(pool.device)))
+                           out.data_ptr(), _stream_at(pool.get_device())))
 
 
 def kv_unpack(pool, ids_dev, src) -> None:
@@ -386,9 +422,9 @@ def kv_unpack(pool, ids_dev, src) -> None:
     L = lib("KV unpack HIP kernel")
     Ls, _, NB = pool.shape[:3]
     page = pool[0, 0, 0].numel() * pool.element_size()
-    with _DeviceGuard(pool.device):
+    with _DeviceGuard(pool.get_device()):
         check(L.hs_kv_unpack(pool.data_ptr(), Ls, NB, page, ids_dev.data_ptr(),
-                             ids_dev.numel(), src.data_ptr(), stream_of(pool.device)))
+                             ids_dev.numel(), src.data_ptr(), _stream_at(pool.get_device())))
 
 
 def kv_gather(cache, block_tables_dev, length: int, out) -> None:
@@ -397,9 +433,9 @@ def kv_gather(cache, block_tables_dev, length: int, out) -> None:
     NB, BS = cache.shape[:2]
     row = cache[0, 0].numel() * cache.element_size()
     B, MB = block_tables_dev.shape
-    with _DeviceGuard(cache.device):
+    with _DeviceGuard(cache.get_device()):
         check(L.hs_kv_gather(cache.data_ptr(), NB, BS, row, block_tables_dev.data_ptr(), MB,
-                             B, int(length), out.data_ptr(), stream_of(cache.device)))
+                             B, int(length), out.data_ptr(), _stream_at(cache.get_device())))
 
 
 def _rows(x, Hkv: int, D: int):
@@ -425,17 +461,22 @@ def _rows(x, Hkv: int, D: int):
 
 
 def _check_write(k_cache, v_cache, k, v):
-    """The caches are written in place: CUDA, contiguous, same shape/dtype."""
-    if k_cache.dim() != 4:
+    """The caches are written in place: CUDA, contiguous, same shape/dtype.
+    Returns their shape and device index."""
+    shape = k_cache.shape
+    if len(shape) != 4:
         raise RuntimeError("k_cache must be [NB, BS, Hkv, D]")
-    if v_cache.shape != k_cache.shape or v_cache.dtype != k_cache.dtype:
+    if v_cache.shape != shape or v_cache.dtype is not k_cache.dtype:
         raise RuntimeError("k_cache and v_cache must have the same shape and dtype")
-    if not (k_cache.is_cuda and v_cache.is_cuda and k.is_cuda and v.is_cuda):
-        raise RuntimeError("kv cache and new rows must be on CUDA")
-    if len({k_cache.device, v_cache.device, k.device, v.device}) != 1:
+    index = k_cache.get_device()
+    if (index < 0 or v_cache.get_device() != index or k.get_device() != index
+            or v.get_device() != index):
+        if not (k_cache.is_cuda and v_cache.is_cuda and k.is_cuda and v.is_cuda):
+            raise RuntimeError("kv cache and new rows must be on CUDA")
         raise RuntimeError("kv cache and new rows must be on the same device")
     if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise RuntimeError("kv cache must be contiguous (it is written in place)")
+    return shape, index
 
 
 def _same_rows(k, v, Hkv: int, D: int):
@@ -452,27 +493,23 @@ def _same_rows(k, v, Hkv: int, D: int):
 def kv_scatter(k_cache, v_cache, slots, k, v) -> None:
     """k_cache.view(-1, Hkv, D)[slots] = k.to(cache dtype); same for v."""
     L = lib("KV scatter HIP kernel")
-    _check_write(k_cache, v_cache, k, v)
-    NB, BS, Hkv, D = k_cache.shape
+    (NB, BS, Hkv, D), index = _check_write(k_cache, v_cache, k, v)
     k, v, stride = _same_rows(k, v, Hkv, D)
     n = k.shape[0]
     if slots.numel() != n:
         raise RuntimeError(f"{slots.numel()} slots for {n} rows")
-    import torch
-
     slots = torch.as_tensor(slots).to(device=k_cache.device, dtype=torch.int64).contiguous()
-    with _DeviceGuard(k_cache.device):
+    with _DeviceGuard(index):
         check(L.hs_kv_scatter(k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype),
                               NB * BS, Hkv, D, slots.data_ptr(), n, k.data_ptr(), v.data_ptr(),
-                              dtype_code(k.dtype), stride, stream_of(k_cache.device)))
+                              dtype_code(k.dtype), stride, _stream_at(index)))
 
 
 def kv_append(k_cache, v_cache, block_tables, positions, k, v, seq_ids=None) -> None:
     """Row i -> slot block_tables[s][pos // BS] * BS + pos % BS of sequence
     s = seq_ids[i] (or i), pos = positions[i]; cast as kv_scatter."""
     L = lib("KV append HIP kernel")
-    _check_write(k_cache, v_cache, k, v)
-    NB, BS, Hkv, D = k_cache.shape
+    (NB, BS, Hkv, D), index = _check_write(k_cache, v_cache, k, v)
     k, v, stride = _same_rows(k, v, Hkv, D)
     n = k.shape[0]
     dev = k_cache.device
@@ -485,16 +522,16 @@ def kv_append(k_cache, v_cache, block_tables, positions, k, v, seq_ids=None) -> 
         raise RuntimeError(f"{sid.numel()} sequence ids for {n} rows")
     if sid is None and n > bt.shape[0]:
         raise RuntimeError("without seq_ids, row i uses table row i: more rows than tables")
-    with _DeviceGuard(dev):
+    with _DeviceGuard(index):
         check(L.hs_kv_append(k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype), NB,
                              BS, Hkv, D, bt.data_ptr(), bt.shape[0], bt.shape[1], pos.data_ptr(),
                              None if sid is None else sid.data_ptr(), n, k.data_ptr(),
-                             v.data_ptr(), dtype_code(k.dtype), stride, stream_of(dev)))
+                             v.data_ptr(), dtype_code(k.dtype), stride, _stream_at(index)))
 
 
 def block_tables(packed_dev, B: int, width: int, out) -> None:
     """out[B, width] int32 from the packed [off[0..B], ids...] device buffer."""
     L = lib("block table HIP kernel")
-    with _DeviceGuard(out.device):
+    with _DeviceGuard(out.get_device()):
         check(L.hs_block_tables(packed_dev.data_ptr(), B, width, out.data_ptr(),
-                                stream_of(out.device)))
+                                _stream_at(out.get_device())))
