@@ -62,6 +62,12 @@ static int device_cu_count(int device) {
   return cus;
 }
 
+// CUs of the current device (1 when it cannot be read).
+static int current_cus() {
+  int dev = 0;
+  return hipGetDevice(&dev) == hipSuccess ? std::max(1, device_cu_count(dev)) : 1;
+}
+
 static bool valid_dtype(int t) {
   return t == HS_DTYPE_F32 || t == HS_DTYPE_F16 || t == HS_DTYPE_BF16;
 }
@@ -87,13 +93,11 @@ struct DecodePlan {
   int mode, part_tokens, splits, P;
 };
 
-// Default partition: 512 tokens, shorter when a wave serves G > 2 query
-// heads of a GQA group (fewer waves, each doing G times the work per token):
-// measured on C2's geometry with 8 and 4 KV heads, 256 and 128 tokens.  With
-// 8 or more query heads per KV head and at most 2 waves' worth of heads per
-// row (matrix-core path, 32 heads a wave), 512 again: there the merge of many
-// short partitions cost more than the waves it adds (MQA with 32 heads on
-// C2's geometry: 65 us at 512 tokens, 90 us at 128).
+// Default partition, which the workspace is sized for: 512 tokens, 1024 / G with
+// G = 4 or 8 query heads per KV head (the largest of 1, 2, 4, 8 dividing the
+// group), and 512 again with 8 or more query heads per KV head and at most 2
+// KV heads' worth of 32.  Grouped heads on the fp32 matrix cores take several
+// such partitions together (rows_partition).
 //
 // bf16 and fp16 caches with 2 or more query heads per KV head run the
 // split-operand matrix-core decode, whose workgroups of splitmm_waves(G)
@@ -144,20 +148,71 @@ static int default_partition(int B, int H, int Hkv, int BS, int MB, int kv_dtype
                                sat_mul(B, Hkv, G / row_attn_heads_per_wave(H, Hkv)), BS, MB);
 }
 
-// Rows of at most this many keys (by the table's width) can take mode 3.
+// Grouped heads on the fp32 matrix cores: workgroups of 8 waves take 16-key
+// tiles in turn, so a partition is 2048 keys, cut down to 128 (a tile a wave)
+// while the launch has fewer workgroups than CUs; never shorter than the
+// partition that the workspace was sized for.  16 sequences of 256..4096
+// tokens, us from 1024 keys and two workgroups a CU / from 2048 and one: 32 / 8
+// heads, D 128, fp32 72 / 60; 16 / 1, fp32 24 / 18; 32 / 4, bf16, 32-token
+// blocks 37 / 33.
+static int rows_partition(int B, int H, int Hkv, int BS, int MB, int default_pt) {
+  const int pt = shrink_for_small_grid(2048, 128, sat_mul(B, Hkv, ceil_div(H / Hkv, 16)), BS, MB, 1);
+  return std::max(pt, default_pt);
+}
+
+// Rows of at most this many keys (by the table's width) can take one
+// workgroup per (row, head).
 constexpr int64_t kWgSplitMaxTokens = 1024;
 
 // The default decomposition of a small grid whose rows are short: instead of
 // partitions cut down to a few tokens and a merge launch, one workgroup per
-// (row, head group) splits the row's keys over its waves and combines their
-// states in LDS (mode 3; the caller's workspace goes unused).  Applies where
-// the VALU kernel runs and the partition above was shortened for the grid.
-// Measured on C1 (8 sequences, 12 heads, head dim 64, fp16, up to 512
-// tokens): step 14.3 us with 32-token partitions and the merge, 12.6 us so.
+// (row, head) splits the row's keys over its waves and combines their states
+// in LDS (the caller's workspace goes unused).  Applies to plain multi-head
+// attention where the partition above was shortened for the grid.  Measured
+// on C1 (8 sequences, 12 heads, head dim 64, fp16, up to 512 tokens): step
+// 14.3 us with 32-token partitions and the merge, 12.6 us so.
 static bool wg_split_applies(int B, int H, int Hkv, int BS, int MB, int kv_dtype, int D) {
-  if (splitmm_serves(kv_dtype, BS, D, H, Hkv)) return false;
-  if ((int64_t)MB * BS > kWgSplitMaxTokens) return false;
-  return default_partition(B, H, Hkv, BS, MB, kv_dtype, D) < valu_partition(H, Hkv);
+  if (H != Hkv || (int64_t)MB * BS > kWgSplitMaxTokens) return false;
+  return default_partition(B, H, Hkv, BS, MB, kv_dtype, D) < kDefaultPartition;
+}
+
+// Decode by explicit splits: the slices that are taken together.  Neighbouring
+// slices are one key range, so several at once write (and merge) fewer
+// states.  `fill` parts in all rows are enough, and at least 512 keys of the
+// longest row that the table holds for a wave of its own; no part gets fewer
+// than 128 (a wave) or 256 (a workgroup of 8).  Against one state per slice,
+// us: 8 sequences of 256..4096 tokens, 12 heads, D 64, fp32 (64 splits) 29 /
+// 25; 16 of them, 32 / 8 heads, bf16 49 / 43; 64 of up to 8192, 32 heads, bf16
+// 553 / 488.
+static int slices_together(int splits, int64_t units, int64_t width, int64_t fill, bool waves) {
+  int64_t parts = ceil_div(fill, units);
+  if (waves) parts = std::max(parts, ceil_div(width, 512));
+  parts = std::min({parts, ceil_div(width, waves ? 128 : 256), (int64_t)splits});
+  return (int)ceil_div(splits, std::max((int64_t)1, parts));
+}
+
+// Multi-head decode in one pass: a workgroup (8 waves) per (row, head) rather
+// than a wave, unless the waves alone fill the device or have little to do.
+// us, a wave / a workgroup per row: 16 sequences of 256..4096 tokens, 12 heads
+// 131 / 32; 64 of up to 8192, 32 heads 724 / 446; 256 of up to 2048, 12 heads
+// 177 / 153; 256 of up to 256 25 / 26.
+static bool wg_per_row(int64_t rows_heads, int64_t width, int cus) {
+  return rows_heads < 4 * (int64_t)cus || (rows_heads < 16 * (int64_t)cus && width > 256);
+}
+
+// Grouped heads that the split-operand kernel does not take (fp32 caches, other
+// block sizes, head dim 256, explicit splits), on the fp32 matrix cores
+// instead of the VALU kernel: 16 columns for G heads, so not for 16-bit caches
+// with G = 2 or 4, where the VALU kernel reads each page once too and does
+// less per byte; but always in one pass, which is a workgroup here and a
+// wave there.  16 sequences of 256..4096 tokens, us VALU / here: 32 / 8 heads
+// fp32 99 / 60, bf16 with 8-token blocks 56 / 59, the same in one pass 613 /
+// 95; 32 / 4 heads bf16 with 32-token blocks 57 / 33; 16 / 1 heads 51 / 16;
+// 8 / 4 heads, D 256, fp16 61 / 67, fp32 117 / 76.
+static bool grouped_on_matrix_cores(int H, int Hkv, int kv_dtype, int num_splits) {
+  const int G = H / Hkv;
+  return G > 1 && (kv_dtype == HS_DTYPE_F32 || G > 4 || row_attn_heads_per_wave(H, Hkv) < G ||
+                   num_splits == 1);
 }
 
 // The workspace queries take no kv dtype: they size for the shortest default
@@ -331,6 +386,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
     return fail(HS_EUNSUPPORTED, "unsupported head_dim " + std::to_string(D));
   if (B == 0) return HS_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int cus = current_cus();
   if (!shared_pages &&
       even_applies(kv_dtype, BS, D, B, H, Hkv, MB, num_splits, partition_tokens)) {
     const int M = splitmm_even_groups(kv_dtype, D, H, Hkv, B, MB);
@@ -365,7 +421,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
     a.even_slots = M + B;
     a.even_min_pages = splitmm_even_min_pages();
     a.qscale = scale * kLog2e;
-    return launch_row_attn(a, kv_dtype, D, st);
+    return launch_row_attn(a, kv_dtype, D, cus, st);
   }
   DecodePlan plan;
   if ((rc = plan_decode(BS, MB, num_splits, partition_tokens,
@@ -403,16 +459,34 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
   a.P = plan.P;
   a.qscale = scale * kLog2e;
   if (!shared_pages || !shared_pages_apply(a, kv_dtype, D)) {
-    // the default decomposition of a small grid of short rows: one
-    // workgroup per row and head group (the workspace, sized for the
-    // partitions above, goes unused)
+    const bool mha = H == Hkv;
+    a.mma = grouped_on_matrix_cores(H, Hkv, kv_dtype, num_splits) &&
+            !splitmm_applies(a, kv_dtype, D) && rows_serves(a, kv_dtype, D);
+    const int64_t width = (int64_t)MB * BS;
     if (num_splits == 0 && partition_tokens == 0 &&
         wg_split_applies(B, H, Hkv, BS, MB, kv_dtype, D)) {
-      a.mode = 3;
-      a.part_tokens = 0;
+      // the workspace, sized for the partitions above, goes unused
+      a.mode = 0;
       a.P = 1;
+      a.wg = 1;
+    } else if (num_splits == 0 && partition_tokens == 0 && a.mma) {
+      a.part_tokens = rows_partition(B, H, Hkv, BS, MB, plan.part_tokens);
+      a.P = (int)ceil_div(width, a.part_tokens);
+    } else if (num_splits == 1) {
+      a.wg = mha && wg_per_row((int64_t)B * H, width, cus);
+    } else if (num_splits > 1) {
+      // workgroups of 8 waves, a few for each CU, or waves, 16 for each CU
+      const int64_t units = a.mma ? sat_mul(B, Hkv, ceil_div(H / Hkv, 16))
+                                  : sat_mul(B, H / row_attn_heads_per_wave(H, Hkv));
+      a.wg = mha && sat_mul(units, num_splits) < 64 * (int64_t)cus;
+      a.slices = slices_together(num_splits, units, width,
+                                 (a.mma ? 2 : a.wg ? 3 : 16) * (int64_t)cus, !a.mma && !a.wg);
+      a.P = (int)ceil_div(num_splits, a.slices);
     }
-    return launch_row_attn(a, kv_dtype, D, st);
+    a.ranked = a.wg && B > 1 && B <= 64 && (int64_t)B * H > cus;
+    const size_t acc = ((size_t)B * H * a.P * D * sizeof(float) + 255) & ~(size_t)255;
+    a.part_ml = a.P > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + acc) : nullptr;
+    return launch_row_attn(a, kv_dtype, D, cus, st);
   }
   SharePlanArgs sp{};
   sp.per_unit = share_per_unit(H, Hkv);
@@ -428,7 +502,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
   sp.units = reinterpret_cast<int4*>(ws + l.units);
   sp.n_units = reinterpret_cast<int32_t*>(ws + l.n_units);
   a.skip = sp.skip;
-  return launch_row_attn(a, kv_dtype, D, st, &sp);
+  return launch_row_attn(a, kv_dtype, D, cus, st, &sp);
 }
 
 }  // namespace hs
@@ -587,10 +661,8 @@ static int prefill_common(const float* q, const int32_t* cu_q, int S, int max_ro
   a.splits = 1;
   a.P = 1;
   a.qscale = scale * kLog2e;
-  int dev = 0;
-  if (rows_prefill_serves(a, kv_dtype, D) && hipGetDevice(&dev) == hipSuccess)
-    return launch_rows_prefill(a, kv_dtype, D, std::max(1, device_cu_count(dev)), st);
-  return launch_row_attn(a, kv_dtype, D, st);
+  if (rows_serves(a, kv_dtype, D)) return launch_rows(a, kv_dtype, D, current_cus(), st);
+  return launch_row_attn(a, kv_dtype, D, current_cus(), st);
 }
 
 int hs_prefill(const float* q, const void* k_cache, const void* v_cache, int kv_dtype,

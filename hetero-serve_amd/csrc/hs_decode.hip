@@ -75,72 +75,86 @@ __attribute__((amdgpu_waves_per_eu(G >= 8 ? 2 : (D > 128 ? 3 : 4)))) void row_at
   }
 }
 
-// Small grids (mode 3): one workgroup per (row, head group of G) walks the
-// whole row, its W waves on W contiguous slices of the keys, and the waves'
-// states are combined through LDS, so a batch too small to fill the CUs gets
-// W times the waves without partition states or a merge launch.  Each wave
-// runs the same RowWalk as the partition kernel; the combine is the
-// log-sum-exp merge of paged_attn_v3.py:170-208 over the slices.
-template <typename T, int D, bool kPaged, int G, int W>
-__global__ __launch_bounds__(W * 64) void row_attn_wg_kernel(RowAttnArgs a) {
-  using Walk = RowWalk<T, D, kPaged, G>;
-  __shared__ float s_m[W][G], s_l[W][G];
-  __shared__ float s_acc[W][G][D];
+// The sequence with the k-th longest context, among a.B <= 64: with more
+// workgroups than CUs, the longest rows start first and the short ones fill in
+// behind them (32 sequences of 64..1024 tokens, 12 heads, fp16: 18 -> 15 us).
+__device__ inline int ranked_row(const RowAttnArgs& a, int k) {
   const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int n_hw = a.H / G;
-  const int row = (int)(blockIdx.x / n_hw);
-  const int h0 = (int)(blockIdx.x % n_hw) * G;
+  const int c = lane < a.B ? a.ctx[lane] : 0;
+  int rank = 0;
+  for (int q = 0; q < a.B; ++q) {
+    const int cq = __builtin_amdgcn_readlane(c, q);
+    rank += cq > c || (cq == c && q < lane);
+  }
+  return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < a.B && rank == k));
+}
+
+// One workgroup per (row, head, partition): its W waves walk W contiguous
+// slices of the keys and their states are combined through LDS, so a batch
+// too small to fill the CUs gets W times the waves without that many
+// partition states.  Each wave runs the same RowWalk as the partition kernel;
+// the combine is the log-sum-exp merge of paged_attn_v3.py:170-208 over the
+// slices.
+template <typename T, int D, bool kPaged, int W>
+__global__ __launch_bounds__(W * 64) void row_attn_wg_kernel(RowAttnArgs a) {
+  using Walk = RowWalk<T, D, kPaged, 1>;
+  __shared__ float s_m[W], s_l[W];
+  __shared__ float s_acc[W][D];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = (int)(blockIdx.x % a.H);
+  const int rp = (int)(blockIdx.x / a.H);
+  const int p = rp % a.P;
+  const int row = a.ranked ? ranked_row(a, rp / a.P) : rp / a.P;
   int b, end;
   if (!row_geometry(a, row, b, end)) return;       // workgroup-uniform
-  const int64_t orow0 = ((int64_t)row * a.H + h0) * D;
-  if (end <= 0) {                                  // nothing to attend to: zero rows
-    for (int d = threadIdx.x; d < G * D; d += W * 64) a.out[orow0 + d] = 0.0f;
+  const int64_t orow = ((int64_t)row * a.H + h) * D;
+  int lo = 0, hi = end, nparts = 1;
+  if (end <= 0) {                                  // nothing to attend to: a zero row
+    if (p == 0)
+      for (int d = threadIdx.x; d < D; d += W * 64) a.out[orow + d] = 0.0f;
     return;
   }
+  if (a.P > 1 && !partition_range(a, end, p, lo, hi, nparts)) return;
   // slices of whole load groups, so that no two waves load the same group
-  const int chunk = ((end + W - 1) / W + Walk::kTpl - 1) / Walk::kTpl * Walk::kTpl;
-  const int lo = wv * chunk;
-  const int hi = min(end, lo + chunk);
+  const int chunk = ((hi - lo + W - 1) / W + Walk::kTpl - 1) / Walk::kTpl * Walk::kTpl;
+  const int first = lo - lo % Walk::kTpl + wv * chunk;
+  const int my_lo = max(lo, first);
+  const int my_hi = wv == W - 1 ? hi : min(hi, first + chunk);
   Walk w;
-  if (lo < hi) {
-    w.run(KvPages{a.k, a.v, a.Hkv, a.BS, a.NB}, a.q + orow0, a.qscale, h0 / (a.H / a.Hkv),
-          a.bt + (int64_t)b * a.MB, lo, hi);
-  } else {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      w.m[g] = kNegBig;
-      w.l[g] = 0.0f;
-#pragma unroll
-      for (int e = 0; e < Walk::kVec; ++e) w.acc[g][e] = 0.0f;
-    }
-  }
+  if (my_lo < my_hi)
+    w.run(KvPages{a.k, a.v, a.Hkv, a.BS, a.NB}, a.q + orow, a.qscale, h / (a.H / a.Hkv),
+          a.bt + (int64_t)b * a.MB, my_lo, my_hi);
+  else
+    w.clear();
   if (Walk::slot(lane) == 0) {
     const int c = Walk::chunk(lane);
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-#pragma unroll
-      for (int e = 0; e < Walk::kVec; ++e) s_acc[wv][g][c * Walk::kVec + e] = w.acc[g][e];
-      if (c == 0) {
-        s_m[wv][g] = w.m[g];
-        s_l[wv][g] = w.l[g];
-      }
+    for (int e = 0; e < Walk::kVec; ++e) s_acc[wv][c * Walk::kVec + e] = w.acc[0][e];
+    if (c == 0) {
+      s_m[wv] = w.m[0];
+      s_l[wv] = w.l[0];
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < G * D; i += W * 64) {
-    const int g = i / D, d = i - g * D;
-    float mm = s_m[0][g];
+  for (int d = threadIdx.x; d < D; d += W * 64) {
+    float mm = s_m[0];
 #pragma unroll
-    for (int v = 1; v < W; ++v) mm = fmaxf(mm, s_m[v][g]);
+    for (int v = 1; v < W; ++v) mm = fmaxf(mm, s_m[v]);
     float l = 0.0f, o = 0.0f;
 #pragma unroll
     for (int v = 0; v < W; ++v) {
-      const float wt = fast_exp2(s_m[v][g] - mm);   // an empty slice: exp2(-3e38 - mm) = 0
-      l = fmaf(s_l[v][g], wt, l);
-      o = fmaf(s_acc[v][g][d], wt, o);
+      const float wt = fast_exp2(s_m[v] - mm);   // an empty slice: exp2(-3e38 - mm) = 0
+      l = fmaf(s_l[v], wt, l);
+      o = fmaf(s_acc[v][d], wt, o);
     }
-    a.out[orow0 + i] = l > 0.0f ? o / l : 0.0f;
+    if (nparts == 1) {
+      a.out[orow + d] = l > 0.0f ? o / l : 0.0f;
+    } else {
+      const int64_t pi = ((int64_t)row * a.H + h) * a.P + p;
+      a.part_acc[pi * D + d] = o;
+      if (d == 0) reinterpret_cast<float2*>(a.part_ml)[pi] = make_float2(mm, l);
+    }
   }
 }
 
@@ -215,11 +229,6 @@ __global__ __launch_bounds__(256) void row_attn_merge_kernel(RowAttnArgs a) {
 // host launch
 // ---------------------------------------------------------------------------
 
-static int elem_vec(int kv_dtype) { return kv_dtype == HS_DTYPE_F32 ? 4 : 8; }
-
-// Tokens one wave-wide load covers for this dtype and head_dim.
-int row_attn_tokens_per_load(int kv_dtype, int D) { return 64 / (D / elem_vec(kv_dtype)); }
-
 // Query heads per wave: the largest of 1, 2, 4, 8 dividing the GQA group.
 int row_attn_heads_per_wave(int H, int Hkv) {
   const int group = H / Hkv;
@@ -250,38 +259,31 @@ static void launch_part(const RowAttnArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((row_attn_part_kernel<T, D, false, G>), grid, block, 0, stream, a);
 }
 
-// Waves of a mode-3 workgroup: 16 (4 per SIMD, at most 128 VGPRs each), or 8
-// where the walk holds more state (G = 8 heads, or head dim 256), as the
-// partition kernel's occupancy hints allow.  The waves' states take
-// W * G * D floats of LDS, 64 KiB at most.
-constexpr int wg_waves(int G, int D) { return G >= 8 || D > 128 ? 8 : 16; }
+// Waves of a row_attn_wg_kernel workgroup.  8 and 16 measured the same on C1
+// (6.0 us) and 8 better where a row is longer (fp32, 4096 tokens: 27 against
+// 33 us): twice the workgroups fit a CU, so the last ones wait less.
+constexpr int kWgWaves = 8;
 
-template <typename T, int D, int G>
+template <typename T, int D>
 static void launch_wg(const RowAttnArgs& a, hipStream_t stream) {
-  constexpr int W = wg_waves(G, D);
+  constexpr int W = kWgWaves;
   const int tpl = 64 / (D / Elem<T>::kVec);
-  // the grid size is checked by the caller
-  const dim3 grid((unsigned)((int64_t)a.rows * (a.H / G))), block(W * 64);
+  const dim3 grid((unsigned)sat_mul(a.rows, a.P, a.H)), block(W * 64);   // checked by the caller
   if (a.BS % tpl == 0)
-    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, true, G, W>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, true, W>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, false, G, W>), grid, block, 0, stream, a);
-}
-
-template <typename T, int D, int G>
-static void launch_mode(const RowAttnArgs& a, hipStream_t stream) {
-  if (a.mode == 3) launch_wg<T, D, G>(a, stream);
-  else launch_part<T, D, G>(a, stream);
+    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, false, W>), grid, block, 0, stream, a);
 }
 
 template <typename T, int D>
 static void launch_typed(const RowAttnArgs& a, hipStream_t stream) {
   profile_begin(stream);
-  switch (row_attn_heads_per_wave(a.H, a.Hkv)) {
-    case 8: launch_mode<T, D, 8>(a, stream); break;
-    case 4: launch_mode<T, D, 4>(a, stream); break;
-    case 2: launch_mode<T, D, 2>(a, stream); break;
-    default: launch_mode<T, D, 1>(a, stream); break;
+  if (a.wg) launch_wg<T, D>(a, stream);
+  else switch (row_attn_heads_per_wave(a.H, a.Hkv)) {
+    case 8: launch_part<T, D, 8>(a, stream); break;
+    case 4: launch_part<T, D, 4>(a, stream); break;
+    case 2: launch_part<T, D, 2>(a, stream); break;
+    default: launch_part<T, D, 1>(a, stream); break;
   }
   profile_end(stream);
 }
@@ -301,12 +303,13 @@ static int launch_dim(const RowAttnArgs& a, int D, hipStream_t stream) {
 // Launch the partition kernel (+ merge when P > 1).  Arguments are validated
 // by the caller.  Grouped-query calls on 16-bit caches with 16-token pages
 // and fixed partitions go to the split-operand matrix-core kernel
-// (hs_decode_splitmm.hip); the rest run the VALU kernel above.  With
+// (hs_decode_splitmm.hip), those with a.mma set to the fp32 matrix cores
+// (hs_prefill_rows.hip); the rest run the VALU kernels above.  With
 // `shared`: the plan kernel, then the shared-page kernel, then the partition
 // kernel (which skips the grouped partitions), then the merge.  The shared
 // kernel runs first, alone: beside the partition kernel its large workgroups
 // waited for whole CUs to drain and finished last.
-int launch_row_attn(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t stream,
+int launch_row_attn(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream,
                     const SharePlanArgs* shared) {
   if (a.mode == 4) {   // even split, then the merge of the rows it cut (hs_decode_splitmm.hip)
     const int64_t gx = sat_mul(a.Hkv, ceil_div(a.H / a.Hkv, 16), a.even_m);
@@ -315,14 +318,16 @@ int launch_row_attn(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t strea
     return check_launch("paged attention");
   }
   const bool splitmm = splitmm_applies(a, kv_dtype, D);
-  int64_t gx;
-  if (splitmm) {
-    gx = splitmm_grid(a);
-  } else {
-    const int G = row_attn_heads_per_wave(a.H, a.Hkv);
-    gx = a.mode == 3 ? sat_mul(a.rows, a.H / G)
-                     : sat_mul(a.rows, a.P, ceil_div(a.H / G, kDecodeWaves));
+  if (a.mma) {
+    const int rc = launch_rows(a, kv_dtype, D, cus, stream);
+    if (rc != HS_OK) return rc;
+    if (a.P > 1) launch_merge(a, D, stream);
+    return check_launch("paged attention");
   }
+  int64_t gx;
+  if (splitmm) gx = splitmm_grid(a);
+  else if (a.wg) gx = sat_mul(a.rows, a.P, a.H);
+  else gx = sat_mul(a.rows, a.P, ceil_div(a.H / row_attn_heads_per_wave(a.H, a.Hkv), kDecodeWaves));
   if (gx <= 0) return HS_OK;
   if (gx > 0x7fffffffLL)
     return fail(HS_EUNSUPPORTED, "grid too large: rows * partitions * head groups = " +

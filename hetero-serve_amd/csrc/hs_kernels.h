@@ -22,10 +22,13 @@ struct RowAttnArgs {
   int S;                  // rows per sequence when cu_q is null
   int B, H, Hkv, BS, MB, NB;
   int mode;               // 0 one pass, 1 fixed partitions, 2 num_splits slices,
-                          // 3 one pass per workgroup, keys split over its waves,
                           // 4 even split (16-bit caches, up to 4 query heads per KV head)
+  int wg;                 // VALU kernel: a workgroup, not a wave, per (row, head, partition)
+  int mma;                // grouped heads on the fp32 matrix cores (hs_prefill_rows.hip)
+  int ranked;             // with wg: rows dealt longest context first (B <= 64)
   int part_tokens;        // mode 1
   int splits;             // mode 2
+  int slices;             // mode 2: neighbouring slices taken together (0 or 1: one)
   int P;                  // partition slots per (row, head) in the grid
   float qscale;           // scale * log2(e)
   const uint8_t* skip;    // [rows * P] or null: partitions the shared-page kernel serves
@@ -72,7 +75,7 @@ __device__ inline bool partition_range(const RowAttnArgs& a, int end, int p, int
   int chunk;
   if (a.mode == 0) chunk = end;
   else if (a.mode == 1) chunk = a.part_tokens;
-  else chunk = (end + a.splits - 1) / a.splits;
+  else chunk = (int)min((int64_t)end, (int64_t)max(1, a.slices) * ((end + a.splits - 1) / a.splits));
   nparts = (end + chunk - 1) / chunk;
   lo = p * chunk;
   hi = min(lo + chunk, end);
@@ -105,7 +108,7 @@ void launch_shared_pages(const RowAttnArgs& a, const SharePlanArgs& s, int kv_dt
 
 // Partition kernel + merge; with `shared`, the plan kernel before and the
 // shared-page kernel between them.
-int launch_row_attn(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t stream,
+int launch_row_attn(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream,
                     const SharePlanArgs* shared = nullptr);
 
 // Grouped-query decode of bf16 and fp16 caches on the matrix cores with split
@@ -128,7 +131,7 @@ struct EvenLayout {
 EvenLayout splitmm_even_layout(int B, int H, int Hkv, int D, int M);
 void launch_splitmm_even(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t stream);
 
-// Query heads one decode wave serves (GQA packing): 1, 2, 4 or 8.
+// Query heads one wave of the VALU kernel serves: 1, 2, 4 or 8.
 int row_attn_heads_per_wave(int H, int Hkv);
 
 int launch_page_copy(const void* pool, void* buf, bool unpack, int L, int NB, int64_t page_bytes,
@@ -150,13 +153,14 @@ int launch_kv_append(void* k_cache, void* v_cache, int kv_dtype, int NB, int BS,
                      const int32_t* seq_ids, int64_t n, const void* k_src, const void* v_src,
                      int src_dtype, int64_t src_row_stride, hipStream_t stream);
 
-// Causal prefill in fp32 arithmetic on the fp32 matrix cores
-// (hs_prefill_rows.hip): a.S rows per sequence, or with a.cu_q ragged rows, at
-// most a.S per sequence, on a device of `cus` CUs.  `serves` is false for sizes
+// Attention in fp32 arithmetic on the fp32 matrix cores (hs_prefill_rows.hip)
+// on a device of `cus` CUs: causal prefill (a.S rows per sequence, or with
+// a.cu_q ragged rows, at most a.S per sequence; a.P == 1), and the partitions
+// of a decode with grouped heads (a.S == 1; the caller merges).  `serves` is false for sizes
 // that its 32-bit offsets and positions cannot hold (a cache of 256 GiB, a table
 // of 2^30 tokens); launch_row_attn's one wave per row takes those.
-bool rows_prefill_serves(const RowAttnArgs& a, int kv_dtype, int D);
-int launch_rows_prefill(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream);
+bool rows_serves(const RowAttnArgs& a, int kv_dtype, int D);
+int launch_rows(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream);
 
 // Matrix-core causal prefill (hs_prefill_mfma.hip).  cu_q null: S rows per
 // sequence, q/out [B, S, H, D]; else ragged rows as in hs_prefill_varlen.

@@ -5,7 +5,10 @@
 // position ctx - S + s and attends to keys [0, that position]; rows at
 // negative positions are zero).  This is hs_prefill*'s use_mfma = 0 path: any
 // cache dtype, any block size, head dims 32 to 256, nothing rounded below
-// fp32 anywhere.
+// fp32 anywhere.  A decode with grouped heads whose cache the split-operand
+// kernel does not take (hs_decode_splitmm.hip) is the same thing with one query
+// and its heads as rows; there a workgroup serves one partition of the keys
+// and writes its state for the merge (hs_decode.hip).
 //
 // What bounds it.  The products run on v_mfma_f32_16x16x4_f32 (64 FLOPs a
 // cycle and SIMD, 157 TFLOP/s over the device at 2.4 GHz), whose 32 cycles
@@ -109,10 +112,11 @@ __device__ inline void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// The rows of row tile `tile` of (sequence b, KV head kvh); every thread of the
-// workgroup calls it (it holds barriers).
+// The rows of row tile `tile` of (sequence b, KV head kvh) against the keys of
+// partition p (decode; prefill has one partition, all keys); every thread of
+// the workgroup calls it (it holds barriers).
 template <typename T, int D, int NT, int W>
-__device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
+__device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, int p) {
   const RowAttnArgs& a = ra.a;
   constexpr int kRows = kKeys * NT;
   constexpr int kRow = D + 4;                    // floats of a staged row: 16-byte reads of 16
@@ -154,9 +158,12 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
     const int s = query_of(r);
     return (((int64_t)row0 + s) * a.H + kvh * G + (r - s * G)) * D;
   };
-  const int hi = row_end(min(r_first + kRows, n_rows) - 1);   // rows see more keys as r grows
+  const int end = row_end(min(r_first + kRows, n_rows) - 1);   // rows see more keys as r grows
   const int seen_by_all = row_end(r_first);
-  if (hi <= 0) {
+  int lo = 0, hi = end, nparts = 1;
+  if (a.P > 1 && end > 0 && !partition_range(a, end, p, lo, hi, nparts)) return;
+  if (end <= 0) {
+    if (p > 0) return;
     for (int i = tid; i < kRows * (D / 4); i += 64 * W) {
       const int r = r_first + i / (D / 4);
       if (r < n_rows)
@@ -167,17 +174,17 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
   }
 
   // ---- the tiles of this wave: wv, wv + W, ... ------------------------------
-  const int n_kt = (hi + kKeys - 1) / kKeys;
+  const int n_kt = (hi - lo + kKeys - 1) / kKeys;
   const int32_t* bt = a.bt + (int64_t)b * a.MB;
   const uint32_t tok_units = (uint32_t)(a.Hkv * (D * (int)sizeof(T) / 64));   // 64-byte units
   const char* kbase = static_cast<const char*>(a.k) + (int64_t)kvh * D * (int)sizeof(T) +
                       (lane % kLpr) * 16;
   const char* vbase = static_cast<const char*>(a.v) +
                       ((int64_t)kvh * D + kVE * j) * (int)sizeof(T);
-  // Where key 16 n + j lies in the cache, in 64-byte units (a key past the last
-  // is read as the last).  The launcher keeps the cache within 32 bits of them.
+  // Where key lo + 16 n + j lies in the cache, in 64-byte units (a key past the
+  // last is read as the last).  The launcher keeps the cache within 32 bits of them.
   auto slot_of = [&](int n) -> uint32_t {
-    const int t = min(n * kKeys + j, hi - 1);
+    const int t = min(lo + n * kKeys + j, hi - 1);
     const int blk = ra.bs_shift >= 0 ? t >> ra.bs_shift : t / a.BS;
     return ((uint32_t)safe_block(bt[blk], a.NB) * (uint32_t)a.BS + (uint32_t)(t - blk * a.BS)) *
            tok_units;
@@ -224,7 +231,7 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const int r = r_first + t * kKeys + j;
-    lim[t] = r < n_rows ? row_end(r) : 0;
+    lim[t] = r < n_rows ? min(row_end(r), hi) : 0;
   }
   __syncthreads();
 
@@ -260,7 +267,7 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
     // S^T: lane (j, g) gets keys 4 g + i of row j of each row tile.  kAcc
     // accumulators per row tile, summed at the end: short chains of dependent
     // products, and of roundings.
-    constexpr int kAcc = NT == 1 ? 4 : 2;
+    constexpr int kAcc = NT > 1 ? 2 : D >= 128 ? 8 : 4;
     float4x sa[NT][kAcc];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
@@ -273,21 +280,26 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
       for (int t = 0; t < NT; ++t) {
         const float4 qf =
             *reinterpret_cast<const float4*>(&qs[t * kKeys + j][g * (D / 4) + 4 * c]);
-        sa[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf.x, sa[t][0], 0, 0, 0);
-        sa[t][1 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf.y, sa[t][1 % kAcc], 0, 0, 0);
-        sa[t][2 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf.z, sa[t][2 % kAcc], 0, 0, 0);
-        sa[t][3 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf.w, sa[t][3 % kAcc], 0, 0, 0);
+        float4x* acc = &sa[t][4 * c % kAcc];
+        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf.x, acc[0], 0, 0, 0);
+        acc[1 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf.y, acc[1 % kAcc], 0, 0, 0);
+        acc[2 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf.z, acc[2 % kAcc], 0, 0, 0);
+        acc[3 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf.w, acc[3 % kAcc], 0, 0, 0);
       }
     }
     float4x s[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-      s[t] = kAcc == 4 ? (sa[t][0] + sa[t][1]) + (sa[t][2] + sa[t][3 % kAcc])
-                       : sa[t][0] + sa[t][1];
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int n2 = kAcc / 2; n2 > 0; n2 /= 2)
+#pragma unroll
+        for (int c = 0; c < n2; ++c) sa[t][c] += sa[t][c + n2];
+      s[t] = sa[t][0];
+    }
     wave_lds_fence();
 
-    const int t0 = n * kKeys;
-    const bool masked = t0 + kKeys > seen_by_all;   // wave-uniform
+    const int t0 = lo + n * kKeys;
+    const bool masked = t0 + kKeys > min(seen_by_all, hi);   // wave-uniform
     float p[NT][4];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -325,18 +337,21 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
       one_by_one = __builtin_amdgcn_ballot_w64(chk != 0.0f) != 0;   // NaN != 0
     }
     if (!one_by_one) {
-      // O^T += V^T . P^T: output tile (u, e) holds dims 16 kVE u + kVE row + e
+      // O^T += V^T . P^T: output tile (u, e) holds dims 16 kVE u + kVE row + e.
+      // The 16 keys are summed by themselves first: a wave's sum over its keys
+      // then has one rounding per tile and not one per key.
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int u = 0; u < kNV; ++u)
 #pragma unroll
-        for (int u = 0; u < kNV; ++u)
+        for (int e = 0; e < kVE; ++e)
 #pragma unroll
-          for (int e = 0; e < kVE; ++e) {
-            const float vf = word_elem<T>(vr[i][u], e);
+          for (int t = 0; t < NT; ++t) {
+            float4x sum = float4x{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
-              o[t][u * kVE + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf, p[t][i],
-                                                                      o[t][u * kVE + e], 0, 0, 0);
+            for (int i = 0; i < 4; ++i)
+              sum = __builtin_amdgcn_mfma_f32_16x16x4f32(word_elem<T>(vr[i][u], e), p[t][i], sum,
+                                                         0, 0, 0);
+            o[t][u * kVE + e] += sum;
           }
     } else {
 #pragma unroll 1
@@ -383,7 +398,7 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
     for (int w = 0; w < W; ++w)
       ll += wave_l[w][t * kKeys + j] * fast_exp2(wave_m[w][t * kKeys + j] - mm);
     const float sc = fast_exp2(m[t] - mm);
-    const float inv = ll > 0.0f ? 1.0f / ll : 0.0f;
+    const float inv = nparts > 1 ? 1.0f : ll > 0.0f ? 1.0f / ll : 0.0f;
     // row j of the tile, this wave's part; its K rows are no longer needed
 #pragma unroll
     for (int u = 0; u < kNV; ++u)
@@ -392,7 +407,13 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
 #pragma unroll
         for (int e = 0; e < kVE; ++e)
           ks[wv][j][16 * kVE * u + kVE * (4 * g + i) + e] = o[t][u * kVE + e][i] * sc;
-    if (wv == 0 && g == 0) inv_l[j] = inv;
+    if (wv == 0 && g == 0) {
+      inv_l[j] = inv;
+      const int r = r_first + t * kKeys + j;
+      if (nparts > 1 && r < n_rows)   // decode: one query, row r is head r of the group
+        reinterpret_cast<float2*>(a.part_ml)[((int64_t)b * a.H + kvh * G + r) * a.P + p] =
+            make_float2(mm, ll);
+    }
     __syncthreads();
     for (int i = tid; i < kKeys * (D / 4); i += 64 * W) {
       const int rr = i / (D / 4), c = 4 * (i % (D / 4));
@@ -404,9 +425,12 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile) {
       }
       const float f = inv_l[rr];
       const int r = r_first + t * kKeys + rr;
-      if (r < n_rows)
-        *reinterpret_cast<float4*>(a.out + out_row(r) + c) =
-            make_float4(x.x * f, x.y * f, x.z * f, x.w * f);
+      if (r < n_rows) {
+        float* dst = nparts > 1
+                         ? a.part_acc + (((int64_t)b * a.H + kvh * G + r) * a.P + p) * D + c
+                         : a.out + out_row(r) + c;
+        *reinterpret_cast<float4*>(dst) = make_float4(x.x * f, x.y * f, x.z * f, x.w * f);
+      }
     }
     __syncthreads();
   }
@@ -421,9 +445,11 @@ __global__ __launch_bounds__(64 * W) void rows_prefill_kernel(RowsArgs ra) {
   const int b = pair / a.Hkv;
   const int kvh = pair - b * a.Hkv;
   const int rows = (a.cu_q ? a.cu_q[b + 1] - a.cu_q[b] : a.S) * (a.H / a.Hkv);
+  const int tp = wg / n_pairs;
+  const int p = tp % a.P;
   // heaviest first; the step is for a ragged sequence of more than a.S rows
-  for (int tile = ra.n_tiles - 1 - wg / n_pairs; tile * kKeys * NT < rows; tile += ra.n_tiles)
-    rows_tile<T, D, NT, W>(ra, b, kvh, tile);
+  for (int tile = ra.n_tiles - 1 - tp / a.P; tile * kKeys * NT < rows; tile += ra.n_tiles)
+    rows_tile<T, D, NT, W>(ra, b, kvh, tile, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -436,14 +462,14 @@ void launch_shape(const RowAttnArgs& a, int64_t rows_per_pair, int cus, hipStrea
   ra.a = a;
   ra.n_tiles = (int)ceil_div(rows_per_pair, kKeys * NT);
   ra.bs_shift = (a.BS & (a.BS - 1)) == 0 ? __builtin_ctz((unsigned)a.BS) : -1;
-  const int64_t n_wg = (int64_t)ra.n_tiles * a.B * a.Hkv;
+  const int64_t n_wg = (int64_t)ra.n_tiles * a.B * a.Hkv * a.P;
   // More than one workgroup per CU but not two: the hardware deals the first
   // round out to all CUs and the second to the first of them again, so with
   // the first round reversed those hold its lightest workgroups (and not its
   // heaviest) beside the second's.  Only where two workgroups fit a CU
   // together (their registers, up to head dim 64).  GPT-2's 512-token chunk,
   // 384 workgroups: 26.4 -> 23.7 us.
-  ra.reversed = D <= 64 && n_wg > cus && n_wg <= 2 * (int64_t)cus ? cus : 0;
+  ra.reversed = D <= 64 && a.P == 1 && n_wg > cus && n_wg <= 2 * (int64_t)cus ? cus : 0;
   const dim3 grid((unsigned)n_wg), block(64 * W);
   hipLaunchKernelGGL((rows_prefill_kernel<T, D, NT, W>), grid, block, 0, stream, ra);
 }
@@ -483,15 +509,15 @@ void launch_t(const RowAttnArgs& a, int D, int64_t rows_per_pair, int cus, hipSt
 
 }  // namespace
 
-bool rows_prefill_serves(const RowAttnArgs& a, int kv_dtype, int D) {
+bool rows_serves(const RowAttnArgs& a, int kv_dtype, int D) {
   const int elem = kv_dtype == HS_DTYPE_F32 ? 4 : 2;
-  const int64_t tiles = sat_mul(ceil_div(sat_mul(a.S, a.H / a.Hkv), kKeys), a.B, a.Hkv);
+  const int64_t tiles = sat_mul(ceil_div(sat_mul(a.S, a.H / a.Hkv), kKeys), a.B, a.Hkv, a.P);
   return tiles > 0 && tiles <= 0x7fffffffLL && sat_mul(a.S, a.H / a.Hkv) <= (1LL << 30) &&
          sat_mul(a.NB, a.BS, (int64_t)a.Hkv * (D * elem / 64)) <= 0xffffffffLL &&
          sat_mul(a.MB, a.BS) <= (1LL << 30);
 }
 
-int launch_rows_prefill(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream) {
+int launch_rows(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream) {
   const int64_t rows_per_pair = (int64_t)a.S * (a.H / a.Hkv);
   profile_begin(stream);
   if (kv_dtype == HS_DTYPE_F32) launch_t<float>(a, D, rows_per_pair, cus, stream);

@@ -181,6 +181,17 @@ struct RowWalk {
     }
   }
 
+  // The empty state (no keys).
+  __device__ inline void clear() {
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      m[g] = kNegBig;
+      l[g] = 0.0f;
+#pragma unroll
+      for (int e = 0; e < kVec; ++e) acc[g][e] = 0.0f;
+    }
+  }
+
   // Head g's result on the lanes of slot 0: normalised into out (dims
   // chunk * kVec ..), or un-normalised with (m, l) as a partition state.
   __device__ inline void store_out(int g, float* out_row) const {

@@ -118,7 +118,8 @@ size_t hs_decode_workspace_bytes(int B, int H, int Hkv, int D, int BS, int MB, i
  *   num_splits   1  = one pass per (sequence, head)               (v2)
  *                >1 = the context cut into num_splits slices of
  *                     ceil(ctx_b / num_splits) tokens, then an
- *                     log-sum-exp merge                            (v3)
+ *                     log-sum-exp merge (neighbouring slices may be
+ *                     computed, and merged, as one)                (v3)
  *                0  = fixed partitions of partition_tokens tokens
  *                     plus the merge (the fast default; with
  *                     partition_tokens == 0, a small grid of rows of at most

@@ -1,0 +1,108 @@
+"""Decode paths that give a (row, head) or a KV head's group a workgroup: plain
+multi-head attention in one pass and by splits (8 waves a row, rows dealt
+longest first, several slices taken together), and grouped heads on the fp32
+matrix cores (default partitions, one pass, splits), at the edges of their
+key tiles, slices and partitions.
+
+Tolerance.  fp32 throughout: as in test_prefill_rows_gpu.py, 1e-6 in the
+2-norm against fp64.
+"""
+
+from __future__ import annotations
+
+import math
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+REL = 1e-6
+
+
+def _case(ctxs, H, Hkv, D, BS, dtype, seed=0):
+    rng = np.random.default_rng(seed)
+    need = [-(-max(n, 0) // BS) for n in ctxs]
+    width = max(max(need), 1) + 1
+    ids = rng.permutation(sum(need) + 2)
+    bt = np.full((len(ctxs), width), -1, dtype=np.int32)
+    at = 0
+    for i, k in enumerate(need):
+        bt[i, :k] = ids[at:at + k]
+        at += k
+    gen = torch.Generator().manual_seed(seed)
+    k, v = (torch.randn((sum(need) + 2, BS, Hkv, D), generator=gen).to(dtype) for _ in range(2))
+    return (torch.randn((len(ctxs), H, D), generator=gen), k, v, torch.from_numpy(bt),
+            torch.tensor(ctxs, dtype=torch.int32), 1.0 / math.sqrt(D))
+
+
+def _want(q, k, v, bt, ctx, scale):
+    out = torch.zeros(q.shape, dtype=torch.float64)
+    g = q.shape[1] // k.shape[2]
+    for b, n in enumerate(ctx.tolist()):
+        n = min(n, bt.shape[1] * k.shape[1])
+        if n <= 0:
+            continue
+        pages = bt[b, :-(-n // k.shape[1])].long()
+        kk, vv = (x[pages].reshape(-1, *x.shape[2:])[:n].double().repeat_interleave(g, 1)
+                  for x in (k, v))
+        p = torch.softmax(torch.einsum("hd,nhd->hn", q[b].double(), kk) * scale, -1)
+        out[b] = torch.einsum("hn,nhd->hd", p, vv)
+    return out
+
+
+def _runs(case, splits=(0, 1, 2, 7, 64)):
+    from heteroserve import _hip
+
+    dev = [x.to(DEV) if torch.is_tensor(x) else x for x in case]
+    want = _want(*case)
+    for s in splits:
+        got = _hip.decode(*dev, num_splits=s).cpu().double()
+        err = ((got - want).norm() / want.norm()).item()
+        assert err <= REL, (s, err)
+        assert torch.equal(got[case[4] <= 0], torch.zeros_like(got[case[4] <= 0])), s
+
+
+EDGES = [0, 1, 15, 16, 17, 127, 128, 129, -3, 300, 1031]
+
+
+@pytest.mark.parametrize("dtype,H,Hkv,D,BS", [
+    (torch.float32, 8, 2, 64, 16), (torch.float32, 6, 2, 128, 5), (torch.float32, 4, 2, 256, 16),
+    (torch.float32, 3, 1, 32, 8), (torch.bfloat16, 10, 2, 128, 8), (torch.float16, 40, 2, 64, 32),
+    (torch.float16, 16, 1, 256, 16), (torch.bfloat16, 8, 2, 64, 3), (torch.float16, 4, 2, 256, 16)])
+def test_grouped_heads(dtype, H, Hkv, D, BS):
+    """fp32 caches, groups above 4 or of 3 (one or several row tiles), and 16-bit
+    groups of 2 and 4, which leave the VALU kernel in one pass only."""
+    _runs(_case(EDGES, H, Hkv, D, BS, dtype))
+
+
+@pytest.mark.parametrize("dtype,D,BS", [(torch.float16, 64, 16), (torch.float32, 128, 16),
+                                        (torch.bfloat16, 256, 5), (torch.float32, 32, 3)])
+def test_multi_head_rows(dtype, D, BS):
+    """A workgroup per row: slices that start inside a load group, empty waves."""
+    _runs(_case(EDGES, 5, 5, D, BS, dtype))
+
+
+def test_longest_rows_first():
+    """More workgroups than CUs: rows are dealt by rank, equal lengths and empty
+    rows among them (64 sequences is the most that are ranked)."""
+    ctxs = [(37 * i) % 200 for i in range(60)] + [77, 77, 0, 512]
+    _runs(_case(ctxs, 6, 6, 64, 16, torch.float16, seed=1), splits=(0, 1, 3))
+    _runs(_case(ctxs + [9], 6, 6, 64, 16, torch.float16, seed=2), splits=(0, 1, 3))
+
+
+@pytest.mark.parametrize("splits", [0, 1, 5])
+def test_values_past_the_context(splits):
+    """Stale infinities and NaN in the last page reach no row."""
+    from heteroserve import _hip
+
+    case = _case([21, 40], 8, 2, 64, 16, torch.float32, seed=3)
+    q, k, v, bt, ctx, scale = case
+    want = _want(*case)
+    for b, n in enumerate((21, 40)):
+        for x in (k, v):
+            x[bt[b, n // 16], n % 16:] = math.nan if b else math.inf
+    got = _hip.decode(*(x.to(DEV) for x in (q, k, v, bt, ctx)), scale, num_splits=splits).cpu()
+    assert ((got.double() - want).norm() / want.norm()).item() <= REL
