@@ -10,6 +10,7 @@
 #include <unordered_map>
 
 #include "hs_kernels.h"
+#include "hs_private.h"
 
 namespace hs {
 
@@ -746,6 +747,13 @@ static int check_kv_write(void* k_cache, void* v_cache, int kv_dtype, int Hkv, i
   return HS_OK;
 }
 
+// Rows of one layer, contiguous but for the row stride.
+static KvWrite one_layer(void* k_cache, void* v_cache, int kv_dtype, int Hkv, int D, int64_t n,
+                         const void* k_src, const void* v_src, int src_dtype,
+                         int64_t src_row_stride) {
+  return {k_cache, v_cache, kv_dtype, Hkv, D, 1, 0, k_src, v_src, src_dtype, 0, D, src_row_stride, n};
+}
+
 int hs_kv_scatter(void* k_cache, void* v_cache, int kv_dtype, int64_t num_slots, int Hkv, int D,
                   const int64_t* slots, int64_t n, const void* k_src, const void* v_src,
                   int src_dtype, int64_t src_row_stride, void* stream) {
@@ -755,9 +763,28 @@ int hs_kv_scatter(void* k_cache, void* v_cache, int kv_dtype, int64_t num_slots,
   if (num_slots <= 0) return fail(HS_EINVAL, "num_slots must be positive");
   if (n == 0) return HS_OK;
   if (!slots) return fail(HS_EINVAL, "null pointer");
-  return launch_kv_scatter(k_cache, v_cache, kv_dtype, num_slots, (int64_t)Hkv * D, slots, n,
-                           k_src, v_src, src_dtype, src_row_stride,
-                           static_cast<hipStream_t>(stream));
+  return launch_kv_scatter(one_layer(k_cache, v_cache, kv_dtype, Hkv, D, n, k_src, v_src, src_dtype,
+                                     src_row_stride),
+                           num_slots, slots, false, static_cast<hipStream_t>(stream));
+}
+
+int hs_kv_scatter_layers(void* k_cache, void* v_cache, int kv_dtype, int64_t num_slots, int Hkv,
+                         int D, int L, int64_t cache_layer_stride, const int64_t* slots, int64_t n,
+                         const void* k_src, const void* v_src, int src_dtype,
+                         int64_t src_layer_stride, int64_t src_head_stride,
+                         int64_t src_row_stride, void* stream) {
+  // the strides may come in any order, so only their signs are checked
+  const int rc = check_kv_write(k_cache, v_cache, kv_dtype, Hkv, D, n, k_src, v_src, src_dtype,
+                                INT64_MAX);
+  if (rc != HS_OK) return rc;
+  if (num_slots <= 0 || L <= 0) return fail(HS_EINVAL, "num_slots and L must be positive");
+  if (cache_layer_stride < 0 || src_layer_stride < 0 || src_head_stride < 0 || src_row_stride < 0)
+    return fail(HS_EINVAL, "strides must not be negative");
+  if (n == 0) return HS_OK;
+  if (!slots) return fail(HS_EINVAL, "null pointer");
+  const KvWrite w = {k_cache, v_cache, kv_dtype, Hkv, D, L, cache_layer_stride, k_src, v_src,
+                     src_dtype, src_layer_stride, src_head_stride, src_row_stride, n};
+  return launch_kv_scatter(w, num_slots, slots, true, static_cast<hipStream_t>(stream));
 }
 
 int hs_kv_append(void* k_cache, void* v_cache, int kv_dtype, int NB, int BS, int Hkv, int D,
@@ -771,9 +798,9 @@ int hs_kv_append(void* k_cache, void* v_cache, int kv_dtype, int NB, int BS, int
     return fail(HS_EINVAL, "append sizes must be positive");
   if (n == 0) return HS_OK;
   if (!block_tables || !positions) return fail(HS_EINVAL, "null pointer");
-  return launch_kv_append(k_cache, v_cache, kv_dtype, NB, BS, (int64_t)Hkv * D, block_tables, B,
-                          MB,
-                          positions, seq_ids, n, k_src, v_src, src_dtype, src_row_stride,
+  return launch_kv_append(one_layer(k_cache, v_cache, kv_dtype, Hkv, D, n, k_src, v_src, src_dtype,
+                                    src_row_stride),
+                          NB, BS, block_tables, B, MB, positions, seq_ids,
                           static_cast<hipStream_t>(stream));
 }
 

@@ -140,19 +140,24 @@ int launch_page_copy(const void* pool, void* buf, bool unpack, int L, int NB, in
 int launch_gather_rows(const void* cache, int NB, int BS, int64_t row_bytes, const int32_t* bt,
                        int MB, int B, int length, void* out, hipStream_t stream);
 
-// New K/V rows into the cache (hs_kvwrite.hip): rows of row_elems elements,
-// source rows src_row_stride elements apart, cast to the cache dtype.
-int launch_kv_scatter(void* k_cache, void* v_cache, int kv_dtype, int64_t num_slots,
-                      int64_t row_elems, const int64_t* slots, int64_t n, const void* k_src,
-                      const void* v_src, int src_dtype, int64_t src_row_stride, hipStream_t stream);
+// New K/V rows into the cache (hs_kvwrite.hip): n rows of Hkv * D elements for
+// each of `layers` caches, cast to the cache dtype.  Strides in elements.
+struct KvWrite {
+  void *k_cache, *v_cache;
+  int kv_dtype;
+  int Hkv, D, layers;
+  int64_t cache_layer;                      // between layers of a cache
+  const void *k_src, *v_src;
+  int src_dtype;
+  int64_t src_layer, src_head, src_row;     // between layers, heads, rows of a source
+  int64_t n;
+};
+int launch_kv_scatter(const KvWrite& w, int64_t num_slots, const int64_t* slots, bool wrap,
+                      hipStream_t stream);
+int launch_kv_append(const KvWrite& w, int NB, int BS, const int32_t* bt, int B, int MB,
+                     const int32_t* positions, const int32_t* seq_ids, hipStream_t stream);
 int launch_block_tables(const int32_t* packed, int B, int width, int32_t* out,
                         hipStream_t stream);
-int launch_kv_append(void* k_cache, void* v_cache, int kv_dtype, int NB, int BS,
-                     int64_t row_elems, const int32_t* bt, int B, int MB,
-                     const int32_t* positions,
-                     const int32_t* seq_ids, int64_t n, const void* k_src, const void* v_src,
-                     int src_dtype, int64_t src_row_stride, hipStream_t stream);
-
 // Attention in fp32 arithmetic on the fp32 matrix cores (hs_prefill_rows.hip)
 // on a device of `cus` CUs: causal prefill (a.S rows per sequence, or with
 // a.cu_q ragged rows, at most a.S per sequence; a.P == 1), and the partitions

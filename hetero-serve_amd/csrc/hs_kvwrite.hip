@@ -8,9 +8,10 @@
 //
 // One token row is Hkv * D elements.  A thread converts and moves 8
 // elements (16 bytes of a 16-bit cache), so a D = 128 head row is one
-// 16-lane group and a wave covers 4 heads; K and V are grid.y = 0 / 1 of one
-// launch.  The source may be a strided view (rows of the fused QKV output),
-// so the source row stride is a parameter.  Casts round like torch's
+// 16-lane group and a wave covers 4 heads; K and V, and the layers of a call
+// that writes several, are the y index of one launch.  The source may be a
+// strided view (rows of the fused QKV output, or a [layers, heads, tokens, D]
+// array), so its strides are parameters.  Casts round like torch's
 // `.to()`: fp32 -> bf16 and -> fp16 to nearest even, NaN to the canonical
 // quiet NaN torch produces; equal types are copied bit for bit.
 //
@@ -129,10 +130,12 @@ struct RowMap {
   const int32_t* seq_ids;      //              [n] row -> sequence, or null (row i = sequence i)
   int64_t num_slots;           // NB * BS
   int NB, BS, B, MB;           // B: table rows; a sequence index must be below it
+  int wrap;                    // scatter form: negative slots count from the end
 
   __device__ int64_t slot(int64_t i) const {
     if (slots) {
-      const int64_t s = slots[i];
+      int64_t s = slots[i];
+      if (wrap && s < 0) s += num_slots;
       return (s >= 0 && s < num_slots) ? s : -1;
     }
     const int64_t b = seq_ids ? seq_ids[i] : i;
@@ -144,91 +147,102 @@ struct RowMap {
   }
 };
 
-// grid.x covers n rows x (row / 8) chunks; grid.y = 0 (K) / 1 (V).
+// What one launch writes: n rows of heads * dim elements into each of the
+// layers' K and V caches (a row that is contiguous in the source counts as one
+// head).
+struct WriteArgs {
+  uint8_t *k_cache, *v_cache;
+  const uint8_t *k_src, *v_src;
+  int64_t cache_layer, src_layer, src_head, src_row;   // bytes
+  int64_t n;
+  int heads, dim;
+  RowMap map;
+};
+
+// Row i and element e of it, of the flat index g over rows of `per` units of
+// kUnit elements: 32-bit division where the index fits, since a 64-bit one is
+// most of this kernel's instructions.
+template <int kUnit>
+__device__ inline void split_index(int64_t g, int64_t total, uint32_t per, int64_t& i, int& e) {
+  if (total <= 0xffffffffLL) {   // uniform
+    const uint32_t r = (uint32_t)g / per;
+    i = r;
+    e = (int)((uint32_t)g - r * per) * kUnit;
+  } else {
+    i = g / per;
+    e = (int)(g - i * per) * kUnit;
+  }
+}
+
+// Element e of a row lies in head e / dim; its byte offset in the source row.
+__device__ inline int64_t src_offset(const WriteArgs& a, int e, int elem_bytes) {
+  if (a.heads == 1) return (int64_t)e * elem_bytes;
+  const uint32_t h = (uint32_t)e / (uint32_t)a.dim;
+  return h * a.src_head + (int64_t)(e - (int)h * a.dim) * elem_bytes;
+}
+
+// grid.x covers n rows x (row / 8) chunks; grid.y = 2 * layer + (0: K, 1: V).
 template <typename S, typename C>
-__global__ __launch_bounds__(kWriteThreads) void kv_write_kernel(
-    uint8_t* k_cache, uint8_t* v_cache, const uint8_t* k_src, const uint8_t* v_src,
-    int64_t src_stride_bytes, int64_t row_elems, int64_t n, RowMap map) {
-  const int64_t chunks = row_elems / 8;
+__global__ __launch_bounds__(kWriteThreads) void kv_write_kernel(WriteArgs a) {
+  const uint32_t chunks = (uint32_t)(a.heads * a.dim / 8);
   const int64_t g = (int64_t)blockIdx.x * kWriteThreads + threadIdx.x;
-  if (g >= n * chunks) return;
-  const int64_t i = g / chunks;
-  const int64_t c = g - i * chunks;
-  const int64_t slot = map.slot(i);
+  if (g >= a.n * chunks) return;
+  int64_t i;
+  int e;
+  split_index<8>(g, a.n * chunks, chunks, i, e);
+  const int64_t slot = a.map.slot(i);
   if (slot < 0) return;
-  const uint8_t* src = (blockIdx.y ? v_src : k_src) + i * src_stride_bytes + c * 8 * Codec<S>::kBytes;
-  uint8_t* dst = (blockIdx.y ? v_cache : k_cache) + (slot * row_elems + c * 8) * Codec<C>::kBytes;
-  float x[8];
-  Codec<S>::load8(src, x);
-  Codec<C>::store8(dst, x);
+  const int layer = blockIdx.y >> 1;
+  const uint8_t* src = ((blockIdx.y & 1) ? a.v_src : a.k_src) + layer * a.src_layer +
+                       i * a.src_row + src_offset(a, e, Codec<S>::kBytes);
+  uint8_t* dst = ((blockIdx.y & 1) ? a.v_cache : a.k_cache) + layer * a.cache_layer +
+                 (slot * ((int64_t)a.heads * a.dim) + e) * Codec<C>::kBytes;
+  if constexpr (std::is_same<S, C>::value) {   // a bit copy (NaN payloads included)
+#pragma unroll
+    for (int b = 0; b < 8 * Codec<C>::kBytes; b += 16)
+      *reinterpret_cast<uint4*>(dst + b) = load16(src + b);
+  } else {
+    float x[8];
+    Codec<S>::load8(src, x);
+    Codec<C>::store8(dst, x);
+  }
 }
 
 // Any alignment: one element per thread.
 template <typename S, typename C>
-__global__ __launch_bounds__(kWriteThreads) void kv_write_scalar_kernel(
-    uint8_t* k_cache, uint8_t* v_cache, const uint8_t* k_src, const uint8_t* v_src,
-    int64_t src_stride_bytes, int64_t row_elems, int64_t n, RowMap map) {
+__global__ __launch_bounds__(kWriteThreads) void kv_write_scalar_kernel(WriteArgs a) {
+  const uint32_t row = (uint32_t)(a.heads * a.dim);
   const int64_t g = (int64_t)blockIdx.x * kWriteThreads + threadIdx.x;
-  if (g >= n * row_elems) return;
-  const int64_t i = g / row_elems;
-  const int64_t e = g - i * row_elems;
-  const int64_t slot = map.slot(i);
+  if (g >= a.n * row) return;
+  int64_t i;
+  int e;
+  split_index<1>(g, a.n * row, row, i, e);
+  const int64_t slot = a.map.slot(i);
   if (slot < 0) return;
-  const uint8_t* src = (blockIdx.y ? v_src : k_src) + i * src_stride_bytes + e * Codec<S>::kBytes;
-  uint8_t* dst = (blockIdx.y ? v_cache : k_cache) + (slot * row_elems + e) * Codec<C>::kBytes;
+  const int layer = blockIdx.y >> 1;
+  const uint8_t* src = ((blockIdx.y & 1) ? a.v_src : a.k_src) + layer * a.src_layer +
+                       i * a.src_row + src_offset(a, e, Codec<S>::kBytes);
+  uint8_t* dst = ((blockIdx.y & 1) ? a.v_cache : a.k_cache) + layer * a.cache_layer +
+                 (slot * (int64_t)row + e) * Codec<C>::kBytes;
   Codec<C>::store1(dst, Codec<S>::load1(src));
 }
 
-// Equal types: bit copy (NaN payloads included), 16 bytes per thread.
-template <int kBytes>
-__global__ __launch_bounds__(kWriteThreads) void kv_copy_kernel(
-    uint8_t* k_cache, uint8_t* v_cache, const uint8_t* k_src, const uint8_t* v_src,
-    int64_t src_stride_bytes, int64_t row_elems, int64_t n, RowMap map) {
-  const int64_t row_bytes = row_elems * kBytes;
-  const int64_t pieces = row_bytes / 16;
-  const int64_t g = (int64_t)blockIdx.x * kWriteThreads + threadIdx.x;
-  if (g >= n * pieces) return;
-  const int64_t i = g / pieces;
-  const int64_t c = g - i * pieces;
-  const int64_t slot = map.slot(i);
-  if (slot < 0) return;
-  const uint8_t* src = (blockIdx.y ? v_src : k_src) + i * src_stride_bytes + c * 16;
-  uint8_t* dst = (blockIdx.y ? v_cache : k_cache) + slot * row_bytes + c * 16;
-  *reinterpret_cast<uint4*>(dst) = load16(src);
-}
-
 template <typename S, typename C>
-void launch_pair(uint8_t* kc, uint8_t* vc, const uint8_t* ks, const uint8_t* vs,
-                 int64_t stride_bytes, int64_t row_elems, int64_t n, const RowMap& map,
-                 bool vec, hipStream_t stream) {
-  if (vec) {
-    if (std::is_same<S, C>::value && (row_elems * Codec<C>::kBytes) % 16 == 0) {
-      const int64_t work = n * (row_elems * Codec<C>::kBytes / 16);
-      const dim3 grid((unsigned)((work + kWriteThreads - 1) / kWriteThreads), 2);
-      hipLaunchKernelGGL((kv_copy_kernel<Codec<C>::kBytes>), grid, dim3(kWriteThreads), 0, stream, kc,
-                         vc, ks, vs, stride_bytes, row_elems, n, map);
-    } else {
-      const int64_t work = n * (row_elems / 8);
-      const dim3 grid((unsigned)((work + kWriteThreads - 1) / kWriteThreads), 2);
-      hipLaunchKernelGGL((kv_write_kernel<S, C>), grid, dim3(kWriteThreads), 0, stream, kc, vc,
-                         ks, vs, stride_bytes, row_elems, n, map);
-    }
-  } else {
-    const int64_t work = n * row_elems;
-    const dim3 grid((unsigned)((work + kWriteThreads - 1) / kWriteThreads), 2);
-    hipLaunchKernelGGL((kv_write_scalar_kernel<S, C>), grid, dim3(kWriteThreads), 0, stream, kc,
-                       vc, ks, vs, stride_bytes, row_elems, n, map);
-  }
+void launch_pair(const WriteArgs& a, int layers, bool vec, hipStream_t stream) {
+  const int64_t work = a.n * ((int64_t)a.heads * a.dim / (vec ? 8 : 1));
+  const dim3 grid((unsigned)((work + kWriteThreads - 1) / kWriteThreads), 2 * layers);
+  if (vec)
+    hipLaunchKernelGGL((kv_write_kernel<S, C>), grid, dim3(kWriteThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((kv_write_scalar_kernel<S, C>), grid, dim3(kWriteThreads), 0, stream, a);
 }
 
 template <typename S>
-int launch_src(int kv_dtype, uint8_t* kc, uint8_t* vc, const uint8_t* ks, const uint8_t* vs,
-               int64_t stride_bytes, int64_t row_elems, int64_t n, const RowMap& map, bool vec,
-               hipStream_t stream) {
+int launch_src(int kv_dtype, const WriteArgs& a, int layers, bool vec, hipStream_t stream) {
   switch (kv_dtype) {
-    case HS_DTYPE_F32: launch_pair<S, float>(kc, vc, ks, vs, stride_bytes, row_elems, n, map, vec, stream); break;
-    case HS_DTYPE_F16: launch_pair<S, _Float16>(kc, vc, ks, vs, stride_bytes, row_elems, n, map, vec, stream); break;
-    case HS_DTYPE_BF16: launch_pair<S, Bf16>(kc, vc, ks, vs, stride_bytes, row_elems, n, map, vec, stream); break;
+    case HS_DTYPE_F32: launch_pair<S, float>(a, layers, vec, stream); break;
+    case HS_DTYPE_F16: launch_pair<S, _Float16>(a, layers, vec, stream); break;
+    case HS_DTYPE_BF16: launch_pair<S, Bf16>(a, layers, vec, stream); break;
     default: return fail(HS_EINVAL, "unsupported KV cache dtype code " + std::to_string(kv_dtype));
   }
   return HS_OK;
@@ -238,33 +252,47 @@ int dtype_bytes(int code) { return code == HS_DTYPE_F32 ? 4 : 2; }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-int launch_kv_write(void* k_cache, void* v_cache, int kv_dtype, const void* k_src,
-                    const void* v_src, int src_dtype, int64_t src_row_stride, int64_t row_elems,
-                    int64_t n, const RowMap& map, hipStream_t stream) {
-  if (n == 0) return HS_OK;
-  const int64_t sb = dtype_bytes(src_dtype), cb = dtype_bytes(kv_dtype);
-  const int64_t stride_bytes = sat_mul(src_row_stride, sb);
-  if (stride_bytes == INT64_MAX || sat_mul(n, stride_bytes) == INT64_MAX ||
-      sat_mul(map.num_slots, row_elems, cb) == INT64_MAX)
+// Strides in elements.
+int launch_kv_write(const KvWrite& w, const RowMap& map, hipStream_t stream) {
+  if (w.n == 0) return HS_OK;
+  const int64_t sb = dtype_bytes(w.src_dtype), cb = dtype_bytes(w.kv_dtype);
+  const int64_t row_elems = (int64_t)w.Hkv * w.D;
+  const int64_t row_b = sat_mul(w.src_row, sb), head_b = sat_mul(w.src_head, sb),
+                layer_b = sat_mul(w.src_layer, sb), cache_b = sat_mul(w.cache_layer, cb);
+  if (sat_add(sat_add(sat_mul(w.n, row_b), sat_mul(w.Hkv, head_b)), sat_mul(w.layers, layer_b)) ==
+          INT64_MAX ||
+      sat_add(sat_mul(map.num_slots, row_elems, cb), sat_mul(w.layers, cache_b)) == INT64_MAX)
     return fail(HS_EUNSUPPORTED, "KV write sizes too large for 64-bit offsets");
-  // the vector kernels need 16-byte aligned 8-element groups on both sides
-  const bool vec = row_elems % 8 == 0 && aligned16(k_src) && aligned16(v_src) &&
-                   aligned16(k_cache) && aligned16(v_cache) && stride_bytes % 16 == 0 &&
-                   (row_elems * cb) % 16 == 0;
-  const int64_t work = sat_mul(n, row_elems);
-  if (ceil_div(work, kWriteThreads) > 0x7fffffffLL)
+  const bool one_head = w.src_head == w.D || w.Hkv == 1;   // the row is contiguous in the source
+  // the vector kernel needs 16-byte aligned 8-element groups on both sides
+  const bool vec = (one_head ? row_elems : w.D) % 8 == 0 && aligned16(w.k_src) &&
+                   aligned16(w.v_src) && aligned16(w.k_cache) && aligned16(w.v_cache) &&
+                   row_b % 16 == 0 && (one_head || head_b % 16 == 0) && layer_b % 16 == 0 &&
+                   cache_b % 16 == 0 && (row_elems * cb) % 16 == 0;
+  const int64_t work = sat_mul(w.n, row_elems);
+  if (row_elems > 0x7fffffffLL || ceil_div(work, kWriteThreads) > 0x7fffffffLL ||
+      w.layers > 32767)
     return fail(HS_EUNSUPPORTED, "KV write too large for one launch");
-  auto* kc = static_cast<uint8_t*>(k_cache);
-  auto* vc = static_cast<uint8_t*>(v_cache);
-  const auto* ks = static_cast<const uint8_t*>(k_src);
-  const auto* vs = static_cast<const uint8_t*>(v_src);
+  WriteArgs a;
+  a.k_cache = static_cast<uint8_t*>(w.k_cache);
+  a.v_cache = static_cast<uint8_t*>(w.v_cache);
+  a.k_src = static_cast<const uint8_t*>(w.k_src);
+  a.v_src = static_cast<const uint8_t*>(w.v_src);
+  a.cache_layer = cache_b;
+  a.src_layer = layer_b;
+  a.src_head = head_b;
+  a.src_row = row_b;
+  a.n = w.n;
+  a.heads = one_head ? 1 : w.Hkv;
+  a.dim = one_head ? (int)row_elems : w.D;
+  a.map = map;
   int rc;
   profile_begin(stream);
-  switch (src_dtype) {
-    case HS_DTYPE_F32: rc = launch_src<float>(kv_dtype, kc, vc, ks, vs, stride_bytes, row_elems, n, map, vec, stream); break;
-    case HS_DTYPE_F16: rc = launch_src<_Float16>(kv_dtype, kc, vc, ks, vs, stride_bytes, row_elems, n, map, vec, stream); break;
-    case HS_DTYPE_BF16: rc = launch_src<Bf16>(kv_dtype, kc, vc, ks, vs, stride_bytes, row_elems, n, map, vec, stream); break;
-    default: rc = fail(HS_EINVAL, "unsupported source dtype code " + std::to_string(src_dtype));
+  switch (w.src_dtype) {
+    case HS_DTYPE_F32: rc = launch_src<float>(w.kv_dtype, a, w.layers, vec, stream); break;
+    case HS_DTYPE_F16: rc = launch_src<_Float16>(w.kv_dtype, a, w.layers, vec, stream); break;
+    case HS_DTYPE_BF16: rc = launch_src<Bf16>(w.kv_dtype, a, w.layers, vec, stream); break;
+    default: rc = fail(HS_EINVAL, "unsupported source dtype code " + std::to_string(w.src_dtype));
   }
   profile_end(stream);
   if (rc != HS_OK) return rc;
@@ -297,22 +325,17 @@ int launch_block_tables(const int32_t* packed, int B, int width, int32_t* out,
   return check_launch("block table build");
 }
 
-int launch_kv_scatter(void* k_cache, void* v_cache, int kv_dtype, int64_t num_slots,
-                      int64_t row_elems, const int64_t* slots, int64_t n, const void* k_src,
-                      const void* v_src, int src_dtype, int64_t src_row_stride,
+int launch_kv_scatter(const KvWrite& w, int64_t num_slots, const int64_t* slots, bool wrap,
                       hipStream_t stream) {
   RowMap map{};
   map.slots = slots;
   map.num_slots = num_slots;
-  return launch_kv_write(k_cache, v_cache, kv_dtype, k_src, v_src, src_dtype, src_row_stride,
-                         row_elems, n, map, stream);
+  map.wrap = wrap;
+  return launch_kv_write(w, map, stream);
 }
 
-int launch_kv_append(void* k_cache, void* v_cache, int kv_dtype, int NB, int BS,
-                     int64_t row_elems, const int32_t* bt, int B, int MB,
-                     const int32_t* positions,
-                     const int32_t* seq_ids, int64_t n, const void* k_src, const void* v_src,
-                     int src_dtype, int64_t src_row_stride, hipStream_t stream) {
+int launch_kv_append(const KvWrite& w, int NB, int BS, const int32_t* bt, int B, int MB,
+                     const int32_t* positions, const int32_t* seq_ids, hipStream_t stream) {
   RowMap map{};
   map.bt = bt;
   map.positions = positions;
@@ -322,8 +345,7 @@ int launch_kv_append(void* k_cache, void* v_cache, int kv_dtype, int NB, int BS,
   map.BS = BS;
   map.B = B;
   map.MB = MB;
-  return launch_kv_write(k_cache, v_cache, kv_dtype, k_src, v_src, src_dtype, src_row_stride,
-                         row_elems, n, map, stream);
+  return launch_kv_write(w, map, stream);
 }
 
 }  // namespace hs

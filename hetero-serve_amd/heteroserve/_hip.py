@@ -81,6 +81,13 @@ _SIGNATURES = {
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
+# entry points of this layer's own; must match csrc/hs_private.h
+_PRIVATE = {
+    "hs_kv_scatter_layers": (_c_int, [_c_vp, _c_vp, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_i64,
+                                      _c_vp, _c_i64, _c_vp, _c_vp, _c_int, _c_i64, _c_i64, _c_i64,
+                                      _c_vp]),
+}
+
 
 def lib_path() -> Path:
     env = os.environ.get("HETEROSERVE_HIP_LIB")
@@ -90,7 +97,7 @@ def lib_path() -> Path:
 def open_library(path: Optional[Path] = None) -> ctypes.CDLL:
     """dlopen libhsattn.so and bind its signatures.  Needs no GPU."""
     lib = ctypes.CDLL(str(path or lib_path()))
-    for name, (res, args) in _SIGNATURES.items():
+    for name, (res, args) in {**_SIGNATURES, **_PRIVATE}.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
@@ -490,8 +497,9 @@ def _same_rows(k, v, Hkv: int, D: int):
     return k, v, ks
 
 
-def kv_scatter(k_cache, v_cache, slots, k, v) -> None:
-    """k_cache.view(-1, Hkv, D)[slots] = k.to(cache dtype); same for v."""
+def kv_scatter(k_cache, v_cache, slots, k, v, wrap: bool = False) -> None:
+    """k_cache.view(-1, Hkv, D)[slots] = k.to(cache dtype); same for v.  wrap:
+    negative slots count from the end (otherwise they are skipped)."""
     L = lib("KV scatter HIP kernel")
     (NB, BS, Hkv, D), index = _check_write(k_cache, v_cache, k, v)
     k, v, stride = _same_rows(k, v, Hkv, D)
@@ -500,9 +508,41 @@ def kv_scatter(k_cache, v_cache, slots, k, v) -> None:
         raise RuntimeError(f"{slots.numel()} slots for {n} rows")
     slots = torch.as_tensor(slots).to(device=k_cache.device, dtype=torch.int64).contiguous()
     with _DeviceGuard(index):
-        check(L.hs_kv_scatter(k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype),
-                              NB * BS, Hkv, D, slots.data_ptr(), n, k.data_ptr(), v.data_ptr(),
-                              dtype_code(k.dtype), stride, _stream_at(index)))
+        head = (k_cache.data_ptr(), v_cache.data_ptr(), dtype_code(k_cache.dtype), NB * BS, Hkv, D)
+        rows = (slots.data_ptr(), n, k.data_ptr(), v.data_ptr(), dtype_code(k.dtype))
+        if wrap:
+            check(L.hs_kv_scatter_layers(*head, 1, 0, *rows, 0, D, stride, _stream_at(index)))
+        else:
+            check(L.hs_kv_scatter(*head, *rows, stride, _stream_at(index)))
+
+
+def kv_scatter_layers(pool, slots, k, v) -> None:
+    """pool[l, 0].view(-1, Hkv, D)[slots] = k[l].transpose(0, 1) for every layer of
+    pool [L, 2, NB, BS, Hkv, D] and k, v [>= L, Hkv, T, D], in one launch;
+    negative slots count from the end."""
+    lib_ = lib("KV scatter HIP kernel")
+    L, _, NB, BS, Hkv, D = pool.shape
+    (_, _, _, _), index = _check_write(pool[0, 0], pool[0, 1], k, v)
+    T = slots.numel()
+    for x in (k, v):
+        if x.shape[0] < L:
+            raise IndexError(f"index {x.shape[0]} is out of bounds for dimension 0 with size "
+                             f"{x.shape[0]}")
+        if tuple(x.shape[1:]) != (Hkv, T, D):
+            raise RuntimeError(f"K/V must be [{L}, {Hkv}, {T}, {D}], got {tuple(x.shape)}")
+    if k.dtype != v.dtype:
+        raise RuntimeError("k and v rows must have the same count and dtype")
+    if k.stride() != v.stride() or k.stride(3) != 1:
+        k, v = k.contiguous(), v.contiguous()
+    # a dim of one index has no stride of its own
+    sl, sh, st = (k.stride(i) if k.shape[i] > 1 else n for i, n in
+                  enumerate((Hkv * T * D, T * D, D)))
+    slots = slots.to(device=pool.device, dtype=torch.int64).contiguous()
+    with _DeviceGuard(index):
+        check(lib_.hs_kv_scatter_layers(
+            pool.data_ptr(), pool[0, 1].data_ptr(), dtype_code(pool.dtype), NB * BS, Hkv, D, L,
+            2 * NB * BS * Hkv * D, slots.data_ptr(), T, k.data_ptr(), v.data_ptr(),
+            dtype_code(k.dtype), sl, sh, st, _stream_at(index)))
 
 
 def kv_append(k_cache, v_cache, block_tables, positions, k, v, seq_ids=None) -> None:

@@ -28,6 +28,8 @@ up by inheritance:
 
 from __future__ import annotations
 
+import operator
+
 from .. import _hip
 
 
@@ -192,8 +194,7 @@ def scatter_kv(k_cache, v_cache, slots, k, v) -> None:
         if lo < -n_slots or hi >= n_slots:
             bad = lo if lo < -n_slots else hi
             raise IndexError(f"index {bad} is out of bounds for dimension 0 with size {n_slots}")
-    slots = torch.where(slots < 0, slots + n_slots, slots)
-    _hip.kv_scatter(k_cache, v_cache, slots, k, v)
+    _hip.kv_scatter(k_cache, v_cache, slots, k, v, wrap=True)
 
 
 def append_kv(k_cache, v_cache, block_tables, positions, k, v, seq_ids=None) -> None:
@@ -211,21 +212,20 @@ def append_kv(k_cache, v_cache, block_tables, positions, k, v, seq_ids=None) -> 
 def write_kv(pool, block_ids, start_pos: int, k, v) -> None:
     """``TorchBlockAllocator.write_kv`` (torch_blocks.py:89-106): scatter
     ``[L, Hkv, T, D]`` K/V of one sequence into every layer of the pool at
-    positions ``start_pos .. start_pos + T - 1``; one launch per layer."""
+    positions ``start_pos .. start_pos + T - 1``; one launch for all layers,
+    which reads K and V in the layout they come in."""
     import torch
 
     _check_pool(pool)
-    L, _, NB, BS, H, D = pool.shape
+    BS = pool.shape[3]
     k = torch.as_tensor(k, device=pool.device)
     v = torch.as_tensor(v, device=pool.device)
     T = int(k.shape[2])
     if T == 0:
         return
-    slots = slots_for(block_ids, range(start_pos, start_pos + T), BS).to(pool.device)
-    kt = k.permute(0, 2, 1, 3).contiguous()      # [L, T, H, D]: token-major rows
-    vt = v.permute(0, 2, 1, 3).contiguous()
-    for layer in range(L):
-        scatter_kv(pool[layer, 0], pool[layer, 1], slots, kt[layer], vt[layer])
+    start = operator.index(start_pos)
+    slots = slots_for(block_ids, torch.arange(start, start + T), BS)
+    _hip.kv_scatter_layers(pool, slots, k, v)
 
 
 def block_table_tensor(tables, pad_to=None, device="cuda"):
