@@ -702,24 +702,35 @@ size_t hs_prefill_workspace_bytes(int B, int max_seqlen_q, int H, int D, int use
   return need == INT64_MAX ? 0 : (size_t)need;
 }
 
+static int page_copy(const void* pool, int L, int NB, int64_t page_bytes, const int64_t* ids, int n,
+                     const void* buf, bool unpack, bool host_ids, void* stream) {
+  if (n < 0 || L <= 0 || NB <= 0 || page_bytes <= 0)
+    return fail(HS_EINVAL, unpack ? "unpack sizes must be positive" : "pack sizes must be positive");
+  if (n == 0) return HS_OK;
+  if (!pool || !ids || !buf) return fail(HS_EINVAL, "null pointer");
+  const auto launch = host_ids ? launch_page_copy_host_ids : launch_page_copy;
+  return launch(pool, const_cast<void*>(buf), unpack, L, NB, page_bytes, ids, n,
+                static_cast<hipStream_t>(stream));
+}
+
 int hs_kv_pack(const void* pool, int L, int NB, int64_t page_bytes, const int64_t* block_ids,
                int n, void* out, void* stream) {
-  if (n < 0 || L <= 0 || NB <= 0 || page_bytes <= 0)
-    return fail(HS_EINVAL, "pack sizes must be positive");
-  if (n == 0) return HS_OK;
-  if (!pool || !block_ids || !out) return fail(HS_EINVAL, "null pointer");
-  return launch_page_copy(pool, out, false, L, NB, page_bytes, block_ids, n,
-                          static_cast<hipStream_t>(stream));
+  return page_copy(pool, L, NB, page_bytes, block_ids, n, out, false, false, stream);
 }
 
 int hs_kv_unpack(void* pool, int L, int NB, int64_t page_bytes, const int64_t* block_ids, int n,
                  const void* in, void* stream) {
-  if (n < 0 || L <= 0 || NB <= 0 || page_bytes <= 0)
-    return fail(HS_EINVAL, "unpack sizes must be positive");
-  if (n == 0) return HS_OK;
-  if (!pool || !block_ids || !in) return fail(HS_EINVAL, "null pointer");
-  return launch_page_copy(pool, const_cast<void*>(in), true, L, NB, page_bytes, block_ids, n,
-                          static_cast<hipStream_t>(stream));
+  return page_copy(pool, L, NB, page_bytes, block_ids, n, in, true, false, stream);
+}
+
+int hs_kv_pack_host_ids(const void* pool, int L, int NB, int64_t page_bytes,
+                        const int64_t* host_ids, int n, void* out, void* stream) {
+  return page_copy(pool, L, NB, page_bytes, host_ids, n, out, false, true, stream);
+}
+
+int hs_kv_unpack_host_ids(void* pool, int L, int NB, int64_t page_bytes, const int64_t* host_ids,
+                          int n, const void* in, void* stream) {
+  return page_copy(pool, L, NB, page_bytes, host_ids, n, in, true, true, stream);
 }
 
 int hs_kv_gather(const void* cache, int NB, int BS, int64_t row_bytes, const int32_t* block_tables,

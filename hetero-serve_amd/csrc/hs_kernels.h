@@ -137,6 +137,11 @@ int row_attn_heads_per_wave(int H, int Hkv);
 int launch_page_copy(const void* pool, void* buf, bool unpack, int L, int NB, int64_t page_bytes,
                      const int64_t* ids, int n, hipStream_t stream);
 
+// The same with at most HS_KV_HOST_IDS (hs_private.h) ids in host memory.
+int launch_page_copy_host_ids(const void* pool, void* buf, bool unpack, int L, int NB,
+                              int64_t page_bytes, const int64_t* host_ids, int n,
+                              hipStream_t stream);
+
 int launch_gather_rows(const void* cache, int NB, int BS, int64_t row_bytes, const int32_t* bt,
                        int MB, int B, int length, void* out, hipStream_t stream);
 

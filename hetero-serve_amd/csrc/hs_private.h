@@ -31,6 +31,17 @@ int hs_kv_scatter_layers(void* k_cache, void* v_cache, int kv_dtype, int64_t num
                          int64_t src_layer_stride, int64_t src_head_stride,
                          int64_t src_row_stride, void* stream);
 
+/*
+ * hs_kv_pack and hs_kv_unpack with at most HS_KV_HOST_IDS block ids in host
+ * memory, which are read before the call returns and travel in the kernel's
+ * arguments (of at most 4 KiB): nothing to upload, and a capture holds the ids.
+ */
+#define HS_KV_HOST_IDS 896
+int hs_kv_pack_host_ids(const void* pool, int L, int NB, int64_t page_bytes,
+                        const int64_t* host_ids, int n, void* out, void* stream);
+int hs_kv_unpack_host_ids(void* pool, int L, int NB, int64_t page_bytes, const int64_t* host_ids,
+                          int n, const void* in, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

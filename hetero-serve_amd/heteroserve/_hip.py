@@ -83,6 +83,8 @@ EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 # entry points of this layer's own; must match csrc/hs_private.h
 _PRIVATE = {
+    "hs_kv_pack_host_ids": (_c_int, [_c_vp, _c_int, _c_int, _c_i64, _c_vp, _c_int, _c_vp, _c_vp]),
+    "hs_kv_unpack_host_ids": (_c_int, [_c_vp, _c_int, _c_int, _c_i64, _c_vp, _c_int, _c_vp, _c_vp]),
     "hs_kv_scatter_layers": (_c_int, [_c_vp, _c_vp, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_i64,
                                       _c_vp, _c_i64, _c_vp, _c_vp, _c_int, _c_i64, _c_i64, _c_i64,
                                       _c_vp]),
@@ -414,24 +416,49 @@ def choose_num_splits(num_seqs: int, num_heads: int, max_context: int) -> int:
     return int(s)
 
 
+HOST_IDS = 896   # most block ids that fit a kernel's arguments (csrc/hs_private.h)
+
+
+def _pages(pool):
+    """(layers, blocks, bytes of one page) of pool [L, 2, NB, BS, Hkv, D]."""
+    Ls, _, NB, BS, H, D = pool.shape
+    return Ls, NB, BS * H * D * pool.element_size()
+
+
 def kv_pack(pool, ids_dev, out) -> None:
     """out[n, L, 2, page] = pool[L, 2, NB, page][:, :, ids]  (bitwise)."""
     L = lib("KV pack HIP kernel")
-    Ls, _, NB = pool.shape[:3]
-    page = pool[0, 0, 0].numel() * pool.element_size()
-    with _DeviceGuard(pool.get_device()):
-        check(L.hs_kv_pack(pool.data_ptr(), Ls, NB, page, ids_dev.data_ptr(), ids_dev.numel(),
-                           out.data_ptr(), _stream_at(pool.get_device())))
+    index = pool.get_device()
+    with _DeviceGuard(index):
+        check(L.hs_kv_pack(pool.data_ptr(), *_pages(pool), ids_dev.data_ptr(), ids_dev.numel(),
+                           out.data_ptr(), _stream_at(index)))
 
 
 def kv_unpack(pool, ids_dev, src) -> None:
     """pool[:, :, ids[i]] = src[i]  (bitwise; ids must not repeat)."""
     L = lib("KV unpack HIP kernel")
-    Ls, _, NB = pool.shape[:3]
-    page = pool[0, 0, 0].numel() * pool.element_size()
-    with _DeviceGuard(pool.get_device()):
-        check(L.hs_kv_unpack(pool.data_ptr(), Ls, NB, page, ids_dev.data_ptr(),
-                             ids_dev.numel(), src.data_ptr(), _stream_at(pool.get_device())))
+    index = pool.get_device()
+    with _DeviceGuard(index):
+        check(L.hs_kv_unpack(pool.data_ptr(), *_pages(pool), ids_dev.data_ptr(),
+                             ids_dev.numel(), src.data_ptr(), _stream_at(index)))
+
+
+def kv_pack_host_ids(pool, ids, out) -> None:
+    """kv_pack with at most HOST_IDS ids in a contiguous int64 numpy array."""
+    L = lib("KV pack HIP kernel")
+    index = pool.get_device()
+    with _DeviceGuard(index):
+        check(L.hs_kv_pack_host_ids(pool.data_ptr(), *_pages(pool), ids.ctypes.data, ids.size,
+                                    out.data_ptr(), _stream_at(index)))
+
+
+def kv_unpack_host_ids(pool, ids, src) -> None:
+    """kv_unpack with at most HOST_IDS ids in a contiguous int64 numpy array."""
+    L = lib("KV unpack HIP kernel")
+    index = pool.get_device()
+    with _DeviceGuard(index):
+        check(L.hs_kv_unpack_host_ids(pool.data_ptr(), *_pages(pool), ids.ctypes.data, ids.size,
+                                      src.data_ptr(), _stream_at(index)))
 
 
 def kv_gather(cache, block_tables_dev, length: int, out) -> None:

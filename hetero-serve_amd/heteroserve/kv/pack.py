@@ -69,11 +69,16 @@ def _normalise_ids(block_ids, num_blocks: int):
     return np.where(ids < 0, ids + num_blocks, ids)
 
 
-def _ids_tensor(ids, device):
+def _ids_array(ids):
     import numpy as np
+
+    return np.ascontiguousarray(ids, dtype=np.int64)
+
+
+def _ids_tensor(ids, device):
     import torch
 
-    return torch.from_numpy(np.ascontiguousarray(ids, dtype=np.int64)).to(device)
+    return torch.from_numpy(_ids_array(ids)).to(device)
 
 
 def _check_pool(pool) -> None:
@@ -94,7 +99,9 @@ def export_blocks_device(pool, block_ids):
     ids = _normalise_ids(block_ids, pool.shape[2])
     L, _, _, BS, H, D = pool.shape
     out = torch.empty((len(ids), L, 2, BS, H, D), dtype=pool.dtype, device=pool.device)
-    if len(ids):
+    if 0 < len(ids) <= _hip.HOST_IDS:
+        _hip.kv_pack_host_ids(pool, _ids_array(ids), out)
+    elif len(ids):
         _hip.kv_pack(pool, _ids_tensor(ids, pool.device), out)
     return out
 
@@ -128,7 +135,10 @@ def write_blocks_device(pool, block_ids, payload) -> None:
         ids = ids[last]
         data = data[torch.from_numpy(last).to(data.device)]
     data = data[: len(ids)].contiguous()
-    _hip.kv_unpack(pool, _ids_tensor(ids, pool.device), data)
+    if len(ids) <= _hip.HOST_IDS:
+        _hip.kv_unpack_host_ids(pool, _ids_array(ids), data)
+    else:
+        _hip.kv_unpack(pool, _ids_tensor(ids, pool.device), data)
 
 
 def gather_kv_batch(pool, tables, length: int, layer: int):
