@@ -203,17 +203,21 @@ static bool wg_per_row(int64_t rows_heads, int64_t width, int cus) {
 
 // Grouped heads that the split-operand kernel does not take (fp32 caches, other
 // block sizes, head dim 256, explicit splits), on the fp32 matrix cores
-// instead of the VALU kernel: 16 columns for G heads, so not for 16-bit caches
-// with G = 2 or 4, where the VALU kernel reads each page once too and does
-// less per byte; but always in one pass, which is a workgroup here and a
-// wave there.  16 sequences of 256..4096 tokens, us VALU / here: 32 / 8 heads
-// fp32 99 / 60, bf16 with 8-token blocks 56 / 59, the same in one pass 613 /
-// 95; 32 / 4 heads bf16 with 32-token blocks 57 / 33; 16 / 1 heads 51 / 16;
-// 8 / 4 heads, D 256, fp16 61 / 67, fp32 117 / 76.
-static bool grouped_on_matrix_cores(int H, int Hkv, int kv_dtype, int num_splits) {
+// instead of the VALU kernel: a workgroup per KV head and partition, 16
+// columns for G heads.  With G = 2 or 4 the VALU kernel reads each page once
+// too and does less per byte, so it keeps 16-bit caches, and fp32 ones once
+// there is a workgroup for every CU and its waves fill the device; but in one
+// pass it has a single wave per row.  Sequences of 256..4096 tokens, us VALU /
+// here: 32 / 8 heads fp32, 8 / 16 / 24 / 32 / 64 sequences 93 / 35, 99 / 61,
+// 122 / 100, 124 / 129, 250 / 286; 16 of them in bf16 with 8-token blocks 56 /
+// 59, in one pass 613 / 95; 32 / 4 heads fp32, 16 / 64 sequences 103 / 35, 223 /
+// 140; 16 / 1 heads 94 / 18; 8 / 4 heads, D 256, fp32, 32 / 64 sequences 225 /
+// 144, 268 / 280.
+static bool grouped_on_matrix_cores(int B, int H, int Hkv, int kv_dtype, int num_splits, int cus) {
   const int G = H / Hkv;
-  return G > 1 && (kv_dtype == HS_DTYPE_F32 || G > 4 || row_attn_heads_per_wave(H, Hkv) < G ||
-                   num_splits == 1);
+  if (G == 1) return false;
+  if (G > 4 || row_attn_heads_per_wave(H, Hkv) < G || num_splits == 1) return true;
+  return kv_dtype == HS_DTYPE_F32 && sat_mul(B, Hkv) < cus;
 }
 
 // The workspace queries take no kv dtype: they size for the shortest default
@@ -461,7 +465,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
   a.qscale = scale * kLog2e;
   if (!shared_pages || !shared_pages_apply(a, kv_dtype, D)) {
     const bool mha = H == Hkv;
-    a.mma = grouped_on_matrix_cores(H, Hkv, kv_dtype, num_splits) &&
+    a.mma = grouped_on_matrix_cores(B, H, Hkv, kv_dtype, num_splits, cus) &&
             !splitmm_applies(a, kv_dtype, D) && rows_serves(a, kv_dtype, D);
     const int64_t width = (int64_t)MB * BS;
     if (num_splits == 0 && partition_tokens == 0 &&
