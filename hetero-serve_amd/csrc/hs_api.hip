@@ -425,6 +425,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
     a.even_m = M;
     a.even_slots = M + B;
     a.even_min_pages = splitmm_even_min_pages();
+    a.even_hw = splitmm_even_heads(H, Hkv);
     a.qscale = scale * kLog2e;
     return launch_row_attn(a, kv_dtype, D, cus, st);
   }

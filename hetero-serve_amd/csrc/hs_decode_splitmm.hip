@@ -175,6 +175,13 @@ __device__ inline float sum_across_groups(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Orders a wave's LDS accesses for the compiler (the hardware keeps them in
+// order).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <int D>
 struct PageWalk {
   static constexpr int kDC = D / 8;           // 16-byte chunks per head row
@@ -237,6 +244,46 @@ __device__ inline void page_walk(const RowAttnArgs& a, PageLds<D>& w, int kvh, i
   int idn = npages > kWindow ? bt[min(page0 + kWindow + lane, a.MB - 1)] : 0;
   int win = 0;
 
+  const int64_t tok = (int64_t)a.Hkv * D;          // elements between tokens of a page
+  // Page addresses: a wave-uniform base (scalar registers) plus one 32-bit
+  // lane offset shared by all loads of a page.
+  const uint16_t* kbase = reinterpret_cast<const uint16_t*>(a.k) + kvh * D;
+  const uint16_t* vbase = reinterpret_cast<const uint16_t*>(a.v) + kvh * D;
+  const uint32_t loff = (uint32_t)(slot * tok + 8 * ck) * 2u;   // bytes; < 16 * tok * 2
+
+  typename W::Regs rg;
+  // Loads of page pg of the range (pg < npages).  A wave's pages increase by
+  // step < kWindow, so they enter the windows one at a time.
+  auto load_page = [&](typename W::Regs& r, int pg) {
+    if (pg / kWindow != win) {   // wave-uniform
+      win = pg / kWindow;
+      idv = idn;
+      idn = kWindow * (win + 1) < npages
+                ? bt[min(page0 + kWindow * (win + 1) + lane, a.MB - 1)] : 0;
+    }
+    const int64_t b0 =
+        safe_block(__builtin_amdgcn_readlane(idv, pg % kWindow), a.NB) * kPage;
+    const char* kp = reinterpret_cast<const char*>(kbase + b0 * tok);
+    const char* vp = reinterpret_cast<const char*>(vbase + b0 * tok);
+#pragma unroll
+    for (int u = 0; u < kLi; ++u)
+      r.k[u] = load16_stream(kp + (int64_t)u * kTpi * tok * 2 + loff);
+#pragma unroll
+    for (int u = 0; u < kLi; ++u)
+      r.v[u] = load16_stream(vp + (int64_t)u * kTpi * tok * 2 + loff);
+  };
+  // Registers -> LDS, rows as loaded.
+  auto store_page = [&](const typename W::Regs& r) {
+#pragma unroll
+    for (int u = 0; u < kLi; ++u) {
+      *reinterpret_cast<uint4*>(&w.k[kTpi * u + slot][8 * ck]) = r.k[u];
+      *reinterpret_cast<uint4*>(&w.v[kTpi * u + slot][8 * ck]) = r.v[u];
+    }
+  };
+
+  // The first page's loads go out before anything waits for the query.
+  if (first < npages) load_page(rg, first);
+
   // Q^T fragments, split: lane l holds column j's dims 32 st + 8 g .. + 7.
   // qexp: the power of two the query was multiplied by (kScaleQ), taken back
   // out of every score.
@@ -291,43 +338,6 @@ __device__ inline void page_walk(const RowAttnArgs& a, PageLds<D>& w, int kvh, i
       }
   }
 
-  const int64_t tok = (int64_t)a.Hkv * D;          // elements between tokens of a page
-  // Page addresses: a wave-uniform base (scalar registers) plus one 32-bit
-  // lane offset shared by all loads of a page.
-  const uint16_t* kbase = reinterpret_cast<const uint16_t*>(a.k) + kvh * D;
-  const uint16_t* vbase = reinterpret_cast<const uint16_t*>(a.v) + kvh * D;
-  const uint32_t loff = (uint32_t)(slot * tok + 8 * ck) * 2u;   // bytes; < 16 * tok * 2
-
-  typename W::Regs rg;
-  // Loads of page pg of the range (pg < npages).  A wave's pages increase by
-  // step < kWindow, so they enter the windows one at a time.
-  auto load_page = [&](typename W::Regs& r, int pg) {
-    if (pg / kWindow != win) {   // wave-uniform
-      win = pg / kWindow;
-      idv = idn;
-      idn = kWindow * (win + 1) < npages
-                ? bt[min(page0 + kWindow * (win + 1) + lane, a.MB - 1)] : 0;
-    }
-    const int64_t b0 =
-        safe_block(__builtin_amdgcn_readlane(idv, pg % kWindow), a.NB) * kPage;
-    const char* kp = reinterpret_cast<const char*>(kbase + b0 * tok);
-    const char* vp = reinterpret_cast<const char*>(vbase + b0 * tok);
-#pragma unroll
-    for (int u = 0; u < kLi; ++u)
-      r.k[u] = load16_stream(kp + (int64_t)u * kTpi * tok * 2 + loff);
-#pragma unroll
-    for (int u = 0; u < kLi; ++u)
-      r.v[u] = load16_stream(vp + (int64_t)u * kTpi * tok * 2 + loff);
-  };
-  // Registers -> LDS, rows as loaded.
-  auto store_page = [&](const typename W::Regs& r) {
-#pragma unroll
-    for (int u = 0; u < kLi; ++u) {
-      *reinterpret_cast<uint4*>(&w.k[kTpi * u + slot][8 * ck]) = r.k[u];
-      *reinterpret_cast<uint4*>(&w.v[kTpi * u + slot][8 * ck]) = r.v[u];
-    }
-  };
-
 #pragma unroll
   for (int d = 0; d < kDT; ++d)
 #pragma unroll
@@ -335,7 +345,6 @@ __device__ inline void page_walk(const RowAttnArgs& a, PageLds<D>& w, int kvh, i
   m = kNegBig;
   l = 0.0f;
 
-  if (first < npages) load_page(rg, first);
   for (int pg = first; pg < npages; pg += step) {
     store_page(rg);
     // the next page's loads fly during this page's arithmetic; none past
@@ -561,18 +570,34 @@ __device__ inline int64_t lane_value64(int64_t x, int l) {
   return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-__device__ inline int64_t wave_sum64(int64_t x) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) x += __shfl_xor(x, off);
-  return lane_value64(x, 0);
+// x of the lane that a DPP control names, 0 where it names none (or where the
+// row mask leaves the row out).
+template <int kCtrl, int kRowMask>
+__device__ inline int64_t dpp64(int64_t x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, kCtrl, kRowMask, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)((uint64_t)x >> 32), kCtrl, kRowMask, 0xF,
+                                             false);
+  return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
-// Tp: the pages of all rows (each wave of the caller computes it).
-__device__ inline int64_t total_pages(const RowAttnArgs& a) {
-  const int lane = threadIdx.x & 63;
-  int64_t tp = 0;
-  for (int c = 0; c < a.B; c += 64) tp += wave_sum64(c + lane < a.B ? row_pages(a, c + lane) : 0);
-  return tp;
+// Inclusive scan over the wave: inside each 16-lane row, then the rows before
+// (row_bcast15 into rows 1 and 3, row_bcast31 into rows 2 and 3).  All in
+// registers: the scan is on the way to a workgroup's first load, where six
+// dependent LDS shuffles of two words each took about a microsecond.
+__device__ inline int64_t wave_scan64(int64_t x) {
+  x += dpp64<0x111, 0xF>(x);   // row_shr:1, 2, 4, 8
+  x += dpp64<0x112, 0xF>(x);
+  x += dpp64<0x114, 0xF>(x);
+  x += dpp64<0x118, 0xF>(x);
+  x += dpp64<0x142, 0xA>(x);   // row_bcast:15
+  x += dpp64<0x143, 0xC>(x);   // row_bcast:31
+  return x;
+}
+
+// a / b for a, b > 0 (wave-uniform): the 64-bit division is a long sequence of
+// its own, needed only for batches of 2^32 pages.
+__device__ inline int64_t div_pages(int64_t a, int64_t b) {
+  return ((uint64_t)(a | b) >> 32) == 0 ? (int64_t)((uint32_t)a / (uint32_t)b) : a / b;
 }
 
 // Q, the pages of a range: Tp cut into at most even_m ranges of at least
@@ -580,22 +605,29 @@ __device__ inline int64_t total_pages(const RowAttnArgs& a) {
 // the grid finds its range empty).
 __device__ inline int64_t range_pages(const RowAttnArgs& a, int64_t tp) {
   const int64_t m = max((int64_t)1, min((int64_t)a.even_m,
-                                        (tp + a.even_min_pages - 1) / a.even_min_pages));
-  return max((int64_t)1, (tp + m - 1) / m);
+                                        div_pages(tp + a.even_min_pages - 1, a.even_min_pages)));
+  return max((int64_t)1, div_pages(tp + m - 1, m));
+}
+
+// The pages of rows c .. c + 63 scanned (inclusive), and this lane's own.
+__device__ inline int64_t scan_rows(const RowAttnArgs& a, int c, int64_t& own) {
+  const int lane = threadIdx.x & 63;
+  own = c + lane < a.B ? row_pages(a, c + lane) : 0;
+  return wave_scan64(own);
 }
 
 // Range wr of the even split: pages [s, e) of the rows laid end to end,
 // and its first row r with R_r, the pages of the rows before it (R_r <= s <
 // R_{r+1}).  Every lane computes the same (scalar) values; false for an
-// empty range.  (The first 64 rows' pages stay in registers between the two
+// empty range.  (The first 64 rows' scan stays in registers between the two
 // passes.)
 __device__ inline bool even_range(const RowAttnArgs& a, int wr, int64_t& s, int64_t& e, int& r,
                                   int64_t& Rr) {
   const int lane = threadIdx.x & 63;
-  const int64_t v0 = lane < a.B ? row_pages(a, lane) : 0;
-  int64_t tp = wave_sum64(v0);
-  for (int c = 64; c < a.B; c += 64)
-    tp += wave_sum64(c + lane < a.B ? row_pages(a, c + lane) : 0);
+  int64_t v0, v;
+  const int64_t inc0 = scan_rows(a, 0, v0);
+  int64_t tp = lane_value64(inc0, 63);
+  for (int c = 64; c < a.B; c += 64) tp += lane_value64(scan_rows(a, c, v), 63);
   const int64_t Q = range_pages(a, tp);
   s = (int64_t)wr * Q;
   e = min(s + Q, tp);
@@ -604,13 +636,8 @@ __device__ inline bool even_range(const RowAttnArgs& a, int wr, int64_t& s, int6
   Rr = tp;
   int64_t base = 0;
   for (int c = 0; c < a.B; c += 64) {
-    const int64_t v = c == 0 ? v0 : (c + lane < a.B ? row_pages(a, c + lane) : 0);
-    int64_t inc = v;                                    // inclusive scan over the chunk
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int64_t y = __shfl_up(inc, off);
-      if (lane >= off) inc += y;
-    }
+    v = v0;
+    const int64_t inc = c == 0 ? inc0 : scan_rows(a, c, v);
     const uint64_t hit = __builtin_amdgcn_ballot_w64(c + lane < a.B && base + inc > s);
     if (hit != 0) {
       const int l0 = __builtin_ctzll(hit);
@@ -623,22 +650,97 @@ __device__ inline bool even_range(const RowAttnArgs& a, int wr, int64_t& s, int6
   return true;
 }
 
-template <typename Ops, int D, bool kCols, int kW>
+// The state of one segment of one KV head, from the nph waves of a workgroup
+// that walked it (waves hsub, hsub + hw, ...): write_unit_state's combine and
+// layout, for hw KV heads side by side.  With one wave per head there is
+// nothing to combine and no barrier; otherwise every wave of the workgroup
+// calls it.
+template <int D, int kW>
+__device__ inline void write_head_state(float4x (&o)[D / 16], float m, float l, int gc, int hsub,
+                                        int ph, int hw, int nph, bool single, float* out_rows,
+                                        float* acc_rows, float* ml, PageLds<D> (&lds)[kW],
+                                        float (&wave_m)[kW][kSlots], float (&wave_l)[kW][kSlots]) {
+  const int lane = threadIdx.x & 63;
+  const int wv = hsub + hw * ph;
+  const int j = lane & 15;
+  const int g = lane >> 4;
+  float lsum = sum_across_groups(l);
+#pragma unroll
+  for (int d = 0; d < D / 16; ++d)   // head j < 8: hi column j plus lo column j + 8
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[d][i] += dpp<kDppRowRor8>(o[d][i]);
+  float sc = 1.0f;
+  if (nph > 1) {
+    if (g == 0) {
+      wave_m[wv][j] = m;
+      wave_l[wv][j] = lsum;
+    }
+    __syncthreads();
+    float mm = m;
+    for (int p = 0; p < nph; ++p) mm = fmaxf(mm, wave_m[hsub + hw * p][j]);
+    lsum = 0.0f;
+    for (int p = 0; p < nph; ++p)
+      lsum += wave_l[hsub + hw * p][j] * fast_exp2(wave_m[hsub + hw * p][j] - mm);
+    sc = fast_exp2(m - mm);
+    m = mm;
+  }
+  constexpr int kSt = D + 4;                          // floats per staged row
+  if (single) sc *= lsum > 0.0f ? 1.0f / lsum : 0.0f;
+  float* st = reinterpret_cast<float*>(&lds[wv]);
+#pragma unroll
+  for (int d = 0; d < D / 16; ++d)
+    *reinterpret_cast<float4*>(&st[j * kSt + 16 * d + 4 * g]) =
+        make_float4(o[d][0] * sc, o[d][1] * sc, o[d][2] * sc, o[d][3] * sc);
+  if (!single && ph == 0 && g == 0 && j < gc)
+    *reinterpret_cast<float2*>(ml + 2 * j) = make_float2(m, lsum);
+  if (nph > 1) __syncthreads();
+  else wave_lds_fence();
+  constexpr int kLr = D / 4;                          // lanes per head row
+  constexpr int kHp = 64 / kLr;                       // head rows per wave and pass
+  const int c4 = lane % kLr;
+  float* dst = (single ? out_rows : acc_rows) + 4 * c4;
+  for (int hb = ph * kHp; hb < gc; hb += nph * kHp) {   // wave-uniform
+    const int hh = hb + lane / kLr;
+    if (hh < gc) {
+      float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      for (int p = 0; p < nph; ++p) {
+        const float4 y = *reinterpret_cast<const float4*>(
+            &reinterpret_cast<const float*>(&lds[hsub + hw * p])[hh * kSt + 4 * c4]);
+        x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
+      }
+      *reinterpret_cast<float4*>(dst + (int64_t)hh * D) = x;
+    }
+  }
+  if (nph > 1) __syncthreads();   // staging read by every wave before the buffers are reused
+  else wave_lds_fence();
+}
+
+// A workgroup's kW waves are hw neighbouring KV heads times nph page phases, so
+// the waves in flight together read hw * D * 2 adjacent bytes of every token
+// row of a page.  Reads alone gain from that (C2-gqa's pages, nothing
+// computed: 105.8 us with one head a workgroup, 101.6 with 2, 4 or 8), but
+// more heads and fewer phases also mean more ranges and states to merge:
+// whole calls, us, for 1 x 4 / 2 x 4 / 8 x 1 / 8 x 2 heads x phases:
+//   C2-gqa                                         124.0 122.2 127.3 122.2
+//   the same at head dim 64, fp16                   75.2  69.1  67.8  67.7
+//   the same with 16 KV heads                      232.4 228.3 229.8 224.9
+//   64 x 4096 tokens                               178.6 176.4 182.5 174.9
+//   300 rows of 16..3000 tokens                    330.0 323.1 325.4 317.0
+//   4 rows of 8k..32k tokens, fp16                  65.9  65.1  79.6  69.9
+template <typename Ops, int D, int kW>
 __global__ __launch_bounds__(64 * kW) void splitmm_even_kernel(RowAttnArgs a) {
   __shared__ PageLds<D> lds[kW];
   __shared__ float wave_m[kW][kSlots], wave_l[kW][kSlots];
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int G = a.H / a.Hkv;
-  const int n_hc = (G + kSlots - 1) / kSlots;
-  const int n_units = a.Hkv * n_hc;
-  const int kg = min(G, kSlots);                        // state rows per slot
-  const int unit = (int)(blockIdx.x % n_units);         // unit-fastest: units spread over XCDs
-  const int wr = (int)(blockIdx.x / n_units);           // this workgroup's range, < M
-  const int kvh = unit / n_hc;
-  const int hc = unit - kvh * n_hc;
-  const int h0 = kvh * G + hc * kSlots;
-  const int gc = min(kSlots, G - hc * kSlots);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = a.H / a.Hkv;                            // <= 8: hi and lo terms as columns
+  const int hw = a.even_hw;
+  const int nph = kW / hw;
+  const int n_groups = a.Hkv / hw;
+  const int hsub = wv % hw;
+  const int ph = wv / hw;
+  const int kvh = (int)(blockIdx.x % n_groups) * hw + hsub;
+  const int wr = (int)(blockIdx.x / n_groups);          // this workgroup's range, < M
+  const int h0 = kvh * G;
 
   int64_t s, e, Rr;
   int r;
@@ -656,12 +758,11 @@ __global__ __launch_bounds__(64 * kW) void splitmm_even_kernel(RowAttnArgs a) {
       const int lo = (int)(pa - Rr) * kPage;
       const int hi = (int)min((pb - Rr) * kPage, (int64_t)end);
       const int64_t orow0 = ((int64_t)r * a.H + h0) * D;
-      page_walk<Ops, D, kCols>(a, lds[wv], kvh, gc, a.bt + (int64_t)r * a.MB, lo, hi, wv, kW,
-                               orow0, o, m, l);
-      const int64_t slot = ((int64_t)unit * a.even_slots + wr + r) * kg;   // head h0's state
-      write_unit_state<D, kCols, kW>(o, m, l, gc, pa == Rr && pb == Rn, a.out + orow0,
-                                     a.part_acc + slot * D, D, a.part_ml + 2 * slot, 1, lds,
-                                     wave_m, wave_l);
+      page_walk<Ops, D, true>(a, lds[wv], kvh, G, a.bt + (int64_t)r * a.MB, lo, hi, ph, nph,
+                              orow0, o, m, l);
+      const int64_t slot = ((int64_t)kvh * a.even_slots + wr + r) * G;   // head h0's state
+      write_head_state<D, kW>(o, m, l, G, hsub, ph, hw, nph, pa == Rr && pb == Rn, a.out + orow0,
+                              a.part_acc + slot * D, a.part_ml + 2 * slot, lds, wave_m, wave_l);
     }
     Rr = Rn;
   }
@@ -726,16 +827,16 @@ __global__ __launch_bounds__(256) void even_merge_kernel(RowAttnArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t wg = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (wg >= (int64_t)a.B * a.H) return;
-  const int r = (int)(wg / a.H);
+  const int r = __builtin_amdgcn_readfirstlane((int)(wg / a.H));
   const int h = (int)(wg - (int64_t)r * a.H);
   float* dst = a.out + wg * D;
   constexpr int kPer = (D + 63) / 64;
   int64_t tp = 0, Rr = 0;                               // all pages; pages of rows before r
   for (int c = 0; c < a.B; c += 64) {
-    const int b = c + lane;
-    const int64_t v = b < a.B ? row_pages(a, b) : 0;
-    tp += wave_sum64(v);
-    Rr += wave_sum64(b < r ? v : 0);
+    int64_t v;
+    const int64_t inc = scan_rows(a, c, v);
+    if (r >= c && r < c + 64) Rr = tp + lane_value64(inc - v, r - c);
+    tp += lane_value64(inc, 63);
   }
   const int pr = row_pages(a, r);
   if (pr == 0) {
@@ -745,7 +846,7 @@ __global__ __launch_bounds__(256) void even_merge_kernel(RowAttnArgs a) {
     return;
   }
   const int64_t Q = range_pages(a, tp);
-  const int64_t w_first = Rr / Q, w_last = (Rr + pr - 1) / Q;
+  const int64_t w_first = div_pages(Rr, Q), w_last = div_pages(Rr + pr - 1, Q);
   if (w_first == w_last) return;
   const int G = a.H / a.Hkv;
   const int n_hc = (G + kSlots - 1) / kSlots;
@@ -875,8 +976,8 @@ void launch_splitmm_part(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t 
 // even split: host side
 // ---------------------------------------------------------------------------
 
-// The even split serves groups of at most 4 query heads per KV head (one
-// 4-wave workgroup per unit, hi and lo terms as MFMA columns) on grids whose
+// The even split serves groups of at most 4 query heads per KV head (hi and lo
+// terms as MFMA columns) on grids whose
 // fixed partitions would take more than one round of the device.  Measured
 // on MI355X against fixed partitions (whole call, us): C2-gqa 109 / 113, 300
 // sequences of 16..3000 tokens 328 / 378, 64 x 4096 tokens 177 / 189, C2
@@ -886,7 +987,8 @@ void launch_splitmm_part(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t 
 // 768-token partition each: 31.8 / 24.0; 8 rows of 1-4k tokens: 25.5 /
 // 24.8): there the merge launch costs more than the last round's idle slots.
 constexpr int kEvenMaxGroup = 4;
-constexpr int kEvenWaves = 4;
+constexpr int kEvenWaves = 8;
+constexpr int kEvenHeads = 2;
 // Workgroups of the device's occupancy per CU taken by the grid: filled once
 // (C2-gqa: 109 us; twice 114, three times 116), and the least pages of a
 // range (16: 4 a wave; 32 measured the same on C2-gqa).
@@ -895,9 +997,9 @@ constexpr int kEvenMinPages = 16;
 
 template <typename Ops>
 static const void* even_kernel_t(int D) {
-  if (D == 32) return (const void*)splitmm_even_kernel<Ops, 32, true, kEvenWaves>;
-  if (D == 64) return (const void*)splitmm_even_kernel<Ops, 64, true, kEvenWaves>;
-  return (const void*)splitmm_even_kernel<Ops, 128, true, kEvenWaves>;
+  if (D == 32) return (const void*)splitmm_even_kernel<Ops, 32, kEvenWaves>;
+  if (D == 64) return (const void*)splitmm_even_kernel<Ops, 64, kEvenWaves>;
+  return (const void*)splitmm_even_kernel<Ops, 128, kEvenWaves>;
 }
 
 static const void* even_kernel(int kv_dtype, int D) {
@@ -905,6 +1007,9 @@ static const void* even_kernel(int kv_dtype, int D) {
 }
 
 int splitmm_even_min_pages() { return kEvenMinPages; }
+
+// KV heads side by side in a workgroup of the even split.
+int splitmm_even_heads(int H, int Hkv) { return H != Hkv && Hkv % kEvenHeads == 0 ? kEvenHeads : 1; }
 
 // Plain multi-head attention (H == Hkv) on 16-bit caches with 16-token
 // pages: the VALU even split, against the VALU kernel's fixed 512-token
@@ -964,7 +1069,7 @@ int splitmm_even_groups(int kv_dtype, int D, int H, int Hkv, int B, int MB) {
     part = kValuFixedPartition;
   } else if (splitmm_serves(kv_dtype, kPage, D, H, Hkv) && G <= kEvenMaxGroup) {
     even_occupancy(even_kernel(kv_dtype, D), 64 * kEvenWaves, &occ, &cus);
-    groups = Hkv;
+    groups = Hkv / splitmm_even_heads(H, Hkv);
     part = splitmm_default_partition(G, D);
   } else {
     return 0;
@@ -972,7 +1077,8 @@ int splitmm_even_groups(int kv_dtype, int D, int H, int Hkv, int B, int MB) {
   if (occ <= 0 || cus <= 0) return 0;
   const int64_t fill = ceil_div((int64_t)cus * occ * kEvenRounds, groups);
   const int64_t parts = sat_mul(B, ceil_div((int64_t)MB * kPage, part));
-  if (parts <= fill) return 0;
+  const int64_t one = H == Hkv ? fill : ceil_div((int64_t)cus * occ * (kEvenWaves / 4), Hkv);
+  if (parts <= one) return 0;
   return (int)std::min<int64_t>(fill, 1 << 20);
 }
 
@@ -990,13 +1096,13 @@ EvenLayout splitmm_even_layout(int B, int H, int Hkv, int D, int M) {
 
 template <typename Ops>
 static void launch_even_for(const RowAttnArgs& a, int D, hipStream_t stream) {
-  const dim3 grid((unsigned)((int64_t)a.Hkv * a.even_m)), block(64 * kEvenWaves);
+  const dim3 grid((unsigned)((int64_t)(a.Hkv / a.even_hw) * a.even_m)), block(64 * kEvenWaves);
   if (D == 32)
-    hipLaunchKernelGGL((splitmm_even_kernel<Ops, 32, true, kEvenWaves>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((splitmm_even_kernel<Ops, 32, kEvenWaves>), grid, block, 0, stream, a);
   else if (D == 64)
-    hipLaunchKernelGGL((splitmm_even_kernel<Ops, 64, true, kEvenWaves>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((splitmm_even_kernel<Ops, 64, kEvenWaves>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((splitmm_even_kernel<Ops, 128, true, kEvenWaves>), grid, block, 0, stream,
+    hipLaunchKernelGGL((splitmm_even_kernel<Ops, 128, kEvenWaves>), grid, block, 0, stream,
                        a);
 }
 

@@ -37,6 +37,7 @@ struct RowAttnArgs {
   int even_m;
   int even_slots;
   int even_min_pages;
+  int even_hw;            // grouped heads: KV heads side by side in a workgroup
 };
 
 // Sequence of a row and the end of its key range (exclusive).  Returns false
@@ -125,6 +126,7 @@ void launch_splitmm_part(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t 
 // geometry on the current device), and the workspace its states take.
 int splitmm_even_groups(int kv_dtype, int D, int H, int Hkv, int B, int MB);   // 0: not served
 int splitmm_even_min_pages();
+int splitmm_even_heads(int H, int Hkv);   // KV heads side by side in a workgroup
 struct EvenLayout {
   int64_t acc, ml, end;   // byte offsets; end == INT64_MAX when too large
 };
