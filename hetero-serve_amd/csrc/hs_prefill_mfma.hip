@@ -75,7 +75,8 @@ template <int D>
 constexpr int v_pad() { return D == 32 ? 0 : 32; }
 constexpr float kRescaleSlack = 8.0f;        // log2 units
 constexpr int kMaxRanked = 256;              // sequences a workgroup ranks itself
-constexpr int kMaxSplit = 4;                 // key-range parts of one query tile
+constexpr int kMaxSplit = 16;                // key-range parts of one query tile
+constexpr int kPartTiles = 4;                // key tiles of the table a part gets beyond 4 parts
 
 // Workgroup shape: W waves of 32 query rows.  D 128 and 64 run 8 waves (256
 // rows, one workgroup per CU; each K/V tile then serves twice the rows of a
@@ -1994,38 +1995,41 @@ void prefill_stream_kernel(PrefillArgs a) {
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   constexpr int kC = D / 4;
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int g = (int)(blockIdx.x * 256 + threadIdx.x);
+  const int h = g / kC, c = g % kC;
+  const int i = (int)blockIdx.y, b = (int)blockIdx.z;
+  if (h >= a.H || i >= seq_rows(a, b)) return;
   const int64_t n_pairs = (int64_t)a.B * a.rows_cap * a.H;   // pairs per part
-  const int64_t pair = g / kC;
-  if (pair >= n_pairs) return;
-  const int c = (int)(g - pair * kC);
-  const int h = (int)(pair % a.H);
-  const int64_t bi = pair / a.H;
-  const int i = (int)(bi % a.rows_cap);
-  const int b = (int)(bi / a.rows_cap);
-  if (i >= seq_rows(a, b)) return;
+  const int64_t pair = ((int64_t)b * a.rows_cap + i) * a.H + h;
   const int64_t row0 = a.cu_q ? a.cu_q[b] : (int64_t)b * a.S;
-  float2 ml[kMaxSplit];
   float mx = kNegBig;
+  for (int p0 = 0; p0 < a.n_split; p0 += 4) {
+    float m[4];
 #pragma unroll
-  for (int p = 0; p < kMaxSplit; ++p) {
-    if (p < a.n_split) {
-      ml[p] = a.part_ml[p * n_pairs + pair];
-      mx = fmaxf(mx, ml[p].x);
-    }
+    for (int u = 0; u < 4; ++u)
+      m[u] = a.part_ml[min(p0 + u, a.n_split - 1) * n_pairs + pair].x;
+    mx = fmaxf(mx, fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
   }
   float lsum = 0.0f;
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int p0 = 0; p0 < a.n_split; p0 += 4) {
+    float2 ml[4];
+    float4 o[4];
 #pragma unroll
-  for (int p = 0; p < kMaxSplit; ++p) {
-    if (p < a.n_split) {
-      const float w = fast_exp2(ml[p].x - mx);
-      const float4 o = reinterpret_cast<const float4*>(a.part_o)[(p * n_pairs + pair) * kC + c];
-      lsum += w * ml[p].y;
-      acc.x += w * o.x;
-      acc.y += w * o.y;
-      acc.z += w * o.z;
-      acc.w += w * o.w;
+    for (int u = 0; u < 4; ++u) {   // past the last part: its loads again, not used
+      const int64_t pi = min(p0 + u, a.n_split - 1) * n_pairs + pair;
+      ml[u] = a.part_ml[pi];
+      o[u] = reinterpret_cast<const float4*>(a.part_o)[pi * kC + c];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (p0 + u >= a.n_split) break;
+      const float w = fast_exp2(ml[u].x - mx);
+      lsum += w * ml[u].y;
+      acc.x += w * o[u].x;
+      acc.y += w * o[u].y;
+      acc.z += w * o[u].z;
+      acc.w += w * o[u].w;
     }
   }
   const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
@@ -2061,11 +2065,13 @@ int launch_typed(PrefillArgs a, int max_rows_per_seq, int stream_ns, hipStream_t
     hipLaunchKernelGGL((prefill_mfma_kernel<T, D, W>), grid, block, 0, stream, a);
   }
   if (a.n_split > 1) {
-    // the workspace of B * rows_cap * H * (D + 2) floats per part exists, so
-    // this product fits; the grid must still fit one launch
-    const int64_t groups = ceil_div(sat_mul(a.B, a.rows_cap, a.H, D / 4), 256);
-    if (groups > 0x7fffffffLL) return fail(HS_EUNSUPPORTED, "prefill merge grid too large");
-    hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned)groups), dim3(256), 0, stream, a);
+    // a split has at most cus / 2 query tiles (plan_prefill_mfma), which bounds
+    // the rows and the sequences far below a grid's limits
+    const int64_t groups = ceil_div((int64_t)a.H * (D / 4), 256);
+    if (a.rows_cap > 0xffff || a.B > 0xffff)
+      return fail(HS_EUNSUPPORTED, "prefill merge grid too large");
+    hipLaunchKernelGGL((prefill_merge_kernel<D>), dim3((unsigned)groups, a.rows_cap, a.B), dim3(256),
+                       0, stream, a);
   }
   return HS_OK;
 }
@@ -2091,8 +2097,12 @@ int launch_dim(const PrefillArgs& a, int D, bool wide, int max_rows_per_seq, int
 // Launch shape of the MFMA prefill for B sequences of up to max_rows query
 // rows on a device with `cus` CUs.  Full-width workgroups (256 rows; 128 at
 // head dim 32) when their query tiles cover every CU.  Otherwise, with a
-// workspace, each tile's key range is split over floor(cus / tiles) <= 4
-// workgroups (a 1024-row chunk of 32 heads: 128 tiles, 2 parts); without one,
+// workspace, each tile's key range is split over floor(cus / tiles) <= 16
+// workgroups (a 1024-row chunk of 32 heads: 128 tiles, 2 parts); at up to 4
+// parts a short chunk on a long prefix still walked 17 tiles a workgroup beside
+// idle CUs.  One sequence, prefix 4096, us a call at up to 4 / 16 parts: 16 rows
+// 32 / 8 heads 27.4 / 22.8, 12 heads D 64 21.2 / 17.6, 8 heads D 32 22.2 / 16.4;
+// 128 rows 33.2 / 28.5, 24.3 / 21.6, 24.0 / 17.8.  Without one,
 // 128-row workgroups, which run one wave per SIMD but reach twice as many CUs.
 //
 // With a workspace, full-width grids of at least two query tiles per CU run
@@ -2113,7 +2123,11 @@ PrefillPlan plan_prefill_mfma(int B, int max_rows, int H, int D, int cus, bool c
       p.stream_ns = cus / kXcds;
     return p;
   }
-  const int64_t splits = std::min<int64_t>(kMaxSplit, tiles > 0 ? cus / tiles : 1);
+  // head h's workgroups run on XCD h % 8: beyond 4 parts, no more workgroups
+  // than CUs on the XCD with the most heads
+  const int64_t on_xcd = sat_mul(B, ceil_div(max_rows, bm), ceil_div(H, kXcds));
+  const int64_t splits = std::max(std::min<int64_t>(4, tiles > 0 ? cus / tiles : 1),
+                                  std::min<int64_t>(kMaxSplit, on_xcd > 0 ? cus / kXcds / on_xcd : 1));
   if (can_split && splits >= 2 && B <= kMaxRanked) p.n_split = (int)splits;
   else p.wide = false;
   return p;
@@ -2164,6 +2178,15 @@ int launch_prefill_mfma(const float* q, const int32_t* cu_q, int S, int max_rows
     a.counters = static_cast<int*>(workspace);
   }
   if (plan.n_split > 1) {
+    // more than 4 parts only for what the table can hold, and in the
+    // workspace that is there
+    const int64_t key_tiles = ceil_div(sat_mul(MB, 16), kBN);
+    plan.n_split = (int)std::min<int64_t>(plan.n_split,
+                                          std::max<int64_t>(4, ceil_div(key_tiles, kPartTiles)));
+    while (plan.n_split > 4 &&
+           prefill_workspace_bytes(plan, B, max_rows_per_seq, H, D) > (int64_t)workspace_bytes)
+      --plan.n_split;
+    a.n_split = plan.n_split;
     const int64_t need_i = prefill_workspace_bytes(plan, B, max_rows_per_seq, H, D);
     if (need_i == INT64_MAX) return fail(HS_EUNSUPPORTED, "prefill split too large");
     const size_t need = (size_t)need_i;

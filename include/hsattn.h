@@ -211,7 +211,7 @@ int hs_decode_shared(const float* q, const void* k_cache, const void* v_cache, i
  * up to max_seqlen_q query rows (S for hs_prefill), for the current HIP
  * device; 0 when they need none.  Only the matrix-core path (use_mfma = 1)
  * uses one: when its query tiles cannot cover every CU, each tile's key range
- * is split over up to 4 workgroups, whose partial results (fp32, (D + 2) * 4
+ * is split over up to 16 workgroups, whose partial results (fp32, (D + 2) * 4
  * bytes per part, row and head) are merged by a second kernel; when they give
  * every CU at least two (head dim 64 or 128, H a multiple of 8, at most 256
  * sequences), a persistent kernel of one workgroup per CU takes them from
