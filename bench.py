@@ -1183,7 +1183,7 @@ def main() -> int:
                 "us_per_call": round(host_us, 2), "device_us_per_call": round(dev_us, 2),
                 "tflops": round(pre["flops"] / (dev_us * 1e-6) / 1e12, 3),
                 "max_abs_err": float(f"{serr:.3e}"),
-                "path": "hs_prefill_varlen(use_mfma=0): the fp32 row kernel of "
+                "path": "hs_prefill_varlen(use_mfma=0): the fp32 kernel of "
                         "paged_attention_prefill"}
             errors["C4_scalar"] = serr
             log(f"C4 scalar prefill: {dev_us:.1f} us, err {serr:.2e}")
