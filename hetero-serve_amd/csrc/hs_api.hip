@@ -155,8 +155,13 @@ static int default_partition(int B, int H, int Hkv, int BS, int MB, int kv_dtype
 // partition that the workspace was sized for.  16 sequences of 256..4096
 // tokens, us from 1024 keys and two workgroups a CU / from 2048 and one: 32 / 8
 // heads, D 128, fp32 72 / 60; 16 / 1, fp32 24 / 18; 32 / 4, bf16, 32-token
-// blocks 37 / 33.
-static int rows_partition(int B, int H, int Hkv, int BS, int MB, int default_pt) {
+// blocks 37 / 33.  A row that the waves finish in a few tiles each is one partition,
+// without a merge: 256 keys at head dim 128 (8 to 32 sequences of 64..256 tokens,
+// 32 / 8 heads, fp32: 14.3 / 12.4; at 512 keys 17 against 15).
+constexpr int kOnePassElems = 256 * 128;
+static int rows_partition(int B, int H, int Hkv, int D, int BS, int MB, int default_pt) {
+  const int one_pass = kOnePassElems / D;
+  if ((int64_t)MB * BS <= one_pass) return std::max(default_pt, one_pass);
   const int pt = shrink_for_small_grid(2048, 128, sat_mul(B, Hkv, ceil_div(H / Hkv, 16)), BS, MB, 1);
   return std::max(pt, default_pt);
 }
@@ -175,6 +180,16 @@ constexpr int64_t kWgSplitMaxTokens = 1024;
 static bool wg_split_applies(int B, int H, int Hkv, int BS, int MB, int kv_dtype, int D) {
   if (H != Hkv || (int64_t)MB * BS > kWgSplitMaxTokens) return false;
   return default_partition(B, H, Hkv, BS, MB, kv_dtype, D) < kDefaultPartition;
+}
+
+// Short rows of groups of 2 and 4 at head dim 256 go the same way, each query
+// head a workgroup of its own: the group's pages come from the caches again,
+// which up to 512 tokens (fp32: 256) costs less than the states and the merge.
+// 8 / 4 heads, fp16, 32 sequences of 128..512 tokens, VALU partitions / so: 21.5 /
+// 16.1 us; fp32, of 64..256 tokens, fp32 matrix cores / so: 19.4 / 16.6.
+static bool short_rows_in_wg(int H, int Hkv, int D, int kv_dtype, int64_t width) {
+  return D > 128 && H != Hkv && H / Hkv <= 4 && row_attn_heads_per_wave(H, Hkv) == H / Hkv &&
+         width <= (kv_dtype == HS_DTYPE_F32 ? 256 : 512);
 }
 
 // Decode by explicit splits: the slices that are taken together.  Neighbouring
@@ -212,11 +227,15 @@ static bool wg_per_row(int64_t rows_heads, int64_t width, int cus) {
 // 122 / 100, 124 / 129, 250 / 286; 16 of them in bf16 with 8-token blocks 56 /
 // 59, in one pass 613 / 95; 32 / 4 heads fp32, 16 / 64 sequences 103 / 35, 223 /
 // 140; 16 / 1 heads 94 / 18; 8 / 4 heads, D 256, fp32, 32 / 64 sequences 225 /
-// 144, 268 / 280.
-static bool grouped_on_matrix_cores(int B, int H, int Hkv, int kv_dtype, int num_splits, int cus) {
+// 144, 268 / 280.  Short rows, whose default partitions the VALU kernel has cut
+// for a small grid, come here up to head dim 128: 32 / 8 heads, 8-token blocks,
+// fp16, 16 sequences of 256..1024 tokens 31.7 / 21.3, 32 of 64..256 19.9 / 12.2,
+// 32 of them in fp32 29.2 / 13.7.
+static bool grouped_on_matrix_cores(int B, int H, int Hkv, int kv_dtype, int num_splits,
+                                    bool short_rows, int cus) {
   const int G = H / Hkv;
   if (G == 1) return false;
-  if (G > 4 || row_attn_heads_per_wave(H, Hkv) < G || num_splits == 1) return true;
+  if (G > 4 || row_attn_heads_per_wave(H, Hkv) < G || num_splits == 1 || short_rows) return true;
   return kv_dtype == HS_DTYPE_F32 && sat_mul(B, Hkv) < cus;
 }
 
@@ -466,17 +485,21 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
   a.qscale = scale * kLog2e;
   if (!shared_pages || !shared_pages_apply(a, kv_dtype, D)) {
     const bool mha = H == Hkv;
-    a.mma = grouped_on_matrix_cores(B, H, Hkv, kv_dtype, num_splits, cus) &&
-            !splitmm_applies(a, kv_dtype, D) && rows_serves(a, kv_dtype, D);
     const int64_t width = (int64_t)MB * BS;
-    if (num_splits == 0 && partition_tokens == 0 &&
-        wg_split_applies(B, H, Hkv, BS, MB, kv_dtype, D)) {
+    const bool short_rows = num_splits == 0 && partition_tokens == 0 && width <= kWgSplitMaxTokens &&
+                            plan.part_tokens < valu_partition(H, Hkv);
+    const bool wg_rows = short_rows && short_rows_in_wg(H, Hkv, D, kv_dtype, width);
+    a.mma = !wg_rows &&
+            grouped_on_matrix_cores(B, H, Hkv, kv_dtype, num_splits, short_rows && D <= 128, cus) &&
+            !splitmm_applies(a, kv_dtype, D) && rows_serves(a, kv_dtype, D);
+    if (wg_rows || (num_splits == 0 && partition_tokens == 0 &&
+                    wg_split_applies(B, H, Hkv, BS, MB, kv_dtype, D))) {
       // the workspace, sized for the partitions above, goes unused
       a.mode = 0;
       a.P = 1;
       a.wg = 1;
     } else if (num_splits == 0 && partition_tokens == 0 && a.mma) {
-      a.part_tokens = rows_partition(B, H, Hkv, BS, MB, plan.part_tokens);
+      a.part_tokens = rows_partition(B, H, Hkv, D, BS, MB, plan.part_tokens);
       a.P = (int)ceil_div(width, a.part_tokens);
     } else if (num_splits == 1) {
       a.wg = mha && wg_per_row((int64_t)B * H, width, cus);

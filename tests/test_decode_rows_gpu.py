@@ -78,6 +78,18 @@ def test_grouped_heads(dtype, H, Hkv, D, BS):
     _runs(_case(EDGES, H, Hkv, D, BS, dtype))
 
 
+@pytest.mark.parametrize("dtype,H,Hkv,D,BS", [
+    (torch.float16, 8, 2, 128, 8), (torch.bfloat16, 4, 2, 64, 32), (torch.float16, 8, 4, 256, 16),
+    (torch.float32, 32, 8, 128, 16), (torch.float32, 8, 4, 256, 16)])
+@pytest.mark.parametrize("ctxs", [[0, 1, 15, 16, 17, 127, 128, 129, -3, 200],
+                                  [0, 1, 15, 16, 17, 127, 128, 129, -3, 300, 975],
+                                  [(29 * i) % 250 for i in range(32)]])
+def test_grouped_short_rows(dtype, H, Hkv, D, BS, ctxs):
+    """Groups of 2 and 4 whose tables hold at most 1024 tokens, in the default
+    partitions: one or several, with and without a workgroup for every CU."""
+    _runs(_case(ctxs, H, Hkv, D, BS, dtype, seed=4), splits=(0,))
+
+
 @pytest.mark.parametrize("dtype,D,BS", [(torch.float16, 64, 16), (torch.float32, 128, 16),
                                         (torch.bfloat16, 256, 5), (torch.float32, 32, 3)])
 def test_multi_head_rows(dtype, D, BS):
