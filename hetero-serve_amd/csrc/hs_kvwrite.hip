@@ -224,7 +224,12 @@ __global__ __launch_bounds__(kWriteThreads) void kv_write_scalar_kernel(WriteArg
                        i * a.src_row + src_offset(a, e, Codec<S>::kBytes);
   uint8_t* dst = ((blockIdx.y & 1) ? a.v_cache : a.k_cache) + layer * a.cache_layer +
                  (slot * (int64_t)row + e) * Codec<C>::kBytes;
-  Codec<C>::store1(dst, Codec<S>::load1(src));
+  if constexpr (std::is_same<S, C>::value) {   // a bit copy here too
+    using Word = std::conditional_t<Codec<C>::kBytes == 4, uint32_t, uint16_t>;
+    *reinterpret_cast<Word*>(dst) = *reinterpret_cast<const Word*>(src);
+  } else {
+    Codec<C>::store1(dst, Codec<S>::load1(src));
+  }
 }
 
 template <typename S, typename C>

@@ -48,6 +48,50 @@ def test_write_kv_layers(src, cache, L, H, T, D, BS, start):
         assert torch.equal(_bits(pool), _bits(want)), name
 
 
+def _random_bits(shape, dtype, gen):
+    """Every bit pattern, NaN payloads and signs of NaN among them; at least one
+    element in sixteen is a NaN."""
+    size = torch.empty(0, dtype=dtype).element_size()
+    word = torch.int32 if size == 4 else torch.int16
+    low, high = torch.iinfo(word).min, torch.iinfo(word).max
+    bits = torch.randint(low, high + 1, shape, generator=gen, dtype=torch.int64)
+    nan = {torch.float32: 0x7F800001, torch.float16: 0x7C01, torch.bfloat16: 0x7F81}[dtype]
+    bits = torch.where(torch.randint(0, 16, shape, generator=gen) == 0, bits | nan, bits)
+    return bits.to(word).view(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L,H,T,D", [(2, 2, 9, 36), (2, 2, 9, 64), (1, 3, 5, 32), (1, 1, 4, 7)])
+def test_equal_types_keep_every_bit(dtype, L, H, T, D):
+    """Sources of the cache's type are copied word for word in every layout,
+    also where a head's rows are no 16-byte groups: write_kv, scatter_kv and
+    append_kv."""
+    from heteroserve.kv import pack
+
+    gen = torch.Generator().manual_seed(D)
+    wide = _random_bits((L, H, T, D + 1), dtype, gen)
+    nb, table = 4, [2, 0]
+    for x in (wide[..., :D], wide[..., 1:], wide[..., :D].contiguous()):
+        xd = wide.to(DEV)[..., 1:] if x.storage_offset() else x.to(DEV)
+        want = torch.zeros(L, 2, nb, 8, H, D, dtype=dtype)
+        kvp.write_kv(want, table, 3, x, x)
+        pool = torch.zeros_like(want, device=DEV)
+        pack.write_kv(pool, table, 3, xd, xd)
+        assert torch.equal(_bits(pool), _bits(want))
+        if L > 1:
+            continue
+        rows = xd[0].transpose(0, 1).contiguous()
+        slots = pack.slots_for(table, range(3, 3 + T), 8)
+        pool.zero_()
+        pack.scatter_kv(pool[0, 0], pool[0, 1], slots, rows, rows)
+        assert torch.equal(_bits(pool), _bits(want))
+        pool.zero_()
+        pack.append_kv(pool[0, 0], pool[0, 1], torch.tensor([table], dtype=torch.int32),
+                       torch.arange(3, 3 + T, dtype=torch.int32), rows, rows,
+                       torch.zeros(T, dtype=torch.int32))
+        assert torch.equal(_bits(pool), _bits(want))
+
+
 def test_write_kv_refuses_what_does_not_fit():
     from heteroserve.kv import pack
 
