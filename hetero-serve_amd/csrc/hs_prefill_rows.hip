@@ -112,6 +112,42 @@ __device__ inline void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Scheduling barrier mask: everything but matrix instructions may cross it.
+// Without it the compiler holds the results of many products at once.
+constexpr int kAllButProducts = 0x3F6;
+
+// The products of 4 dims or keys, summed.
+__device__ inline float4x product4(float a, float b) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, float4x{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+}
+
+// Dot products over the lane's 4 N dims (16 N in all) of NT row tiles, row
+// tiles `step` floats apart.  Each matrix instruction starts from zero and
+// the results are added as a tree: a row with few keys has the error of its
+// scores, and accumulating in the instructions, in chains of 16 to 64
+// products, it was up to 1.6 times that of the VALU kernel's chains of 4 or 8
+// and trees over the lanes (2-norm against fp64, head dim 128, 17 keys, bf16:
+// 1.79e-7, 1.12e-7 there, 1.12e-7 so).
+template <int N, int NT>
+__device__ inline void dot_tree(const float* k, const float* q, int step, float4x (&s)[NT]) {
+  if constexpr (N == 1) {
+    const float4 kf = *reinterpret_cast<const float4*>(k);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float4 qf = *reinterpret_cast<const float4*>(q + t * step);
+      s[t] = (product4(kf.x, qf.x) + product4(kf.y, qf.y)) +
+             (product4(kf.z, qf.z) + product4(kf.w, qf.w));
+      __builtin_amdgcn_sched_barrier(kAllButProducts);
+    }
+  } else {
+    float4x r[NT];
+    dot_tree<N / 2, NT>(k, q, step, s);
+    dot_tree<N / 2, NT>(k + 2 * N, q + 2 * N, step, r);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) s[t] += r[t];
+  }
+}
+
 // The rows of row tile `tile` of (sequence b, KV head kvh) against the keys of
 // partition p (decode; prefill has one partition, all keys); every thread of
 // the workgroup calls it (it holds barriers).
@@ -133,7 +169,7 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
 
   __shared__ __align__(16) float ks[W][kKeys][kRow];
   __shared__ __align__(16) float qs[kRows][kRow];
-  __shared__ float wave_m[W][kRows], wave_l[W][kRows], inv_l[kKeys];
+  __shared__ float wave_m[W][kRows], wave_l[W][kRows], row_l[kKeys];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -264,38 +300,9 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
     next_slots = slot_of(n + 2 * W);
     load_k(slots);
 
-    // S^T: lane (j, g) gets keys 4 g + i of row j of each row tile.  kAcc
-    // accumulators per row tile, summed at the end: short chains of dependent
-    // products, and of roundings.
-    constexpr int kAcc = NT > 1 ? 2 : D >= 128 ? 8 : 4;
-    float4x sa[NT][kAcc];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int c = 0; c < kAcc; ++c) sa[t][c] = float4x{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int c = 0; c < D / 16; ++c) {
-      const float4 kf = *reinterpret_cast<const float4*>(&ks[wv][j][g * (D / 4) + 4 * c]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const float4 qf =
-            *reinterpret_cast<const float4*>(&qs[t * kKeys + j][g * (D / 4) + 4 * c]);
-        float4x* acc = &sa[t][4 * c % kAcc];
-        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qf.x, acc[0], 0, 0, 0);
-        acc[1 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qf.y, acc[1 % kAcc], 0, 0, 0);
-        acc[2 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qf.z, acc[2 % kAcc], 0, 0, 0);
-        acc[3 % kAcc] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qf.w, acc[3 % kAcc], 0, 0, 0);
-      }
-    }
+    // S^T: lane (j, g) gets keys 4 g + i of row j of each row tile.
     float4x s[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-#pragma unroll
-      for (int n2 = kAcc / 2; n2 > 0; n2 /= 2)
-#pragma unroll
-        for (int c = 0; c < n2; ++c) sa[t][c] += sa[t][c + n2];
-      s[t] = sa[t][0];
-    }
+    dot_tree<D / 16, NT>(&ks[wv][j][g * (D / 4)], &qs[j][g * (D / 4)], kKeys * kRow, s);
     wave_lds_fence();
 
     const int t0 = lo + n * kKeys;
@@ -338,20 +345,21 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
     }
     if (!one_by_one) {
       // O^T += V^T . P^T: output tile (u, e) holds dims 16 kVE u + kVE row + e.
-      // The 16 keys are summed by themselves first: a wave's sum over its keys
-      // then has one rounding per tile and not one per key.
+      // The 16 keys are summed by themselves first, as a tree over their
+      // products of 4: a wave's sum over its keys then has one rounding per
+      // tile and not one per key.
 #pragma unroll
       for (int u = 0; u < kNV; ++u)
 #pragma unroll
         for (int e = 0; e < kVE; ++e)
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
-            float4x sum = float4x{0.0f, 0.0f, 0.0f, 0.0f};
+            float4x x[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              sum = __builtin_amdgcn_mfma_f32_16x16x4f32(word_elem<T>(vr[i][u], e), p[t][i], sum,
-                                                         0, 0, 0);
-            o[t][u * kVE + e] += sum;
+              x[i] = product4(word_elem<T>(vr[i][u], e), p[t][i]);
+            o[t][u * kVE + e] += (x[0] + x[1]) + (x[2] + x[3]);
+            __builtin_amdgcn_sched_barrier(kAllButProducts);
           }
     } else {
 #pragma unroll 1
@@ -398,7 +406,6 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
     for (int w = 0; w < W; ++w)
       ll += wave_l[w][t * kKeys + j] * fast_exp2(wave_m[w][t * kKeys + j] - mm);
     const float sc = fast_exp2(m[t] - mm);
-    const float inv = nparts > 1 ? 1.0f : ll > 0.0f ? 1.0f / ll : 0.0f;
     // row j of the tile, this wave's part; its K rows are no longer needed
 #pragma unroll
     for (int u = 0; u < kNV; ++u)
@@ -408,7 +415,7 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
         for (int e = 0; e < kVE; ++e)
           ks[wv][j][16 * kVE * u + kVE * (4 * g + i) + e] = o[t][u * kVE + e][i] * sc;
     if (wv == 0 && g == 0) {
-      inv_l[j] = inv;
+      row_l[j] = nparts > 1 || ll == 0.0f ? 1.0f : ll;   // a row without keys: 0 / 1
       const int r = r_first + t * kKeys + j;
       if (nparts > 1 && r < n_rows)   // decode: one query, row r is head r of the group
         reinterpret_cast<float2*>(a.part_ml)[((int64_t)b * a.H + kvh * G + r) * a.P + p] =
@@ -423,13 +430,13 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
         const float4 y = *reinterpret_cast<const float4*>(&ks[w][rr][c]);
         x = make_float4(x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
       }
-      const float f = inv_l[rr];
+      const float f = row_l[rr];
       const int r = r_first + t * kKeys + rr;
       if (r < n_rows) {
         float* dst = nparts > 1
                          ? a.part_acc + (((int64_t)b * a.H + kvh * G + r) * a.P + p) * D + c
                          : a.out + out_row(r) + c;
-        *reinterpret_cast<float4*>(dst) = make_float4(x.x * f, x.y * f, x.z * f, x.w * f);
+        *reinterpret_cast<float4*>(dst) = make_float4(x.x / f, x.y / f, x.z / f, x.w / f);
       }
     }
     __syncthreads();

@@ -142,3 +142,67 @@ def test_rows_do_not_see_later_values(bad, dtype, D, H, Hkv):
         assert (got[hit] == bad).all()
     # the others: the same values, up to the order of the sums in that tile
     assert _rel(got[~hit], clean[~hit].double()) <= REL
+
+
+def _fma(a, b, c):
+    return (a.double() * b.double() + c.double()).float()
+
+
+def _tree(parts):
+    while len(parts) > 1:
+        half = len(parts) // 2
+        parts = [parts[i] + parts[i + half] for i in range(half)]
+    return parts[0]
+
+
+def _row_walk(q, k, v):
+    """One query row against its keys in fp32, summed as the VALU kernel sums:
+    scores in chains of the elements of a 16-byte load and a tree over the
+    lanes of a token, values in chains over the tokens of a lane group and a
+    tree over the groups.  q [R, D], k and v [R, n, D]."""
+    D = q.shape[1]
+    vec = 16 // k.element_size()
+    k, v = k.float(), v.float()
+    qs = q * (math.log2(math.e) / math.sqrt(D))
+    parts = []
+    for c in range(D // vec):
+        x = torch.zeros(k.shape[:2])
+        for e in range(c * vec, (c + 1) * vec):
+            x = _fma(qs[:, None, e], k[..., e], x)
+        parts.append(x)
+    s = _tree(parts)
+    p = torch.exp2(s.double() - s.amax(1, keepdim=True).double()).float()
+    tokens = 64 // (D // vec)
+    accs, sums = [], []
+    for r in range(tokens):
+        acc, total = torch.zeros_like(q), torch.zeros(q.shape[0])
+        for t in range(r, k.shape[1], tokens):
+            acc, total = _fma(p[:, t, None], v[:, t], acc), total + p[:, t]
+        accs.append(acc)
+        sums.append(total)
+    return _tree(accs) * (1.0 / _tree(sums))[:, None]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D,H,Hkv,batch,keys", [
+    (128, 32, 32, 32, 17), (128, 32, 32, 8, 64), (128, 32, 8, 128, 17), (128, 32, 8, 96, 40),
+    (256, 8, 4, 16, 17), (64, 12, 12, 64, 33), (32, 8, 8, 128, 33)])
+def test_sums_no_further_off_than_the_row_walk(dtype, D, H, Hkv, batch, keys):
+    """With few keys the error is that of the scores' sums.  It must not exceed
+    the VALU kernel's order of sums (its error is computed here): both are
+    random walks over at least 500 rows of D values, so a tenth between their
+    2-norms is more than chance gives."""
+    q, k, v, bt, ctx = _case([1] * batch, [keys] * batch, H, Hkv, D, 8, dtype, seed=keys + D)
+    q = torch.randn(q.shape, generator=torch.Generator().manual_seed(D))
+    want = _want(q, k, v, bt, ctx, [1] * batch)
+    pages = bt[:, :-(-keys // 8)].long()
+    kk, vv = (x[pages].reshape(batch, -1, Hkv, D)[:, :keys].repeat_interleave(H // Hkv, 2)
+              .permute(0, 2, 1, 3).reshape(batch * H, keys, D) for x in (k, v))
+    walk = _row_walk(q.reshape(-1, D), kk, vv).view(q.shape)
+    got = _run(q, k, v, bt, ctx, [1] * batch)
+    assert _rel(got, want) <= 1.1 * _rel(walk, want)
+    from heteroserve import _hip
+
+    got = _hip.decode(q.to(DEV), k.to(DEV), v.to(DEV), bt.to(DEV), ctx.to(DEV),
+                      1.0 / math.sqrt(D), num_splits=1).cpu()
+    assert _rel(got, want) <= 1.1 * _rel(walk, want)
