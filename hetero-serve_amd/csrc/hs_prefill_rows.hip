@@ -113,7 +113,6 @@ __device__ inline void wave_lds_fence() {
 }
 
 // Scheduling barrier mask: everything but matrix instructions may cross it.
-// Without it the compiler holds the results of many products at once.
 constexpr int kAllButProducts = 0x3F6;
 
 // The products of 4 dims or keys, summed.
@@ -128,7 +127,7 @@ __device__ inline float4x product4(float a, float b) {
 // products, it was up to 1.6 times that of the VALU kernel's chains of 4 or 8
 // and trees over the lanes (2-norm against fp64, head dim 128, 17 keys, bf16:
 // 1.79e-7, 1.12e-7 there, 1.12e-7 so).
-template <int N, int NT>
+template <int N, int NT, bool kHold>
 __device__ inline void dot_tree(const float* k, const float* q, int step, float4x (&s)[NT]) {
   if constexpr (N == 1) {
     const float4 kf = *reinterpret_cast<const float4*>(k);
@@ -137,12 +136,12 @@ __device__ inline void dot_tree(const float* k, const float* q, int step, float4
       const float4 qf = *reinterpret_cast<const float4*>(q + t * step);
       s[t] = (product4(kf.x, qf.x) + product4(kf.y, qf.y)) +
              (product4(kf.z, qf.z) + product4(kf.w, qf.w));
-      __builtin_amdgcn_sched_barrier(kAllButProducts);
+      if constexpr (kHold) __builtin_amdgcn_sched_barrier(kAllButProducts);
     }
   } else {
     float4x r[NT];
-    dot_tree<N / 2, NT>(k, q, step, s);
-    dot_tree<N / 2, NT>(k + 2 * N, q + 2 * N, step, r);
+    dot_tree<N / 2, NT, kHold>(k, q, step, s);
+    dot_tree<N / 2, NT, kHold>(k + 2 * N, q + 2 * N, step, r);
 #pragma unroll
     for (int t = 0; t < NT; ++t) s[t] += r[t];
   }
@@ -302,7 +301,8 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
 
     // S^T: lane (j, g) gets keys 4 g + i of row j of each row tile.
     float4x s[NT];
-    dot_tree<D / 16, NT>(&ks[wv][j][g * (D / 4)], &qs[j][g * (D / 4)], kKeys * kRow, s);
+    dot_tree<D / 16, NT, sizeof(T) == 4 && D <= 64>(&ks[wv][j][g * (D / 4)], &qs[j][g * (D / 4)],
+                                                    kKeys * kRow, s);
     wave_lds_fence();
 
     const int t0 = lo + n * kKeys;
@@ -359,7 +359,6 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
             for (int i = 0; i < 4; ++i)
               x[i] = product4(word_elem<T>(vr[i][u], e), p[t][i]);
             o[t][u * kVE + e] += (x[0] + x[1]) + (x[2] + x[3]);
-            __builtin_amdgcn_sched_barrier(kAllButProducts);
           }
     } else {
 #pragma unroll 1
@@ -481,26 +480,43 @@ void launch_shape(const RowAttnArgs& a, int64_t rows_per_pair, int cus, hipStrea
   hipLaunchKernelGGL((rows_prefill_kernel<T, D, NT, W>), grid, block, 0, stream, ra);
 }
 
-// The workgroup's shape.  Measured on MI355X (us, rows x waves 16 x 4 / 16 x 8
-// / 32 x 8; one sequence unless said):
-//   12 heads, D 64, fp32, 512 rows on 512 tokens     27 / 24 / 26
-//   the same, 16 rows on 1000                         20 / 17 / 25
-//   32 heads, D 128, fp32, 512 rows on 512            89 / 90 / 86
-//   32 / 8 heads, D 128, bf16, 256 rows on 512        38 / 39 / 37
-//   32 / 8 heads, D 128, fp16, 9 rows on 3000         87 / 72 / 121
-//   8 / 4 heads, D 256, fp32, 700 rows on 1000        142 / 170 / -
-// (the row kernel before: 117, 59, 766, 109, 442, 803).  So 8 waves of 16
-// rows; 32 rows, which read K and V half as often, once they still give every
-// CU two workgroups; and 4 waves at head dim 256, where the registers hold
-// one wave a SIMD.
+// The workgroup's shape: 8 waves of 16 rows, and 4 at head dim 256, where the
+// registers hold one wave a SIMD.  Measured on MI355X (us, rows x waves 16 x 4 /
+// 16 x 8 with an earlier order of sums, 5 to 20% cheaper than this one; one
+// sequence):
+//   12 heads, D 64, fp32, 512 rows on 512 tokens     27 / 24
+//   the same, 16 rows on 1000                         20 / 17
+//   32 / 8 heads, D 128, bf16, 256 rows on 512        38 / 39
+//   32 / 8 heads, D 128, fp16, 9 rows on 3000         87 / 72
+//   8 / 4 heads, D 256, fp32, 700 rows on 1000        142 / 170
+//
+// 32 rows halve what is read of K and V but hold twice the state, which at
+// head dim 128 spills.  16 / 32 rows, us, 64 sequences unless said:
+//   8 heads, D 32, bf16, 128 rows on 64 / on 1024     49 / 38, 175 / 136
+//   the same, fp32, 128 rows on 64                    0.93 of the time with 16
+//   12 heads, D 64, fp32, 32 rows on 512 / on 1024    77 / 72, 151 / 115
+//   the same, bf16                                    0.90 to 0.94
+//   16 sequences, 12 heads, D 64, fp32, 512 rows      136 / 153
+//   3 sequences, 32 heads, D 128, fp32, 512 rows      157 / 309
+// So 32 rows, where there are more than 16 and every CU gets two workgroups
+// either way: with 16-bit caches at head dim 32; and with fp32 ones where every
+// sequence has one row tile instead of two and long rows of K and V to read.
 template <typename T, int D>
 void launch_d(const RowAttnArgs& a, int64_t rows_per_pair, int cus, hipStream_t stream) {
   if constexpr (D == 256) {
     launch_shape<T, D, 1, 4>(a, rows_per_pair, cus, stream);
   } else {
-    const int64_t wide = sat_mul(ceil_div(rows_per_pair, 2 * kKeys), a.B, a.Hkv);
-    if (wide >= 2 * (int64_t)cus) launch_shape<T, D, 2, 8>(a, rows_per_pair, cus, stream);
-    else launch_shape<T, D, 1, 8>(a, rows_per_pair, cus, stream);
+    if constexpr (D == 32 || (D == 64 && sizeof(T) == 4)) {
+      const int64_t wide = sat_mul(ceil_div(rows_per_pair, 2 * kKeys), a.B, a.Hkv, a.P);
+      const bool pays = sizeof(T) == 2
+                            ? D == 32
+                            : !a.cu_q && rows_per_pair <= 2 * kKeys && (int64_t)a.MB * a.BS >= 1024;
+      if (pays && rows_per_pair > kKeys && wide >= 2 * (int64_t)cus) {
+        launch_shape<T, D, 2, 8>(a, rows_per_pair, cus, stream);
+        return;
+      }
+    }
+    launch_shape<T, D, 1, 8>(a, rows_per_pair, cus, stream);
   }
 }
 

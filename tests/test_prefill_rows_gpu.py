@@ -206,3 +206,29 @@ def test_sums_no_further_off_than_the_row_walk(dtype, D, H, Hkv, batch, keys):
     got = _hip.decode(q.to(DEV), k.to(DEV), v.to(DEV), bt.to(DEV), ctx.to(DEV),
                       1.0 / math.sqrt(D), num_splits=1).cpu()
     assert _rel(got, want) <= 1.1 * _rel(walk, want)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 128), (torch.bfloat16, 64),
+                                     (torch.bfloat16, 32), (torch.float32, 64)])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33])
+def test_few_rows_of_many_sequences(dtype, D, rows):
+    """A row tile or two of each of 64 sequences, 8 heads: grids of 512
+    workgroups, on both sides of the rule for the 32-row tile."""
+    chunks = [rows] * 64
+    ctxs = [rows + 3 * i for i in range(64)]
+    args = _case(chunks, ctxs, 8, 8, D, 16, dtype, seed=rows)
+    assert _rel(_run(*args, chunks), _want(*args, chunks)) <= REL
+
+
+def test_uniform_chunks_on_long_prefixes():
+    """32-row tiles of an fp32 cache: uniform chunks of 17 to 32 rows on tables of
+    1024 tokens or more."""
+    from heteroserve.model.paged_attn_prefill import paged_attention_prefill
+
+    for S, n in ((17, 1024), (32, 1040), (32, 1008)):
+        chunks, ctxs = [S] * 64, [n - (i % 7) for i in range(64)]
+        q, k, v, bt, ctx = _case(chunks, ctxs, 8, 8, 32, 16, torch.float32, seed=S)
+        bt = bt[:, :-(-n // 16)].contiguous()
+        got = paged_attention_prefill(q.view(64, S, 8, 32).to(DEV), k.to(DEV), v.to(DEV),
+                                      bt.to(DEV), ctx.to(DEV), 1.0 / math.sqrt(32)).cpu()
+        assert _rel(got.view(q.shape), _want(q, k, v, bt, ctx, chunks)) <= REL
