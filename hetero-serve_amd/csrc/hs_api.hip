@@ -690,8 +690,10 @@ static int prefill_common(const float* q, const int32_t* cu_q, int S, int max_ro
   a.splits = 1;
   a.P = 1;
   a.qscale = scale * kLog2e;
-  if (rows_serves(a, kv_dtype, D)) return launch_rows(a, kv_dtype, D, current_cus(), st);
-  return launch_row_attn(a, kv_dtype, D, current_cus(), st);
+  const int cus = current_cus();
+  if (rows_serves(a, kv_dtype, D) && rows_prefill_pays(a, kv_dtype, D, cus))
+    return launch_rows(a, kv_dtype, D, cus, st);
+  return launch_row_attn(a, kv_dtype, D, cus, st);
 }
 
 int hs_prefill(const float* q, const void* k_cache, const void* v_cache, int kv_dtype,

@@ -172,6 +172,8 @@ int launch_block_tables(const int32_t* packed, int B, int width, int32_t* out,
 // that its 32-bit offsets and positions cannot hold (a cache of 256 GiB, a table
 // of 2^30 tokens); launch_row_attn's one wave per row takes those.
 bool rows_serves(const RowAttnArgs& a, int kv_dtype, int D);
+// Whether a prefill that it serves is faster there than one wave per row.
+bool rows_prefill_pays(const RowAttnArgs& a, int kv_dtype, int D, int cus);
 int launch_rows(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream);
 
 // Matrix-core causal prefill (hs_prefill_mfma.hip).  cu_q null: S rows per

@@ -39,6 +39,8 @@
 // row must not see values past its own position.  Tiles in which some row
 // masks some key therefore look at their V values, and one with a non-finite
 // value adds its keys one by one, to the rows that see them.
+#include <algorithm>
+
 #include "hs_kernels.h"
 
 namespace hs {
@@ -538,6 +540,36 @@ bool rows_serves(const RowAttnArgs& a, int kv_dtype, int D) {
   return tiles > 0 && tiles <= 0x7fffffffLL && sat_mul(a.S, a.H / a.Hkv) <= (1LL << 30) &&
          sat_mul(a.NB, a.BS, (int64_t)a.Hkv * (D * elem / 64)) <= 0xffffffffLL &&
          sat_mul(a.MB, a.BS) <= (1LL << 30);
+}
+
+// A workgroup here costs its set-up (8 us alone, 22 to 40 ns each in a full
+// device) whatever its keys are; the VALU kernel costs each row its keys.  us,
+// VALU / here, chunks of rows x keys of the table:
+//   1 chunk,  32 heads of 8 groups, D 128, fp32    8 x 8 7.2 / 8.5, 8 x 24 11.6 / 8.6
+//   1 chunk,  8 heads of 4 groups, D 256, bf16     8 x 8 6.7 / 12.6, 8 x 40 11.3 / 12.7
+//   64 chunks, 32 heads, D 128, fp32               2 x 66 37 / 73, 2 x 258 128 / 124,
+//                                                  8 x 8 24 / 48, 8 x 72 107 / 75
+//   64 chunks, 32 heads of 8 groups, D 128, bf16   8 x 72 29 / 36, 8 x 264 76 / 62
+// With one head a group the rows of a tile are what the VALU kernel repeats; with
+// grouped heads a wave there serves up to 8 of them.  Ragged chunks have tiles
+// that are empty here.  Over 22000 shapes (1 to 128 chunks of 1 to 128 rows, tables
+// of 16 to 640 tokens) the rule is within 2% of the better kernel in the mean.
+bool rows_prefill_pays(const RowAttnArgs& a, int kv_dtype, int D, int cus) {
+  const bool half = kv_dtype != HS_DTYPE_F32;
+  const int G = a.H / a.Hkv;
+  const int64_t rows = (int64_t)a.S * G;
+  int keys;   // up to here the VALU kernel
+  if (sat_mul(ceil_div(rows, kKeys), a.B, a.Hkv) < 2 * (int64_t)cus) {
+    keys = D == 256 ? (half ? 64 : 32) : G == 1 ? 32 : 16;
+  } else if (G == 1) {
+    keys = 640 / (int)std::min<int64_t>(rows, kKeys);
+    if (D >= 128 && half) keys *= 2;
+    if (D == 32) keys /= 2;
+  } else {
+    keys = G > 4 ? (half ? 40 : 32) : D >= 128 && half ? 112 : 64;
+    if (a.cu_q) keys = keys * 3 / 2;
+  }
+  return (int64_t)a.MB * a.BS > keys;
 }
 
 int launch_rows(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t stream) {

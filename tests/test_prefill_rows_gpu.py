@@ -232,3 +232,17 @@ def test_uniform_chunks_on_long_prefixes():
         got = paged_attention_prefill(q.view(64, S, 8, 32).to(DEV), k.to(DEV), v.to(DEV),
                                       bt.to(DEV), ctx.to(DEV), 1.0 / math.sqrt(32)).cpu()
         assert _rel(got.view(q.shape), _want(q, k, v, bt, ctx, chunks)) <= REL
+
+
+@pytest.mark.parametrize("H,Hkv,D,dtype", [(4, 4, 64, torch.float32), (8, 2, 128, torch.bfloat16),
+                                           (16, 1, 128, torch.float32), (4, 2, 256, torch.float16)])
+@pytest.mark.parametrize("batch", [3, 200])
+@pytest.mark.parametrize("keys", [16, 32, 48, 64, 96, 112, 160, 176])
+def test_both_kernels_of_short_tables(H, Hkv, D, dtype, batch, keys):
+    """Tables of 16 to 176 tokens, on both sides of the lines below which a wave
+    per row serves the chunks: few sequences and a full device, ragged rows."""
+    chunks = [1 + (5 * i) % min(13, keys) for i in range(batch)]
+    ctxs = [max(n, keys - 3 * (i % 5)) for i, n in enumerate(chunks)]
+    q, k, v, bt, ctx = _case(chunks, ctxs, H, Hkv, D, 16, dtype, seed=keys)
+    bt = bt[:, :-(-max(ctxs) // 16)].contiguous()
+    assert _rel(_run(q, k, v, bt, ctx, chunks), _want(q, k, v, bt, ctx, chunks)) <= REL
