@@ -194,17 +194,18 @@ static bool short_rows_in_wg(int H, int Hkv, int D, int kv_dtype, int64_t width)
 
 // Decode by explicit splits: the slices that are taken together.  Neighbouring
 // slices are one key range, so several at once write (and merge) fewer
-// states.  `fill` parts in all rows are enough, and at least 512 keys of the
-// longest row that the table holds for a wave of its own; no part gets fewer
-// than 128 (a wave) or 256 (a workgroup of 8).  Against one state per slice,
-// us: 8 sequences of 256..4096 tokens, 12 heads, D 64, fp32 (64 splits) 29 /
-// 25; 16 of them, 32 / 8 heads, bf16 49 / 43; 64 of up to 8192, 32 heads, bf16
-// 553 / 488.
-static int slices_together(int splits, int64_t units, int64_t width, int64_t fill, bool waves) {
-  int64_t parts = ceil_div(fill, units);
-  if (waves) parts = std::max(parts, ceil_div(width, 512));
-  parts = std::min({parts, ceil_div(width, waves ? 128 : 256), (int64_t)splits});
-  return (int)ceil_div(splits, std::max((int64_t)1, parts));
+// states: `parts` of them, or more where so few would lengthen the longest chain
+// of additions past that of one state per slice (a wave adds up the tokens that
+// its lane groups see in turn, `tpl` a step; a workgroup the states of its
+// `waves`; the merge those of all slices).  One wave of 32 heads, D 128, fp32, 128
+// sequences of 200 tokens in 7 slices: 1.56e-7 from fp64, with the slices in
+// pairs 2.24e-7.
+static int slices_together(int splits, int64_t parts, int64_t width, int tpl, int waves) {
+  const int64_t slice = ceil_div(ceil_div(width, splits), tpl);   // steps of one slice
+  for (int64_t p = std::max((int64_t)1, std::min(parts, (int64_t)splits));; ++p) {
+    const int64_t s = ceil_div(splits, p);
+    if (s <= waves || ceil_div(s * slice, waves) + waves <= slice + splits) return (int)s;
+  }
 }
 
 // Multi-head decode in one pass: a workgroup (8 waves) per (row, head) rather
@@ -504,12 +505,35 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
     } else if (num_splits == 1) {
       a.wg = mha && wg_per_row((int64_t)B * H, width, cus);
     } else if (num_splits > 1) {
-      // workgroups of 8 waves, a few for each CU, or waves, 16 for each CU
+      // Multi-head attention: workgroups of 8 waves, three for each CU, of at
+      // least 256 keys, or 512 where that many fill a round of the device (1024
+      // where there is a row for every CU).  Waves, one a slice or 16 for each CU,
+      // where rows that fill two rounds are short, or the slices fill the device and
+      // are long.  us, one state per slice / at least 256 keys / so: 64
+      // sequences of 16..64 tokens, 32 heads, D 128, bf16 17 / 41 / 17; 32 of
+      // 128..512, 12 heads, D 64, fp32 22 / 23 / 18; 4 of 8k..32k, 16 heads, bf16 65 / 76
+      // / 66; 8 of 1k..4k, 12 heads, fp32 33 / 32 / 32.  Grouped heads on the VALU
+      // kernel: waves, cut no shorter than the caller's slices: 4 sequences of 32..128 tokens,
+      // 32 / 8 heads, bf16 11 / 23 / 11.
       const int64_t units = a.mma ? sat_mul(B, Hkv, ceil_div(H / Hkv, 16))
                                   : sat_mul(B, H / row_attn_heads_per_wave(H, Hkv));
-      a.wg = mha && sat_mul(units, num_splits) < 64 * (int64_t)cus;
-      a.slices = slices_together(num_splits, units, width,
-                                 (a.mma ? 2 : a.wg ? 3 : 16) * (int64_t)cus, !a.mma && !a.wg);
+      const int tpl = a.mma ? 16 : row_attn_tokens_per_load(kv_dtype, D);
+      a.wg = mha && sat_mul(units, num_splits) < 64 * (int64_t)cus &&
+             (units <= 2 * (int64_t)cus || width > 128) &&
+             (sat_mul(units, num_splits) < 8 * (int64_t)cus || width < 256 * (int64_t)num_splits);
+      int64_t parts = ceil_div((a.mma ? 2 : a.wg ? 3 : 16) * (int64_t)cus, units);
+      if (a.mma) {
+        parts = std::min(parts, ceil_div(width, 256));
+      } else if (a.wg) {
+        int64_t cap = ceil_div(width, units >= cus ? 1024 : 512);
+        if (units < cus && width > 512 && (units * cap > cus || 2 * units * cap < cus))
+          cap = ceil_div(width, 256);
+        if (units < 2 * (int64_t)cus) parts = std::max(parts, ceil_div(width, 1024));
+        parts = std::min(parts, cap);
+      } else {
+        parts = std::max(parts, ceil_div(width, 512));
+      }
+      a.slices = slices_together(num_splits, parts, width, tpl, a.mma || a.wg ? 8 : 1);
       a.P = (int)ceil_div(num_splits, a.slices);
     }
     a.ranked = a.wg && B > 1 && B <= 64 && (int64_t)B * H > cus;

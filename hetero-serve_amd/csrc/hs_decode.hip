@@ -229,6 +229,10 @@ __global__ __launch_bounds__(256) void row_attn_merge_kernel(RowAttnArgs a) {
 // host launch
 // ---------------------------------------------------------------------------
 
+int row_attn_tokens_per_load(int kv_dtype, int D) {
+  return 64 / (D / (kv_dtype == HS_DTYPE_F32 ? 4 : 8));
+}
+
 // Query heads per wave: the largest of 1, 2, 4, 8 dividing the GQA group.
 int row_attn_heads_per_wave(int H, int Hkv) {
   const int group = H / Hkv;

@@ -136,6 +136,9 @@ void launch_splitmm_even(const RowAttnArgs& a, int kv_dtype, int D, hipStream_t 
 // Query heads one wave of the VALU kernel serves: 1, 2, 4 or 8.
 int row_attn_heads_per_wave(int H, int Hkv);
 
+// Tokens that one load of a wave of the VALU kernel covers.
+int row_attn_tokens_per_load(int kv_dtype, int D);
+
 int launch_page_copy(const void* pool, void* buf, bool unpack, int L, int NB, int64_t page_bytes,
                      const int64_t* ids, int n, hipStream_t stream);
 

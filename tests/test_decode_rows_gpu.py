@@ -118,3 +118,71 @@ def test_values_past_the_context(splits):
             x[bt[b, n // 16], n % 16:] = math.nan if b else math.inf
     got = _hip.decode(*(x.to(DEV) for x in (q, k, v, bt, ctx)), scale, num_splits=splits).cpu()
     assert ((got.double() - want).norm() / want.norm()).item() <= REL
+
+
+def _fma(a, b, c):
+    return (a.double() * b.double() + c.double()).float()
+
+
+def _tree(parts):
+    while len(parts) > 1:
+        half = len(parts) // 2
+        parts = [parts[i] + parts[i + half] for i in range(half)]
+    return parts[0]
+
+
+def _sliced_walk(q, k, v, splits):
+    """One query row against its keys in fp32, a state per slice, summed as the
+    VALU kernel sums a slice (chains over the elements of a 16-byte load and the
+    tokens of a lane group, trees over lanes and groups) and the merge adds the
+    slices up.  q [R, D], k and v [R, n, D]."""
+    n, D = k.shape[1:]
+    vec = 16 // k.element_size()
+    tokens = 64 // (D // vec)
+    k, v = k.float(), v.float()
+    qs = q * (math.log2(math.e) / math.sqrt(D))
+    parts = []
+    for c in range(D // vec):
+        x = torch.zeros(k.shape[:2])
+        for e in range(c * vec, (c + 1) * vec):
+            x = _fma(qs[:, None, e], k[..., e], x)
+        parts.append(x)
+    s = _tree(parts)
+    p = torch.exp2(s.double() - s.amax(1, keepdim=True).double()).float()
+    acc, total = torch.zeros_like(q), torch.zeros(q.shape[0])
+    size = -(-n // splits)
+    for lo in range(0, n, size):
+        accs, sums = [], []
+        for r in range(tokens):
+            a, t_sum = torch.zeros_like(q), torch.zeros(q.shape[0])
+            for t in range(lo + r, min(lo + size, n), tokens):
+                a, t_sum = _fma(p[:, t, None], v[:, t], a), t_sum + p[:, t]
+            accs.append(a)
+            sums.append(t_sum)
+        acc, total = acc + _tree(accs), total + _tree(sums)
+    return acc * (1.0 / total)[:, None]
+
+
+@pytest.mark.parametrize("dtype,H,Hkv,D,batch,n,splits", [
+    (torch.float32, 32, 32, 128, 128, 200, 7), (torch.float32, 8, 4, 256, 128, 64, 7),
+    (torch.bfloat16, 8, 4, 256, 16, 200, 7), (torch.float32, 32, 8, 128, 128, 64, 7),
+    (torch.float32, 12, 12, 64, 32, 500, 16), (torch.bfloat16, 32, 8, 64, 8, 700, 64)])
+def test_splits_no_further_off_than_their_slices(dtype, H, Hkv, D, batch, n, splits):
+    """Slices that are taken together add up no longer chains than one state per
+    slice does: the error of that order, computed here, is not exceeded (both are
+    random walks over at least 96 rows of D values; a tenth is more than chance
+    gives)."""
+    from heteroserve import _hip
+
+    case = _case([n] * batch, H, Hkv, D, 8, dtype, seed=splits + n)
+    q, k, v, bt, _, scale = case
+    want = _want(*case)
+    pages = bt[:, :-(-n // 8)].long()
+    kk, vv = (x[pages].reshape(batch, -1, Hkv, D)[:, :n].repeat_interleave(H // Hkv, 2)
+              .permute(0, 2, 1, 3).reshape(batch * H, n, D) for x in (k, v))
+    rows = slice(0, 512)
+    walk = _sliced_walk(q.reshape(-1, D)[rows], kk[rows], vv[rows], splits)
+    exact = want.reshape(-1, D)[rows]
+    limit = 1.1 * ((walk.double() - exact).norm() / exact.norm()).item()
+    got = _hip.decode(*(x.to(DEV) for x in case[:5]), scale, num_splits=splits).cpu().double()
+    assert ((got - want).norm() / want.norm()).item() <= limit
