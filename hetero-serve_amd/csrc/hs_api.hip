@@ -170,26 +170,35 @@ static int rows_partition(int B, int H, int Hkv, int D, int BS, int MB, int defa
 // workgroup per (row, head).
 constexpr int64_t kWgSplitMaxTokens = 1024;
 
-// The default decomposition of a small grid whose rows are short: instead of
-// partitions cut down to a few tokens and a merge launch, one workgroup per
-// (row, head) splits the row's keys over its waves and combines their states
-// in LDS (the caller's workspace goes unused).  Applies to plain multi-head
-// attention where the partition above was shortened for the grid.  Measured
-// on C1 (8 sequences, 12 heads, head dim 64, fp16, up to 512 tokens): step
-// 14.3 us with 32-token partitions and the merge, 12.6 us so.
-static bool wg_split_applies(int B, int H, int Hkv, int BS, int MB, int kv_dtype, int D) {
-  if (H != Hkv || (int64_t)MB * BS > kWgSplitMaxTokens) return false;
-  return default_partition(B, H, Hkv, BS, MB, kv_dtype, D) < kDefaultPartition;
-}
-
-// Short rows of groups of 2 and 4 at head dim 256 go the same way, each query
-// head a workgroup of its own: the group's pages come from the caches again,
-// which up to 512 tokens (fp32: 256) costs less than the states and the merge.
-// 8 / 4 heads, fp16, 32 sequences of 128..512 tokens, VALU partitions / so: 21.5 /
-// 16.1 us; fp32, of 64..256 tokens, fp32 matrix cores / so: 19.4 / 16.6.
-static bool short_rows_in_wg(int H, int Hkv, int D, int kv_dtype, int64_t width) {
-  return D > 128 && H != Hkv && H / Hkv <= 4 && row_attn_heads_per_wave(H, Hkv) == H / Hkv &&
-         width <= (kv_dtype == HS_DTYPE_F32 ? 256 : 512);
+// The default decomposition of a small grid whose rows are short (where the
+// partition above was shortened for the grid): instead of partitions cut down to
+// a few tokens and a merge launch, one workgroup per (row, heads) splits the
+// row's keys over its waves and combines their states in LDS (the caller's
+// workspace goes unused).  Measured on C1 (8 sequences, 12 heads, head dim 64,
+// fp16, up to 512 tokens): step 14.3 us with 32-token partitions and the merge,
+// 12.6 us so.
+//
+// Query heads of such a workgroup, or 0 for another kernel.  Multi-head attention
+// has one.  A group of 2 or 4 walks its keys once for all its heads, but where that
+// leaves CUs idle at head dim 256 each head its own; larger groups go to the
+// fp32 matrix cores, and groups of 4 where that measured faster (head dims to 64;
+// rows past 256 tokens; 16-bit rows of up to 64).  us, a head / the group / the fp32
+// matrix cores: 8 / 4 heads, D 256, bf16, 64 sequences of 64..256 tokens 23 / 14 / -,
+// 32 of 128..512 20 / 22 / -; 16 / 8 heads, D 64, fp32, 4 of 64..256 - / 7.5 / 10.4;
+// 32 / 8 heads, D 128, 8-token blocks, bf16, 32 of 64..256 - / 12.2 / 15, 32 of
+// 128..512 - / 16.7 / 23, 8 of 128..512 - / 16 / 14, 32 of 16..64 - / 9.6 / 8; fp32, 64 of
+// 16..64 - / 13.3 / 16.
+static int short_rows_heads(int B, int H, int Hkv, int D, int kv_dtype, int64_t width, int cus) {
+  const int G = H / Hkv, Gw = row_attn_heads_per_wave(H, Hkv);
+  const bool half = kv_dtype != HS_DTYPE_F32;
+  if (G > 4) return 0;
+  if (D > 128) {
+    if (sat_mul(B, H) > cus || width <= 64) return Gw;
+    return width <= (half ? 512 : 256) ? 1 : 0;
+  }
+  if (G < 4) return Gw;
+  if (D < 128 || (half && width <= 64)) return 0;
+  return width <= 256 || (half && width <= 512 && sat_mul(B, Hkv) >= cus / 2) ? Gw : 0;
 }
 
 // Decode by explicit splits: the slices that are taken together.  Neighbouring
@@ -218,26 +227,46 @@ static bool wg_per_row(int64_t rows_heads, int64_t width, int cus) {
 }
 
 // Grouped heads that the split-operand kernel does not take (fp32 caches, other
-// block sizes, head dim 256, explicit splits), on the fp32 matrix cores
+// block sizes, head dim 256, one pass, explicit splits), on the fp32 matrix cores
 // instead of the VALU kernel: a workgroup per KV head and partition, 16
-// columns for G heads.  With G = 2 or 4 the VALU kernel reads each page once
-// too and does less per byte, so it keeps 16-bit caches, and fp32 ones once
-// there is a workgroup for every CU and its waves fill the device; but in one
-// pass it has a single wave per row.  Sequences of 256..4096 tokens, us VALU /
-// here: 32 / 8 heads fp32, 8 / 16 / 24 / 32 / 64 sequences 93 / 35, 99 / 61,
-// 122 / 100, 124 / 129, 250 / 286; 16 of them in bf16 with 8-token blocks 56 /
-// 59, in one pass 613 / 95; 32 / 4 heads fp32, 16 / 64 sequences 103 / 35, 223 /
-// 140; 16 / 1 heads 94 / 18; 8 / 4 heads, D 256, fp32, 32 / 64 sequences 225 /
-// 144, 268 / 280.  Short rows, whose default partitions the VALU kernel has cut
-// for a small grid, come here up to head dim 128: 32 / 8 heads, 8-token blocks,
-// fp16, 16 sequences of 256..1024 tokens 31.7 / 21.3, 32 of 64..256 19.9 / 12.2,
-// 32 of them in fp32 29.2 / 13.7.
-static bool grouped_on_matrix_cores(int B, int H, int Hkv, int kv_dtype, int num_splits,
-                                    bool short_rows, int cus) {
+// columns for G heads.  Groups of 5 and more always.  With G = 2 or 4 the VALU
+// kernel reads each page once too and does less per byte (with G = 3 it reads
+// it for every head), so it keeps 16-bit caches, and fp32 ones once there is a
+// workgroup for every CU or long rows give its waves enough to do.  In one pass
+// it has a single wave per row, which loses until there are about two
+// workgroups' worth of rows for each CU and the rows are short.  us, VALU / here, 16
+// to 64 tokens at the shortest and a quarter of the longest named:
+//   partitions  32 / 8 heads, D 128, fp32, 8 and 16 sequences of up to 4096 95 / 43,
+//               100 / 73, 16 of up to 8192 124 / 148; 16 / 8 heads, D 64, fp32, 4 of
+//               up to 32768 66 / 84
+//   one pass    32 / 8 heads, D 128, bf16, 64 of up to 256 44 / 26, 128 of up to 256
+//               48 / 51, of up to 512 90 / 78, 256 of up to 512 96 / 138; fp32,
+//               256 of up to 256 94 / 98
+//   splits      32 / 8 heads, D 128, fp32, 16 of up to 128 17 / 10; 16 / 8 heads, 4 of up to
+//               4096 27 / 37; 8 / 4 heads, D 256, fp32, 8 of up to 4096 46 / 67
+static bool grouped_on_matrix_cores(int B, int H, int Hkv, int D, int kv_dtype, int num_splits,
+                                    int64_t width, bool short_rows, int cus) {
   const int G = H / Hkv;
+  const bool f32 = kv_dtype == HS_DTYPE_F32;
   if (G == 1) return false;
-  if (G > 4 || row_attn_heads_per_wave(H, Hkv) < G || num_splits == 1 || short_rows) return true;
-  return kv_dtype == HS_DTYPE_F32 && sat_mul(B, Hkv) < cus;
+  if (G > 4) return true;
+  const int64_t pairs = sat_mul(B, Hkv);
+  const bool long_keys = sat_mul(pairs, width) >= 2560 * (int64_t)cus;
+  if (num_splits > 1) {
+    if (D == 256) return f32 && pairs < 16 && width >= 8192;
+    return f32 && G > 2 && pairs < cus && (4 * pairs < cus || !long_keys);
+  }
+  if (num_splits == 1 || G == 3) {
+    const int64_t wgs = D == 256 && !f32 ? 2 * pairs : pairs;
+    if (wgs < 2 * (int64_t)cus) return true;
+    if (wgs == 2 * (int64_t)cus) return G == 4 || D == 256 || width > 256;
+    if (wgs <= 4 * (int64_t)cus) return width > 256 && (f32 || G > 2 || D == 256);
+    return width > 512 && (f32 || G == 3 || (G == 4 && D <= 64));
+  }
+  if (short_rows && D <= 128) return true;
+  if (!f32 || pairs >= cus) return false;
+  if (D == 256) return short_rows || pairs < 16 || 4 * pairs >= cus;
+  return (G == 4 || 4 * pairs >= cus) && !long_keys;
 }
 
 // The workspace queries take no kv dtype: they size for the shortest default
@@ -489,17 +518,18 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
     const int64_t width = (int64_t)MB * BS;
     const bool short_rows = num_splits == 0 && partition_tokens == 0 && width <= kWgSplitMaxTokens &&
                             plan.part_tokens < valu_partition(H, Hkv);
-    const bool wg_rows = short_rows && short_rows_in_wg(H, Hkv, D, kv_dtype, width);
-    a.mma = !wg_rows &&
-            grouped_on_matrix_cores(B, H, Hkv, kv_dtype, num_splits, short_rows && D <= 128, cus) &&
+    if (short_rows && !splitmm_serves(kv_dtype, BS, D, H, Hkv))
+      a.wg = mha ? 1 : short_rows_heads(B, H, Hkv, D, kv_dtype, width, cus);
+    // a caller's own partitions (which may be shorter than a workgroup's tiles)
+    // stay on the VALU kernel
+    a.mma = !a.wg && partition_tokens == 0 &&
+            grouped_on_matrix_cores(B, H, Hkv, D, kv_dtype, num_splits, width, short_rows, cus) &&
             !splitmm_applies(a, kv_dtype, D) && rows_serves(a, kv_dtype, D);
-    if (wg_rows || (num_splits == 0 && partition_tokens == 0 &&
-                    wg_split_applies(B, H, Hkv, BS, MB, kv_dtype, D))) {
+    if (a.wg) {
       // the workspace, sized for the partitions above, goes unused
       a.mode = 0;
       a.P = 1;
-      a.wg = 1;
-    } else if (num_splits == 0 && partition_tokens == 0 && a.mma) {
+    } else if (num_splits == 0 && a.mma) {
       a.part_tokens = rows_partition(B, H, Hkv, D, BS, MB, plan.part_tokens);
       a.P = (int)ceil_div(width, a.part_tokens);
     } else if (num_splits == 1) {
@@ -536,7 +566,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
       a.slices = slices_together(num_splits, parts, width, tpl, a.mma || a.wg ? 8 : 1);
       a.P = (int)ceil_div(num_splits, a.slices);
     }
-    a.ranked = a.wg && B > 1 && B <= 64 && (int64_t)B * H > cus;
+    a.ranked = a.wg && B > 1 && B <= 64 && (int64_t)B * (H / a.wg) > cus;
     const size_t acc = ((size_t)B * H * a.P * D * sizeof(float) + 255) & ~(size_t)255;
     a.part_ml = a.P > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + acc) : nullptr;
     return launch_row_attn(a, kv_dtype, D, cus, st);

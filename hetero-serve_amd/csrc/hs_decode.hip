@@ -89,30 +89,31 @@ __device__ inline int ranked_row(const RowAttnArgs& a, int k) {
   return __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < a.B && rank == k));
 }
 
-// One workgroup per (row, head, partition): its W waves walk W contiguous
-// slices of the keys and their states are combined through LDS, so a batch
-// too small to fill the CUs gets W times the waves without that many
+// One workgroup per (row, group of G heads, partition): its W waves walk W
+// contiguous slices of the keys and their states are combined through LDS, so
+// a batch too small to fill the CUs gets W times the waves without that many
 // partition states.  Each wave runs the same RowWalk as the partition kernel;
 // the combine is the log-sum-exp merge of paged_attn_v3.py:170-208 over the
 // slices.
-template <typename T, int D, bool kPaged, int W>
+template <typename T, int D, bool kPaged, int G, int W>
 __global__ __launch_bounds__(W * 64) void row_attn_wg_kernel(RowAttnArgs a) {
-  using Walk = RowWalk<T, D, kPaged, 1>;
-  __shared__ float s_m[W], s_l[W];
-  __shared__ float s_acc[W][D];
+  using Walk = RowWalk<T, D, kPaged, G>;
+  __shared__ float s_m[W][G], s_l[W][G];
+  __shared__ float s_acc[W][G][D];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = (int)(blockIdx.x % a.H);
-  const int rp = (int)(blockIdx.x / a.H);
+  const int n_hw = a.H / G;
+  const int h0 = (int)(blockIdx.x % n_hw) * G;
+  const int rp = (int)(blockIdx.x / n_hw);
   const int p = rp % a.P;
   const int row = a.ranked ? ranked_row(a, rp / a.P) : rp / a.P;
   int b, end;
   if (!row_geometry(a, row, b, end)) return;       // workgroup-uniform
-  const int64_t orow = ((int64_t)row * a.H + h) * D;
+  const int64_t orow0 = ((int64_t)row * a.H + h0) * D;
   int lo = 0, hi = end, nparts = 1;
-  if (end <= 0) {                                  // nothing to attend to: a zero row
+  if (end <= 0) {                                  // nothing to attend to: zero rows
     if (p == 0)
-      for (int d = threadIdx.x; d < D; d += W * 64) a.out[orow + d] = 0.0f;
+      for (int d = threadIdx.x; d < G * D; d += W * 64) a.out[orow0 + d] = 0.0f;
     return;
   }
   if (a.P > 1 && !partition_range(a, end, p, lo, hi, nparts)) return;
@@ -123,35 +124,39 @@ __global__ __launch_bounds__(W * 64) void row_attn_wg_kernel(RowAttnArgs a) {
   const int my_hi = wv == W - 1 ? hi : min(hi, first + chunk);
   Walk w;
   if (my_lo < my_hi)
-    w.run(KvPages{a.k, a.v, a.Hkv, a.BS, a.NB}, a.q + orow, a.qscale, h / (a.H / a.Hkv),
+    w.run(KvPages{a.k, a.v, a.Hkv, a.BS, a.NB}, a.q + orow0, a.qscale, h0 / (a.H / a.Hkv),
           a.bt + (int64_t)b * a.MB, my_lo, my_hi);
   else
     w.clear();
   if (Walk::slot(lane) == 0) {
     const int c = Walk::chunk(lane);
 #pragma unroll
-    for (int e = 0; e < Walk::kVec; ++e) s_acc[wv][c * Walk::kVec + e] = w.acc[0][e];
-    if (c == 0) {
-      s_m[wv] = w.m[0];
-      s_l[wv] = w.l[0];
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int e = 0; e < Walk::kVec; ++e) s_acc[wv][g][c * Walk::kVec + e] = w.acc[g][e];
+      if (c == 0) {
+        s_m[wv][g] = w.m[g];
+        s_l[wv][g] = w.l[g];
+      }
     }
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < D; d += W * 64) {
-    float mm = s_m[0];
+  for (int i = threadIdx.x; i < G * D; i += W * 64) {
+    const int g = i / D, d = i - g * D;
+    float mm = s_m[0][g];
 #pragma unroll
-    for (int v = 1; v < W; ++v) mm = fmaxf(mm, s_m[v]);
+    for (int v = 1; v < W; ++v) mm = fmaxf(mm, s_m[v][g]);
     float l = 0.0f, o = 0.0f;
 #pragma unroll
     for (int v = 0; v < W; ++v) {
-      const float wt = fast_exp2(s_m[v] - mm);   // an empty slice: exp2(-3e38 - mm) = 0
-      l = fmaf(s_l[v], wt, l);
-      o = fmaf(s_acc[v][d], wt, o);
+      const float wt = fast_exp2(s_m[v][g] - mm);   // an empty slice: exp2(-3e38 - mm) = 0
+      l = fmaf(s_l[v][g], wt, l);
+      o = fmaf(s_acc[v][g][d], wt, o);
     }
     if (nparts == 1) {
-      a.out[orow + d] = l > 0.0f ? o / l : 0.0f;
+      a.out[orow0 + i] = l > 0.0f ? o / l : 0.0f;
     } else {
-      const int64_t pi = ((int64_t)row * a.H + h) * a.P + p;
+      const int64_t pi = ((int64_t)row * a.H + h0 + g) * a.P + p;
       a.part_acc[pi * D + d] = o;
       if (d == 0) reinterpret_cast<float2*>(a.part_ml)[pi] = make_float2(mm, l);
     }
@@ -263,26 +268,38 @@ static void launch_part(const RowAttnArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((row_attn_part_kernel<T, D, false, G>), grid, block, 0, stream, a);
 }
 
-// Waves of a row_attn_wg_kernel workgroup.  8 and 16 measured the same on C1
-// (6.0 us) and 8 better where a row is longer (fp32, 4096 tokens: 27 against
-// 33 us): twice the workgroups fit a CU, so the last ones wait less.
-constexpr int kWgWaves = 8;
+// Waves of a row_attn_wg_kernel workgroup.  With one head, 8 and 16 measured the
+// same on C1 (6.0 us) and 8 better where a row is longer (fp32, 4096 tokens:
+// 27 against 33 us): twice the workgroups fit a CU, so the last ones wait less.
+// A group of heads walks a short row once for all of them, with 16 (8 at head
+// dim 256, where the walk holds twice the state).
+constexpr int wg_waves(int G, int D) { return G == 1 || D > 128 ? 8 : 16; }
 
-template <typename T, int D>
+template <typename T, int D, int G>
 static void launch_wg(const RowAttnArgs& a, hipStream_t stream) {
-  constexpr int W = kWgWaves;
+  constexpr int W = wg_waves(G, D);
   const int tpl = 64 / (D / Elem<T>::kVec);
-  const dim3 grid((unsigned)sat_mul(a.rows, a.P, a.H)), block(W * 64);   // checked by the caller
+  const dim3 grid((unsigned)sat_mul(a.rows, a.P, a.H / G)), block(W * 64);   // checked by the caller
   if (a.BS % tpl == 0)
-    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, true, W>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, true, G, W>), grid, block, 0, stream, a);
   else
-    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, false, W>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((row_attn_wg_kernel<T, D, false, G, W>), grid, block, 0, stream, a);
+}
+
+// Groups of 4 take a workgroup at head dims 128 and 256 only (decode_common).
+template <typename T, int D>
+static void launch_wg_heads(const RowAttnArgs& a, hipStream_t stream) {
+  if constexpr (D >= 128) {
+    if (a.wg == 4) return launch_wg<T, D, 4>(a, stream);
+  }
+  if (a.wg == 2) return launch_wg<T, D, 2>(a, stream);
+  launch_wg<T, D, 1>(a, stream);
 }
 
 template <typename T, int D>
 static void launch_typed(const RowAttnArgs& a, hipStream_t stream) {
   profile_begin(stream);
-  if (a.wg) launch_wg<T, D>(a, stream);
+  if (a.wg) launch_wg_heads<T, D>(a, stream);
   else switch (row_attn_heads_per_wave(a.H, a.Hkv)) {
     case 8: launch_part<T, D, 8>(a, stream); break;
     case 4: launch_part<T, D, 4>(a, stream); break;
@@ -330,7 +347,7 @@ int launch_row_attn(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStrea
   }
   int64_t gx;
   if (splitmm) gx = splitmm_grid(a);
-  else if (a.wg) gx = sat_mul(a.rows, a.P, a.H);
+  else if (a.wg) gx = sat_mul(a.rows, a.P, a.H / a.wg);
   else gx = sat_mul(a.rows, a.P, ceil_div(a.H / row_attn_heads_per_wave(a.H, a.Hkv), kDecodeWaves));
   if (gx <= 0) return HS_OK;
   if (gx > 0x7fffffffLL)

@@ -23,7 +23,8 @@ struct RowAttnArgs {
   int B, H, Hkv, BS, MB, NB;
   int mode;               // 0 one pass, 1 fixed partitions, 2 num_splits slices,
                           // 4 even split (16-bit caches, up to 4 query heads per KV head)
-  int wg;                 // VALU kernel: a workgroup, not a wave, per (row, head, partition)
+  int wg;                 // VALU kernel: heads of a workgroup per (row, heads, partition);
+                          // 0: waves instead
   int mma;                // grouped heads on the fp32 matrix cores (hs_prefill_rows.hip)
   int ranked;             // with wg: rows dealt longest context first (B <= 64)
   int part_tokens;        // mode 1

@@ -186,3 +186,30 @@ def test_splits_no_further_off_than_their_slices(dtype, H, Hkv, D, batch, n, spl
     limit = 1.1 * ((walk.double() - exact).norm() / exact.norm()).item()
     got = _hip.decode(*(x.to(DEV) for x in case[:5]), scale, num_splits=splits).cpu().double()
     assert ((got - want).norm() / want.norm()).item() <= limit
+
+
+@pytest.mark.parametrize("dtype,H,Hkv,D,BS", [
+    (torch.float32, 4, 2, 64, 16), (torch.bfloat16, 4, 2, 32, 8), (torch.float16, 6, 2, 128, 8),
+    (torch.float32, 8, 2, 128, 16), (torch.bfloat16, 8, 2, 128, 8), (torch.float16, 4, 2, 256, 16),
+    (torch.float32, 8, 2, 256, 16)])
+@pytest.mark.parametrize("batch,longest", [(3, 64), (3, 250), (70, 250), (70, 500), (140, 130),
+                                           (300, 40)])
+def test_grouped_rows_around_the_rules(dtype, H, Hkv, D, BS, batch, longest):
+    """Groups of 2, 3 and 4: few rows and a full device, short rows and longer
+    ones, in the default partitions, in one pass and by splits."""
+    ctxs = [(longest - 7 * i) % longest + (i % 2) for i in range(batch)]
+    ctxs[0] = longest
+    _runs(_case(ctxs, H, Hkv, D, BS, dtype, seed=longest), splits=(0, 1, 5))
+
+
+def test_own_partitions_of_grouped_heads():
+    """Partitions that the caller names, of one tile and of several."""
+    from heteroserve import _hip
+
+    for H, dtype in ((8, torch.float32), (16, torch.bfloat16)):
+        case = _case([0, 1, 15, 16, 17, 100, 300], H, 2, 64, 8, dtype)
+        want = _want(*case)
+        for tokens in (16, 48, 512):
+            got = _hip.decode(*(x.to(DEV) for x in case[:5]), case[5], num_splits=0,
+                              partition_tokens=tokens)
+            assert ((got.cpu().double() - want).norm() / want.norm()).item() <= REL, tokens
