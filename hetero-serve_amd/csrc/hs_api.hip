@@ -219,11 +219,13 @@ static int slices_together(int splits, int64_t parts, int64_t width, int tpl, in
 
 // Multi-head decode in one pass: a workgroup (8 waves) per (row, head) rather
 // than a wave, unless the waves alone fill the device or have little to do.
-// us, a wave / a workgroup per row: 16 sequences of 256..4096 tokens, 12 heads
-// 131 / 32; 64 of up to 8192, 32 heads 724 / 446; 256 of up to 2048, 12 heads
-// 177 / 153; 256 of up to 256 25 / 26.
-static bool wg_per_row(int64_t rows_heads, int64_t width, int cus) {
-  return rows_heads < 4 * (int64_t)cus || (rows_heads < 16 * (int64_t)cus && width > 256);
+// us, a wave / a workgroup per row: 16 sequences of 1024..4096 tokens, 12 heads,
+// fp32 223 / 62; 64 of 128..512 24 / 17, of 16..64 7.0 / 9.6; 32 of 32..128, 16
+// heads, bf16 8.9 / 9.6; 256 of 512..2048, 8 heads, D 32 96 / 120.
+static bool wg_per_row(int64_t rows_heads, int64_t width, int D, int cus) {
+  if (rows_heads <= cus) return true;
+  if (rows_heads <= 2 * (int64_t)cus) return width > 128;
+  return rows_heads <= (D > 32 ? 4 : 3) * (int64_t)cus && width > 256;
 }
 
 // Grouped heads that the split-operand kernel does not take (fp32 caches, other
@@ -533,7 +535,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
       a.part_tokens = rows_partition(B, H, Hkv, D, BS, MB, plan.part_tokens);
       a.P = (int)ceil_div(width, a.part_tokens);
     } else if (num_splits == 1) {
-      a.wg = mha && wg_per_row((int64_t)B * H, width, cus);
+      a.wg = mha && wg_per_row((int64_t)B * H, width, D, cus);
     } else if (num_splits > 1) {
       // Multi-head attention: workgroups of 8 waves, three for each CU, of at
       // least 256 keys, or 512 where that many fill a round of the device (1024

@@ -213,3 +213,15 @@ def test_own_partitions_of_grouped_heads():
             got = _hip.decode(*(x.to(DEV) for x in case[:5]), case[5], num_splits=0,
                               partition_tokens=tokens)
             assert ((got.cpu().double() - want).norm() / want.norm()).item() <= REL, tokens
+
+
+@pytest.mark.parametrize("H,D", [(8, 64), (8, 32)])
+@pytest.mark.parametrize("batch", [32, 33, 65, 97, 129])
+def test_one_pass_around_the_rules(H, D, batch):
+    """Multi-head rows by a workgroup and by a wave: one to four rows a CU, tables
+    on both sides of 128 and 256 tokens."""
+    for longest in (128, 144, 272):
+        ctxs = [longest - (5 * i) % 90 for i in range(batch)]
+        case = _case(ctxs, H, H, D, 16, torch.float16, seed=batch)
+        bt = case[3][:, :-(-longest // 16)].contiguous()
+        _runs((*case[:3], bt, *case[4:]), splits=(1,))
