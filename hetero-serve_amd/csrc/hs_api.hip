@@ -568,7 +568,9 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
       a.slices = slices_together(num_splits, parts, width, tpl, a.mma || a.wg ? 8 : 1);
       a.P = (int)ceil_div(num_splits, a.slices);
     }
-    a.ranked = a.wg && B > 1 && B <= 64 && (int64_t)B * (H / a.wg) > cus;
+    // ranking costs every wave a pass over the batch (2 us at 64 sequences), which
+    // rows of more than 512 tokens give back
+    a.ranked = a.wg && width > 512 && B > 1 && B <= 64 && (int64_t)B * (H / a.wg) > cus;
     const size_t acc = ((size_t)B * H * a.P * D * sizeof(float) + 255) & ~(size_t)255;
     a.part_ml = a.P > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + acc) : nullptr;
     return launch_row_attn(a, kv_dtype, D, cus, st);
