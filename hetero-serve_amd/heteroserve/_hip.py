@@ -97,15 +97,25 @@ def lib_path() -> Path:
 
 
 def open_library(path: Optional[Path] = None) -> ctypes.CDLL:
-    """dlopen libhsattn.so and bind its signatures.  Needs no GPU."""
-    lib = ctypes.CDLL(str(path or lib_path()))
-    for name, (res, args) in {**_SIGNATURES, **_PRIVATE}.items():
-        fn = getattr(lib, name)
+    """dlopen libhsattn.so and bind its signatures.  Needs no GPU.  OSError when the
+    library is of another ABI, or was built without an entry point that this
+    layer calls."""
+    path = path or lib_path()
+    lib = ctypes.CDLL(str(path))
+
+    def bind(name, res, args):
+        fn = getattr(lib, name, None)
+        if fn is None:
+            raise OSError(f"no {name} in {path}: rebuild it")
         fn.restype = res
         fn.argtypes = args
-    got = lib.hs_abi_version()
+        return fn
+
+    got = bind("hs_abi_version", *_SIGNATURES["hs_abi_version"])()
     if got != ABI_VERSION:
         raise OSError(f"libhsattn ABI version {got}, expected {ABI_VERSION}")
+    for name, (res, args) in {**_SIGNATURES, **_PRIVATE}.items():
+        bind(name, res, args)
     return lib
 
 

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -260,3 +261,46 @@ def test_errors_are_per_thread(lib):
         t.join()
     assert len(seen["a"]) == 1 and b"divisible" in next(iter(seen["a"]))
     assert len(seen["b"]) == 1 and b"block_size == 16" in next(iter(seen["b"]))
+
+
+def _stub(tmp_path, abi, names):
+    """A library that exports hs_abi_version and empty functions of these names."""
+    src = tmp_path / "stub.c"
+    src.write_text(f"int hs_abi_version(void) {{ return {abi}; }}\n"
+                   + "".join(f"int {n}(void) {{ return 0; }}\n" for n in names))
+    out = tmp_path / "libstub.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(out), str(src)], check=True)
+    return out
+
+
+@pytest.mark.parametrize("abi,private,reason", [
+    (5, [], "hs_kv_"), (5, ["hs_kv_pack_host_ids", "hs_kv_unpack_host_ids"], "hs_kv_scatter_layers"),
+    (4, [], "ABI version 4"), (None, [], "hs_abi_version")])
+def test_other_libraries_make_the_backend_unavailable(tmp_path, monkeypatch, abi, private, reason):
+    """A library without an entry point that the Python layer calls, or of another
+    ABI, is a reason for the module state, not an exception from it."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from heteroserve import _hip
+
+    if abi is None:
+        (tmp_path / "e.c").write_text("int nothing;")
+        path = tmp_path / "libstub.so"
+        subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(path), str(tmp_path / "e.c")],
+                       check=True)
+    else:
+        path = _stub(tmp_path, abi, [n for n in _hip.EXPORTED_SYMBOLS if n != "hs_abi_version"]
+                     + private)
+    with pytest.raises(OSError, match=reason):
+        _hip.open_library(path)
+    monkeypatch.setenv("HETEROSERVE_HIP_LIB", str(path))
+    monkeypatch.delenv("HETEROSERVE_DISABLE_CUDA_KERNEL", raising=False)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "get_device_properties",
+                        lambda i: SimpleNamespace(gcnArchName="gfx950"))
+    for name, value in (("_state", "unloaded"), ("_error", None), ("_lib", None)):
+        monkeypatch.setattr(_hip, name, value)
+    assert not _hip.ready()
+    assert reason in _hip.error()
