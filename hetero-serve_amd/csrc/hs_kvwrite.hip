@@ -22,6 +22,7 @@
 // for torch's index_put).
 #include "hs_kernels.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace hs {
@@ -29,6 +30,7 @@ namespace hs {
 namespace {
 
 constexpr int kWriteThreads = 256;
+constexpr int kMaxLayers = 32767;   // of one launch: K and V of each are the grid's y index
 
 // ---- element codecs: 8 elements <-> 8 fp32 ------------------------------
 template <typename T>
@@ -275,8 +277,7 @@ int launch_kv_write(const KvWrite& w, const RowMap& map, hipStream_t stream) {
                    row_b % 16 == 0 && (one_head || head_b % 16 == 0) && layer_b % 16 == 0 &&
                    cache_b % 16 == 0 && (row_elems * cb) % 16 == 0;
   const int64_t work = sat_mul(w.n, row_elems);
-  if (row_elems > 0x7fffffffLL || ceil_div(work, kWriteThreads) > 0x7fffffffLL ||
-      w.layers > 32767)
+  if (row_elems > 0x7fffffffLL || ceil_div(work, kWriteThreads) > 0x7fffffffLL)
     return fail(HS_EUNSUPPORTED, "KV write too large for one launch");
   WriteArgs a;
   a.k_cache = static_cast<uint8_t*>(w.k_cache);
@@ -291,13 +292,21 @@ int launch_kv_write(const KvWrite& w, const RowMap& map, hipStream_t stream) {
   a.heads = one_head ? 1 : w.Hkv;
   a.dim = one_head ? (int)row_elems : w.D;
   a.map = map;
-  int rc;
+  int rc = HS_OK;
   profile_begin(stream);
-  switch (w.src_dtype) {
-    case HS_DTYPE_F32: rc = launch_src<float>(w.kv_dtype, a, w.layers, vec, stream); break;
-    case HS_DTYPE_F16: rc = launch_src<_Float16>(w.kv_dtype, a, w.layers, vec, stream); break;
-    case HS_DTYPE_BF16: rc = launch_src<Bf16>(w.kv_dtype, a, w.layers, vec, stream); break;
-    default: rc = fail(HS_EINVAL, "unsupported source dtype code " + std::to_string(w.src_dtype));
+  for (int left = w.layers; left > 0 && rc == HS_OK; left -= kMaxLayers) {
+    const int layers = std::min(left, kMaxLayers);
+    switch (w.src_dtype) {
+      case HS_DTYPE_F32: rc = launch_src<float>(w.kv_dtype, a, layers, vec, stream); break;
+      case HS_DTYPE_F16: rc = launch_src<_Float16>(w.kv_dtype, a, layers, vec, stream); break;
+      case HS_DTYPE_BF16: rc = launch_src<Bf16>(w.kv_dtype, a, layers, vec, stream); break;
+      default: rc = fail(HS_EINVAL, "unsupported source dtype code " + std::to_string(w.src_dtype));
+    }
+    if (left <= kMaxLayers) break;   // (the products below fit where those layers exist)
+    a.k_cache += kMaxLayers * cache_b;
+    a.v_cache += kMaxLayers * cache_b;
+    a.k_src += kMaxLayers * layer_b;
+    a.v_src += kMaxLayers * layer_b;
   }
   profile_end(stream);
   if (rc != HS_OK) return rc;

@@ -559,6 +559,8 @@ def kv_scatter_layers(pool, slots, k, v) -> None:
     negative slots count from the end."""
     lib_ = lib("KV scatter HIP kernel")
     L, _, NB, BS, Hkv, D = pool.shape
+    if L == 0:
+        return
     (_, _, _, _), index = _check_write(pool[0, 0], pool[0, 1], k, v)
     T = slots.numel()
     for x in (k, v):

@@ -125,3 +125,15 @@ def test_device_slots_wrap_and_skip(n):
     want[48 - n:] = rows[:n].cpu().to(torch.bfloat16)
     assert torch.equal(gk.view(48, 2, 32).cpu(), want)
     assert torch.equal(gv.view(48, 2, 32).cpu(), -want)
+
+
+@pytest.mark.parametrize("L", [0, 32767, 32768, 65536])
+def test_any_number_of_layers(L):
+    """No layers, and one more than a launch's grid holds (strided K, one head)."""
+    from heteroserve.kv import pack
+
+    pool = torch.zeros(L, 2, 2, 1, 1, 8, dtype=torch.float16, device=DEV)
+    k = torch.arange(L * 16, device=DEV).remainder(2039).to(torch.float16).view(L, 1, 1, 16)
+    pack.write_kv(pool, [1], 0, k[..., :8], k[..., 8:])
+    assert torch.equal(pool[:, 0, 1, 0], k[:, 0, :, :8]) and not pool[:, :, 0].any()
+    assert torch.equal(pool[:, 1, 1, 0], k[:, 0, :, 8:])
