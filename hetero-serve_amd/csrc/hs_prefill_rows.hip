@@ -13,10 +13,11 @@
 // What bounds it.  The products run on v_mfma_f32_16x16x4_f32 (64 FLOPs a
 // cycle and SIMD, 157 TFLOP/s over the device at 2.4 GHz), whose 32 cycles
 // each leave room for everything else: the softmax, the LDS reads and the
-// loads of a 16-key tile take a fraction of its products' time.  The row
-// kernel that this one replaced gave every (query, head) a wave of its own,
-// which read all the keys of its row again and reduced every score over 16
-// lanes.
+// loads of a 16-key tile take a fraction of its products' time.  The VALU
+// kernel (hs_decode.hip) gives every row and up to 8 of its heads a wave of their
+// own, which reads all the keys of its row again and reduces every score over
+// the lanes; it keeps the short tables (rows_prefill_pays) and some decodes
+// (grouped_on_matrix_cores in hs_api.hip).
 //
 // Work decomposition.  A workgroup owns 16 * NT rows of one (sequence, KV
 // head), a row being a (query, head of the group) pair with the queries
@@ -559,14 +560,15 @@ bool rows_prefill_pays(const RowAttnArgs& a, int kv_dtype, int D, int cus) {
   const int G = a.H / a.Hkv;
   const int64_t rows = (int64_t)a.S * G;
   int keys;   // up to here the VALU kernel
-  if (sat_mul(ceil_div(rows, kKeys), a.B, a.Hkv) < 2 * (int64_t)cus) {
-    keys = D == 256 ? (half ? 64 : 32) : G == 1 ? 32 : 16;
+  const int64_t wgs = sat_mul(ceil_div(rows, kKeys), a.B, a.Hkv);
+  if (wgs < 2 * (int64_t)cus) {
+    keys = D == 256 ? (half ? 64 : 32) : G < 4 || wgs >= cus ? 32 : 16;
   } else if (G == 1) {
     keys = 640 / (int)std::min<int64_t>(rows, kKeys);
-    if (D >= 128 && half) keys *= 2;
+    if (D >= 128 && half) keys *= rows <= 4 ? 4 : 2;
     if (D == 32) keys /= 2;
   } else {
-    keys = G > 4 ? (half ? 40 : 32) : D >= 128 && half ? 112 : 64;
+    keys = G > 4 ? (half ? 48 : 32) : D >= 128 ? (half ? 112 : 86) : 64;
     if (a.cu_q) keys = keys * 3 / 2;
   }
   return (int64_t)a.MB * a.BS > keys;
@@ -579,7 +581,7 @@ int launch_rows(const RowAttnArgs& a, int kv_dtype, int D, int cus, hipStream_t 
   else if (kv_dtype == HS_DTYPE_F16) launch_t<_Float16>(a, D, rows_per_pair, cus, stream);
   else launch_t<Bf16>(a, D, rows_per_pair, cus, stream);
   profile_end(stream);
-  return check_launch("paged prefill");
+  return check_launch(a.mma ? "paged attention" : "paged prefill");
 }
 
 }  // namespace hs
