@@ -149,20 +149,37 @@ static int default_partition(int B, int H, int Hkv, int BS, int MB, int kv_dtype
                                sat_mul(B, Hkv, G / row_attn_heads_per_wave(H, Hkv)), BS, MB);
 }
 
+// Parts of rows of `width` keys for `units` workgroups a part that mostly have a
+// CU for themselves: the number (of up to `most`) whose rounds over the device
+// take the least, a part costing its keys and a set-up worth 64 keys.
+static int64_t parts_by_rounds(int64_t units, int64_t width, int64_t most, int cus) {
+  int64_t best = 1, best_cost = INT64_MAX;
+  for (int64_t p = 1; p <= most; ++p) {
+    const int64_t cost = ceil_div(units * p, cus) * (ceil_div(width, p) + 64);
+    if (cost < best_cost) {
+      best = p;
+      best_cost = cost;
+    }
+    if (units * p >= 4 * (int64_t)cus) break;
+  }
+  return best;
+}
+
 // Grouped heads on the fp32 matrix cores: workgroups of 8 waves take 16-key
-// tiles in turn, so a partition is 2048 keys, cut down to 128 (a tile a wave)
-// while the launch has fewer workgroups than CUs; never shorter than the
-// partition that the workspace was sized for.  16 sequences of 256..4096
-// tokens, us from 1024 keys and two workgroups a CU / from 2048 and one: 32 / 8
-// heads, D 128, fp32 72 / 60; 16 / 1, fp32 24 / 18; 32 / 4, bf16, 32-token
-// blocks 37 / 33.  A row that the waves finish in a few tiles each is one partition,
-// without a merge: 256 keys at head dim 128 (8 to 32 sequences of 64..256 tokens,
-// 32 / 8 heads, fp32: 14.3 / 12.4; at 512 keys 17 against 15).
+// tiles in turn, so a partition is a multiple of 128 keys (a tile a wave), at most
+// 2048, and never shorter than the partition that the workspace was sized for.
+// 32 / 8 heads, D 128, fp32, 24 sequences of 512 tokens in 2 parts (384
+// workgroups) / 1: 34 / 22 us.  A row that the waves finish in a few tiles each is
+// one partition, without a merge: 256 keys at head dim 128 (8 to 32 sequences of
+// 64..256 tokens, 32 / 8 heads, fp32: 14.3 / 12.4; at 512 keys 17 against 15).
 constexpr int kOnePassElems = 256 * 128;
-static int rows_partition(int B, int H, int Hkv, int D, int BS, int MB, int default_pt) {
+static int rows_partition(int B, int H, int Hkv, int D, int BS, int MB, int default_pt, int cus) {
   const int one_pass = kOnePassElems / D;
-  if ((int64_t)MB * BS <= one_pass) return std::max(default_pt, one_pass);
-  const int pt = shrink_for_small_grid(2048, 128, sat_mul(B, Hkv, ceil_div(H / Hkv, 16)), BS, MB, 1);
+  const int64_t width = (int64_t)MB * BS;
+  if (width <= one_pass) return std::max(default_pt, one_pass);
+  const int64_t parts = parts_by_rounds(sat_mul(B, Hkv, ceil_div(H / Hkv, 16)), width,
+                                        ceil_div(width, 128), cus);
+  const int pt = (int)std::min((int64_t)2048, ceil_div(ceil_div(width, parts), 128) * 128);
   return std::max(pt, default_pt);
 }
 
@@ -181,13 +198,15 @@ constexpr int64_t kWgSplitMaxTokens = 1024;
 // Query heads of such a workgroup, or 0 for another kernel.  Multi-head attention
 // has one.  A group of 2 or 4 walks its keys once for all its heads, but where that
 // leaves CUs idle at head dim 256 each head its own; larger groups go to the
-// fp32 matrix cores, and groups of 4 where that measured faster (head dims to 64;
-// rows past 256 tokens; 16-bit rows of up to 64).  us, a head / the group / the fp32
-// matrix cores: 8 / 4 heads, D 256, bf16, 64 sequences of 64..256 tokens 23 / 14 / -,
-// 32 of 128..512 20 / 22 / -; 16 / 8 heads, D 64, fp32, 4 of 64..256 - / 7.5 / 10.4;
+// fp32 matrix cores, and groups of 4 where that measured faster (rows of up to 256
+// tokens at head dims to 64, and of more where their workgroups leave half the
+// CUs free or fill them; 16-bit rows of up to 64).  us, a head / the group / the
+// fp32 matrix cores: 8 / 4 heads, D 256, bf16, 64 sequences of 64..256 tokens 23 / 14
+// / -, 32 of 128..512 20 / 22 / -; 16 / 8 heads, D 64, fp32, 4 of 64..256 - / 7.5 / 10.4;
 // 32 / 8 heads, D 128, 8-token blocks, bf16, 32 of 64..256 - / 12.2 / 15, 32 of
 // 128..512 - / 16.7 / 23, 8 of 128..512 - / 16 / 14, 32 of 16..64 - / 9.6 / 8; fp32, 64 of
-// 16..64 - / 13.3 / 16.
+// 16..64 - / 13.3 / 16, 20 of 512 - / 25 / 32, 16 of 128..512 - / 23 / 19; D 64, 24 of
+// 1024, fp16 - / 22 / 30.
 static int short_rows_heads(int B, int H, int Hkv, int D, int kv_dtype, int64_t width, int cus) {
   const int G = H / Hkv, Gw = row_attn_heads_per_wave(H, Hkv);
   const bool half = kv_dtype != HS_DTYPE_F32;
@@ -197,8 +216,10 @@ static int short_rows_heads(int B, int H, int Hkv, int D, int kv_dtype, int64_t 
     return width <= (half ? 512 : 256) ? 1 : 0;
   }
   if (G < 4) return Gw;
-  if (D < 128 || (half && width <= 64)) return 0;
-  return width <= 256 || (half && width <= 512 && sat_mul(B, Hkv) >= cus / 2) ? Gw : 0;
+  if (half && width <= 64) return 0;
+  // more than half a round of the matrix cores' workgroups, less than one
+  if (width > (D < 128 ? 512 : 256) && 2 * sat_mul(B, Hkv) >= cus + (half ? 0 : 1)) return Gw;
+  return D == 128 && width <= 256 ? Gw : 0;
 }
 
 // Decode by explicit splits: the slices that are taken together.  Neighbouring
@@ -212,7 +233,7 @@ static int short_rows_heads(int B, int H, int Hkv, int D, int kv_dtype, int64_t 
 static int slices_together(int splits, int64_t parts, int64_t width, int tpl, int waves) {
   const int64_t slice = ceil_div(ceil_div(width, splits), tpl);   // steps of one slice
   for (int64_t p = std::max((int64_t)1, std::min(parts, (int64_t)splits));; ++p) {
-    const int64_t s = ceil_div(splits, p);
+    const int64_t s = waves == 1 ? std::max((int64_t)1, splits / p) : ceil_div(splits, p);
     if (s <= waves || ceil_div(s * slice, waves) + waves <= slice + splits) return (int)s;
   }
 }
@@ -260,15 +281,15 @@ static bool grouped_on_matrix_cores(int B, int H, int Hkv, int D, int kv_dtype, 
   }
   if (num_splits == 1 || G == 3) {
     const int64_t wgs = D == 256 && !f32 ? 2 * pairs : pairs;
-    if (wgs < 2 * (int64_t)cus) return true;
-    if (wgs == 2 * (int64_t)cus) return G == 4 || D == 256 || width > 256;
+    if (wgs <= cus) return true;
+    if (wgs <= 2 * (int64_t)cus) return G == 4 || D == 256 || width > (f32 ? 64 : 256);
     if (wgs <= 4 * (int64_t)cus) return width > 256 && (f32 || G > 2 || D == 256);
     return width > 512 && (f32 || G == 3 || (G == 4 && D <= 64));
   }
   if (short_rows && D <= 128) return true;
   if (!f32 || pairs >= cus) return false;
-  if (D == 256) return short_rows || pairs < 16 || 4 * pairs >= cus;
-  return (G == 4 || 4 * pairs >= cus) && !long_keys;
+  if (D == 256 && (short_rows || pairs < 16)) return true;
+  return G == 4 && (D <= 128 || 4 * pairs >= cus) && !long_keys;
 }
 
 // The workspace queries take no kv dtype: they size for the shortest default
@@ -532,7 +553,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
       a.mode = 0;
       a.P = 1;
     } else if (num_splits == 0 && a.mma) {
-      a.part_tokens = rows_partition(B, H, Hkv, D, BS, MB, plan.part_tokens);
+      a.part_tokens = rows_partition(B, H, Hkv, D, BS, MB, plan.part_tokens, cus);
       a.P = (int)ceil_div(width, a.part_tokens);
     } else if (num_splits == 1) {
       a.wg = mha && wg_per_row((int64_t)B * H, width, D, cus);
@@ -550,14 +571,14 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
       const int64_t units = a.mma ? sat_mul(B, Hkv, ceil_div(H / Hkv, 16))
                                   : sat_mul(B, H / row_attn_heads_per_wave(H, Hkv));
       const int tpl = a.mma ? 16 : row_attn_tokens_per_load(kv_dtype, D);
-      a.wg = mha && sat_mul(units, num_splits) < 64 * (int64_t)cus &&
-             (units <= 2 * (int64_t)cus || width > 128) &&
+      a.wg = mha && sat_mul(units, num_splits) < (D == 32 ? 33 : 64) * (int64_t)cus &&
+             (units <= 2 * (int64_t)cus || width > 128) && (D > 32 || width <= 2048) &&
              (sat_mul(units, num_splits) < 8 * (int64_t)cus || width < 256 * (int64_t)num_splits);
-      int64_t parts = ceil_div((a.mma ? 2 : a.wg ? 3 : 16) * (int64_t)cus, units);
+      int64_t parts = ceil_div((a.wg ? 3 : D == 32 ? 32 : 16) * (int64_t)cus, units);
       if (a.mma) {
-        parts = std::min(parts, ceil_div(width, 256));
+        parts = parts_by_rounds(units, width, ceil_div(width, 256), cus);
       } else if (a.wg) {
-        int64_t cap = ceil_div(width, units >= cus ? 1024 : 512);
+        int64_t cap = ceil_div(width, units >= 2 * (int64_t)cus ? 1024 : 512);
         if (units < cus && width > 512 && (units * cap > cus || 2 * units * cap < cus))
           cap = ceil_div(width, 256);
         if (units < 2 * (int64_t)cus) parts = std::max(parts, ceil_div(width, 1024));

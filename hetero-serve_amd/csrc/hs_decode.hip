@@ -286,12 +286,9 @@ static void launch_wg(const RowAttnArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL((row_attn_wg_kernel<T, D, false, G, W>), grid, block, 0, stream, a);
 }
 
-// Groups of 4 take a workgroup at head dims 128 and 256 only (decode_common).
 template <typename T, int D>
 static void launch_wg_heads(const RowAttnArgs& a, hipStream_t stream) {
-  if constexpr (D >= 128) {
-    if (a.wg == 4) return launch_wg<T, D, 4>(a, stream);
-  }
+  if (a.wg == 4) return launch_wg<T, D, 4>(a, stream);
   if (a.wg == 2) return launch_wg<T, D, 2>(a, stream);
   launch_wg<T, D, 1>(a, stream);
 }
