@@ -1042,51 +1042,61 @@ static const void* even_valu_kernel(int kv_dtype, int D) {
   return kv_dtype == HS_DTYPE_F16 ? even_valu_kernel_t<_Float16>(D) : even_valu_kernel_t<Bf16>(D);
 }
 
-// Resident workgroups of the kernel per CU and the CU count, on the current
-// device; looked up once per (device, kernel).
-static void even_occupancy(const void* fn, int block, int* occ, int* cus) {
+// Resident workgroups of the kernel per CU, waves that its registers leave room
+// for per SIMD, and the CU count, on the current device; looked up once per
+// (device, kernel).
+struct EvenOccupancy {
+  int groups = 0, waves = 0, cus = 0;
+};
+
+static EvenOccupancy even_occupancy(const void* fn, int block) {
   static std::mutex mu;
-  static std::map<std::pair<int, const void*>, std::pair<int, int>> cache;
+  static std::map<std::pair<int, const void*>, EvenOccupancy> cache;
   int dev = 0;
-  *occ = 0;
-  *cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return;
+  if (hipGetDevice(&dev) != hipSuccess) return {};
   std::lock_guard<std::mutex> lock(mu);
   auto it = cache.find({dev, fn});
   if (it == cache.end()) {
-    int n = 0, c = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, block, 0) != hipSuccess) n = 0;
-    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) c = 0;
-    it = cache.emplace(std::make_pair(dev, fn), std::make_pair(n, c)).first;
+    EvenOccupancy o;
+    hipFuncAttributes attr;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&o.groups, fn, block, 0) != hipSuccess)
+      o.groups = 0;
+    if (hipDeviceGetAttribute(&o.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      o.cus = 0;
+    if (hipFuncGetAttributes(&attr, fn) == hipSuccess && attr.numRegs > 0)
+      o.waves = (int)std::min<int64_t>(8, 512 / (8 * ceil_div(attr.numRegs, 8)));
+    it = cache.emplace(std::make_pair(dev, fn), o).first;
   }
-  *occ = it->second.first;
-  *cus = it->second.second;
+  return it->second;
 }
 
 // M, the workgroups per unit: the device's resident workgroups (kEvenRounds
 // times over) split between the units.  0 when the even split does not
 // serve the call: more than kEvenMaxGroup query heads per KV head, or fixed
-// default partitions that fit one round (B rows of the table's width, a
-// bound on the real count, at most M partitions per unit).
+// default partitions that fit one round of the device (B rows of the table's
+// width are a bound on the real count).  A round of grouped heads' partitions, 4
+// waves each, is a wave for every SIMD; in 8-wave workgroups fewer waves fit, and
+// taken by those 160 sequences of up to 64 tokens, 32 / 8 heads, D 64, fp16 went to
+// the even split, 9 -> 24 us.
 int splitmm_even_groups(int kv_dtype, int D, int H, int Hkv, int B, int MB) {
   const int G = H / Hkv;
-  int occ = 0, cus = 0;
+  EvenOccupancy o;
   int64_t groups, part;   // workgroups sharing a range; the fixed plan's partition
   if (even_valu_serves(kv_dtype, D, H, Hkv)) {
-    even_occupancy(even_valu_kernel(kv_dtype, D), 64 * kEvenValuWaves, &occ, &cus);
+    o = even_occupancy(even_valu_kernel(kv_dtype, D), 64 * kEvenValuWaves);
     groups = ceil_div(H, kEvenValuWaves);
     part = kValuFixedPartition;
   } else if (splitmm_serves(kv_dtype, kPage, D, H, Hkv) && G <= kEvenMaxGroup) {
-    even_occupancy(even_kernel(kv_dtype, D), 64 * kEvenWaves, &occ, &cus);
+    o = even_occupancy(even_kernel(kv_dtype, D), 64 * kEvenWaves);
     groups = Hkv / splitmm_even_heads(H, Hkv);
     part = splitmm_default_partition(G, D);
   } else {
     return 0;
   }
-  if (occ <= 0 || cus <= 0) return 0;
-  const int64_t fill = ceil_div((int64_t)cus * occ * kEvenRounds, groups);
+  if (o.groups <= 0 || o.cus <= 0) return 0;
+  const int64_t fill = ceil_div((int64_t)o.cus * o.groups * kEvenRounds, groups);
   const int64_t parts = sat_mul(B, ceil_div((int64_t)MB * kPage, part));
-  const int64_t one = H == Hkv ? fill : ceil_div((int64_t)cus * occ * (kEvenWaves / 4), Hkv);
+  const int64_t one = H == Hkv ? fill : ceil_div((int64_t)o.cus * o.waves, Hkv);
   if (parts <= one) return 0;
   return (int)std::min<int64_t>(fill, 1 << 20);
 }
