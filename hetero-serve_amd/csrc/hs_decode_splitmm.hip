@@ -175,13 +175,6 @@ __device__ inline float sum_across_groups(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Orders a wave's LDS accesses for the compiler (the hardware keeps them in
-// order).
-__device__ inline void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 template <int D>
 struct PageWalk {
   static constexpr int kDC = D / 8;           // 16-byte chunks per head row
@@ -661,9 +654,7 @@ __device__ inline bool even_range(const RowAttnArgs& a, int wr, int64_t& s, int6
 
 // The state of one segment of one KV head, from the nph waves of a workgroup
 // that walked it (waves hsub, hsub + hw, ...): write_unit_state's combine and
-// layout, for hw KV heads side by side.  With one wave per head there is
-// nothing to combine and no barrier; otherwise every wave of the workgroup
-// calls it.
+// layout, for hw KV heads side by side.  Every wave of the workgroup calls it.
 template <int D, int kW>
 __device__ inline void write_head_state(float4x (&o)[D / 16], float m, float l, int gc, int hsub,
                                         int ph, int hw, int nph, bool single, float* out_rows,
@@ -678,21 +669,17 @@ __device__ inline void write_head_state(float4x (&o)[D / 16], float m, float l, 
   for (int d = 0; d < D / 16; ++d)   // head j < 8: hi column j plus lo column j + 8
 #pragma unroll
     for (int i = 0; i < 4; ++i) o[d][i] += dpp<kDppRowRor8>(o[d][i]);
-  float sc = 1.0f;
-  if (nph > 1) {
-    if (g == 0) {
-      wave_m[wv][j] = m;
-      wave_l[wv][j] = lsum;
-    }
-    __syncthreads();
-    float mm = m;
-    for (int p = 0; p < nph; ++p) mm = fmaxf(mm, wave_m[hsub + hw * p][j]);
-    lsum = 0.0f;
-    for (int p = 0; p < nph; ++p)
-      lsum += wave_l[hsub + hw * p][j] * fast_exp2(wave_m[hsub + hw * p][j] - mm);
-    sc = fast_exp2(m - mm);
-    m = mm;
+  if (g == 0) {
+    wave_m[wv][j] = m;
+    wave_l[wv][j] = lsum;
   }
+  __syncthreads();
+  float mm = m;
+  for (int p = 0; p < nph; ++p) mm = fmaxf(mm, wave_m[hsub + hw * p][j]);
+  lsum = 0.0f;
+  for (int p = 0; p < nph; ++p)
+    lsum += wave_l[hsub + hw * p][j] * fast_exp2(wave_m[hsub + hw * p][j] - mm);
+  float sc = fast_exp2(m - mm);
   constexpr int kSt = D + 4;                          // floats per staged row
   if (single) sc *= lsum > 0.0f ? 1.0f / lsum : 0.0f;
   float* st = reinterpret_cast<float*>(&lds[wv]);
@@ -701,9 +688,8 @@ __device__ inline void write_head_state(float4x (&o)[D / 16], float m, float l, 
     *reinterpret_cast<float4*>(&st[j * kSt + 16 * d + 4 * g]) =
         make_float4(o[d][0] * sc, o[d][1] * sc, o[d][2] * sc, o[d][3] * sc);
   if (!single && ph == 0 && g == 0 && j < gc)
-    *reinterpret_cast<float2*>(ml + 2 * j) = make_float2(m, lsum);
-  if (nph > 1) __syncthreads();
-  else wave_lds_fence();
+    *reinterpret_cast<float2*>(ml + 2 * j) = make_float2(mm, lsum);
+  __syncthreads();
   constexpr int kLr = D / 4;                          // lanes per head row
   constexpr int kHp = 64 / kLr;                       // head rows per wave and pass
   const int c4 = lane % kLr;
@@ -720,8 +706,7 @@ __device__ inline void write_head_state(float4x (&o)[D / 16], float m, float l, 
       *reinterpret_cast<float4*>(dst + (int64_t)hh * D) = x;
     }
   }
-  if (nph > 1) __syncthreads();   // staging read by every wave before the buffers are reused
-  else wave_lds_fence();
+  __syncthreads();   // staging read by every wave before the buffers are reused
 }
 
 // A workgroup's kW waves are hw neighbouring KV heads times nph page phases, so
@@ -1000,7 +985,7 @@ constexpr int kEvenWaves = 8;
 constexpr int kEvenHeads = 2;
 // Workgroups of the device's occupancy per CU taken by the grid: filled once
 // (C2-gqa: 109 us; twice 114, three times 116), and the least pages of a
-// range (16: 4 a wave; 32 measured the same on C2-gqa).
+// range (16: 4 a wave, 2 with an odd number of KV heads; 32 measured the same on C2-gqa).
 constexpr int kEvenRounds = 1;
 constexpr int kEvenMinPages = 16;
 
