@@ -74,11 +74,11 @@ LEG_KERNELS = {
     "C2": ("hs::row_attn_even_kernel<hs::Bf16, 128>", None, "C2 alone"),
     "C3": ("hs::row_attn_even_kernel<hs::Bf16, 128>", None, "C3 alone"),
     "B64-4k": ("hs::row_attn_even_kernel<hs::Bf16, 128>", None, "B64-4k alone"),
-    "C1": ("hs::row_attn_wg_kernel<_Float16, 64, true, 1, 16>", None, "every leg"),
-    "C2-gqa": ("hs::splitmm_even_kernel<hs::Bf16Ops, 128, true, 4>", None, "every leg"),
+    "C1": ("hs::row_attn_wg_kernel<_Float16, 64, true, 1, 8>", None, "every leg"),
+    "C2-gqa": ("hs::splitmm_even_kernel<hs::Bf16Ops, 128, 8>", None, "every leg"),
     "C4": ("hs::prefill_stream_kernel<hs::Bf16, 128>", None, "every leg"),
-    "C5_pack": ("hs::page_copy_kernel<false, true>", None, "every leg"),
-    "C5_unpack": ("hs::page_copy_kernel<true, true>", None, "every leg"),
+    "C5_pack": ("hs::page_copy_kernel<false, true, true, hs::IdsInMemory>", None, "every leg"),
+    "C5_unpack": ("hs::page_copy_kernel<true, true, true, hs::IdsInMemory>", None, "every leg"),
 }
 
 
@@ -279,7 +279,7 @@ def migration_legs(steps: int, warmup: int, with_cpu: bool) -> dict:
     res = {"pack": {"us_per_step": round(pk_step * 1e3, 2),
                     "gbs": round(nbytes / (pk_kernel * 1e-3) / 1e9, 1),
                     "bytes_moved": nbytes,
-                    "roofline": roofline("hbm", "page_copy_kernel<false, true>", nbytes, pk_kernel,
+                    "roofline": roofline("hbm", "page_copy_kernel<false, true, true, IdsInMemory>", nbytes, pk_kernel,
                                          leg_traffic("C5_pack"))}}
     log(f"C5 pack: {pk_kernel * 1e3:.1f} us, {res['pack']['gbs']:.0f} GB/s")
 
@@ -301,7 +301,7 @@ def migration_legs(steps: int, warmup: int, with_cpu: bool) -> dict:
                      "bytes_moved": nbytes, "bit_exact": up_exact,
                      "check": "torch GPU indexing of the unpacked pool == payload; "
                               "every other block untouched",
-                     "roofline": roofline("hbm", "page_copy_kernel<true, true>", nbytes, up_kernel,
+                     "roofline": roofline("hbm", "page_copy_kernel<true, true, true, IdsInMemory>", nbytes, up_kernel,
                                           leg_traffic("C5_unpack"))}
     log(f"C5 unpack: {up_kernel * 1e3:.1f} us, {res['unpack']['gbs']:.0f} GB/s, exact={up_exact}")
 
@@ -855,8 +855,8 @@ def gqa_one_partition_leg(iters: int = 20) -> dict:
     The library default (fixed partitions here: one round of the device
     holds them, so the even split does not apply) against explicit 768-token
     partitions, one a row, on the split-operand matrix-core kernel, and v2
-    (one pass), which runs the VALU kernel.  Each checked against the
-    oracle, then timed."""
+    (one pass), on the fp32 matrix cores.  Each checked against the oracle,
+    then timed."""
     import numpy as np
     import torch
 
@@ -877,7 +877,7 @@ def gqa_one_partition_leg(iters: int = 20) -> dict:
                lambda: paged_attn.paged_attention(*args), want, nbytes, iters),
            "768-token partitions (matrix cores, one a row)": _entry_row(
                lambda: _hip.decode(*args, 0, partition_tokens=768), want, nbytes, iters),
-           "v2 one pass (VALU)": _entry_row(
+           "v2 one pass (fp32 matrix cores)": _entry_row(
                lambda: paged_attn_v2.paged_attention_v2(*args), want, nbytes, iters)}
     log("GQA one-partition rows: " + ", ".join(
         f"{k.split(' (')[0]} {v['device_us_per_call']:.1f} us" for k, v in res.items()))
@@ -1132,10 +1132,10 @@ def main() -> int:
     if not args.no_secondary and with_cpu and args.config == "C2":
         secondary["C2_entry_points"] = c2_entries
     if not args.no_secondary:
-        legs = [("C1", "row_attn_wg_kernel<_Float16, 64, true, 1, 16>", True, 0),
-                ("C2-gqa", "splitmm_even_kernel<Bf16Ops, 128, true, 4>", False, 16),
-                ("C3", "row_attn_part_kernel<Bf16, 128, true, 1>", False, 4),
-                ("B64-4k", "row_attn_part_kernel<Bf16, 128, true, 1>", False, 8)]
+        legs = [("C1", "row_attn_wg_kernel<_Float16, 64, true, 1, 8>", True, 0),
+                ("C2-gqa", "splitmm_even_kernel<Bf16Ops, 128, 8>", False, 16),
+                ("C3", "row_attn_even_kernel<Bf16, 128>", False, 4),
+                ("B64-4k", "row_attn_even_kernel<Bf16, 128>", False, 8)]
         for name, kernel, batched, n_seq in legs:
             if name == headline_name:
                 continue
