@@ -16,7 +16,7 @@
 // its SIMD issues MFMAs, which measured faster than 64 rows per wave at one
 // wave per SIMD, even though each LDS fragment then feeds one MFMA instead of
 // two.  A grid too small for the CUs (one chunk of one sequence) splits each
-// query tile's keys over up to 4 workgroups whose partial softmax states
+// query tile's keys over up to 16 workgroups whose partial softmax states
 // prefill_merge_kernel combines.
 // Scores are computed transposed, S^T = K . Q^T, with v_mfma_f32_32x32x16_f16:
 // K rows are the A operand (read from LDS), Q^T the B operand (held in
@@ -2097,8 +2097,9 @@ int launch_dim(const PrefillArgs& a, int D, bool wide, int max_rows_per_seq, int
 // Launch shape of the MFMA prefill for B sequences of up to max_rows query
 // rows on a device with `cus` CUs.  Full-width workgroups (256 rows; 128 at
 // head dim 32) when their query tiles cover every CU.  Otherwise, with a
-// workspace, each tile's key range is split over floor(cus / tiles) <= 16
-// workgroups (a 1024-row chunk of 32 heads: 128 tiles, 2 parts); at up to 4
+// workspace, each tile's key range is split over floor(cus / tiles) <= 4
+// workgroups (a 1024-row chunk of 32 heads: 128 tiles, 2 parts), or over up to 16
+// while the XCD with the most heads has a CU for each: with 4
 // parts a short chunk on a long prefix still walked 17 tiles a workgroup beside
 // idle CUs.  One sequence, prefix 4096, us a call at up to 4 / 16 parts: 16 rows
 // 32 / 8 heads 27.4 / 22.8, 12 heads D 64 21.2 / 17.6, 8 heads D 32 22.2 / 16.4;

@@ -9,8 +9,8 @@ build_error :258, paged_attention_prefill :263-278).
                     (padding) are zero
     ->              [B, S, H, D] float32
 
-Runs libhsattn's fp32 prefill (tiles of query rows on the fp32 matrix cores,
-any KV dtype and block size).  Difference from the reference: no torch
+Runs libhsattn's fp32 prefill (tiles of query rows on the fp32 matrix cores, or
+a wave per row where the table is short; any KV dtype and block size).  Difference from the reference: no torch
 fallback -- RuntimeError when the library is unavailable.  The binding that
 goes into the reference tree keeps the reference's torch branch
 (``paged_attention_prefill_torch``) for hosts without the library, which the

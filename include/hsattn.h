@@ -124,16 +124,19 @@ size_t hs_decode_workspace_bytes(int B, int H, int Hkv, int D, int BS, int MB, i
  *                     plus the merge (the fast default; with
  *                     partition_tokens == 0, a small grid of rows of at most
  *                     1024 keys by the table's width instead runs one
- *                     workgroup per (sequence, head group) whose waves split
- *                     the keys and merge in LDS: no merge launch, the
- *                     workspace unused)
+ *                     workgroup per (sequence, head), or per group of 2 to 4
+ *                     heads, whose waves split the keys and merge in LDS: no
+ *                     merge launch, the workspace unused.  Larger groups, and
+ *                     some rows of groups of 3 and 4, keep partitions there)
  *   partition_tokens  used when num_splits == 0; 0 = library default (512
  *                tokens, fewer for GQA groups and for grids of fewer than 4
  *                waves per CU; fp16 and bf16 caches with 2 or more query
  *                heads per KV head, head dim 64 and 128: 768 tokens up to 4
  *                heads per KV head, 384 up to 8, 256 otherwise and at head
  *                dim 32, cut for grids of fewer than 8 waves per CU up to 4
- *                heads per KV head, 4 above).  A row that one partition
+ *                heads per KV head, 4 above; grouped heads on the fp32 matrix
+ *                cores 2048 tokens, down to 128 on small grids, and never
+ *                more partitions than the workspace query counted).  A row that one partition
  *                covers is written directly, without the merge.
  *                Must be a multiple of 16.
  *                With num_splits == 0 and partition_tokens == 0, fp16 and
@@ -230,8 +233,8 @@ size_t hs_prefill_workspace_bytes(int B, int max_seqlen_q, int H, int D, int use
  * Replaces:
  *   use_mfma = 0: paged_attention_prefill,
  *                 heteroserve/model/paged_attn_prefill.py:159-214
- *                 (fp32 arithmetic on the fp32 matrix cores, any KV dtype and
- *                 block size, D in {32,64,128,256})
+ *                 (fp32 arithmetic, on the fp32 matrix cores but for short
+ *                 tables, any KV dtype and block size, D in {32,64,128,256})
  *   use_mfma = 1: paged_attention_prefill_wmma,
  *                 heteroserve/model/paged_attn_wmma.py:256-318
  *                 (fp16 matrix-core operands with fp32 accumulation; KV dtype

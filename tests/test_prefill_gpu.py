@@ -271,7 +271,7 @@ def test_mfma_dispatch_orders(n_seq, H, Hkv):
 ])
 def test_mfma_key_split(prefix, chunk, H, Hkv, D):
     """Grids too small to cover the CUs split each query tile's key range
-    over up to 4 workgroups and merge their partial softmax states; without
+    over several workgroups and merge their partial softmax states; without
     a workspace the same call runs 128-row workgroups instead.  Both against
     the per-sequence oracle, 2e-3."""
     from heteroserve import _hip
