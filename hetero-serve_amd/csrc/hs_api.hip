@@ -242,11 +242,14 @@ static int slices_together(int splits, int64_t parts, int64_t width, int tpl, in
 // than a wave, unless the waves alone fill the device or have little to do.
 // us, a wave / a workgroup per row: 16 sequences of 1024..4096 tokens, 12 heads,
 // fp32 223 / 62; 64 of 128..512 24 / 17, of 16..64 7.0 / 9.6; 32 of 32..128, 16
-// heads, bf16 8.9 / 9.6; 256 of 512..2048, 8 heads, D 32 96 / 120.
-static bool wg_per_row(int64_t rows_heads, int64_t width, int D, int cus) {
+// heads, bf16 8.9 / 9.6, 96 of 512..2048 100 / 107; 256 of 512..2048, 8 heads, D 32
+// 96 / 120; 64 ragged ones of up to 8192, 32 heads, D 128, bf16 675 / 397.
+static bool wg_per_row(int64_t rows_heads, int64_t width, int D, int kv_dtype, int cus) {
   if (rows_heads <= cus) return true;
   if (rows_heads <= 2 * (int64_t)cus) return width > 128;
-  return rows_heads <= (D > 32 ? 4 : 3) * (int64_t)cus && width > 256;
+  if (rows_heads <= (D > 32 ? 4 : 3) * (int64_t)cus) return width > 256;
+  return (D > 64 || (D == 64 && kv_dtype == HS_DTYPE_F32)) && rows_heads < 16 * (int64_t)cus &&
+         width > 512;
 }
 
 // Grouped heads that the split-operand kernel does not take (fp32 caches, other
@@ -556,7 +559,7 @@ static int decode_common(const float* q, const void* k_cache, const void* v_cach
       a.part_tokens = rows_partition(B, H, Hkv, D, BS, MB, plan.part_tokens, cus);
       a.P = (int)ceil_div(width, a.part_tokens);
     } else if (num_splits == 1) {
-      a.wg = mha && wg_per_row((int64_t)B * H, width, D, cus);
+      a.wg = mha && wg_per_row((int64_t)B * H, width, D, kv_dtype, cus);
     } else if (num_splits > 1) {
       // Multi-head attention: workgroups of 8 waves, three for each CU, of at
       // least 256 keys, or 512 where that many fill a round of the device (1024

@@ -225,3 +225,14 @@ def test_one_pass_around_the_rules(H, D, batch):
         case = _case(ctxs, H, H, D, 16, torch.float16, seed=batch)
         bt = case[3][:, :-(-longest // 16)].contiguous()
         _runs((*case[:3], bt, *case[4:]), splits=(1,))
+
+
+@pytest.mark.parametrize("H,D,dtype,batch", [
+    (32, 128, torch.bfloat16, 32), (32, 128, torch.bfloat16, 33), (32, 128, torch.bfloat16, 128),
+    (16, 256, torch.float16, 66), (16, 64, torch.float32, 65), (16, 64, torch.float16, 65)])
+def test_one_pass_of_many_long_rows(H, D, dtype, batch):
+    """More than four rows a CU, up to sixteen, tables on both sides of 512 tokens."""
+    for longest in (496, 512):   # tables of 512 and 528 tokens
+        case = _case([longest] + [1 + (7 * i) % 40 for i in range(1, batch)], H, H, D, 16, dtype,
+                     seed=batch)
+        _runs(case, splits=(1,))
