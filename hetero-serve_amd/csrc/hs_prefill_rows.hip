@@ -118,19 +118,22 @@ __device__ inline void wave_lds_fence() {
 // Scheduling barrier mask: everything but matrix instructions may cross it.
 constexpr int kAllButProducts = 0x3F6;
 
-// The products of 4 dims or keys, summed.
-__device__ inline float4x product4(float a, float b) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, float4x{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+// acc plus the products of 4 dims or keys.
+__device__ inline float4x product4(float a, float b, float4x acc = float4x{0.0f, 0.0f, 0.0f, 0.0f}) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
 }
 
 // Dot products over the lane's 4 N dims (16 N in all) of NT row tiles, row
-// tiles `step` floats apart.  Each matrix instruction starts from zero and
-// the results are added as a tree: a row with few keys has the error of its
-// scores, and accumulating in the instructions, in chains of 16 to 64
-// products, it was up to 1.6 times that of the VALU kernel's chains of 4 or 8
-// and trees over the lanes (2-norm against fp64, head dim 128, 17 keys, bf16:
-// 1.79e-7, 1.12e-7 there, 1.12e-7 so).
-template <int N, int NT, bool kHold>
+// tiles `step` floats apart: chains of kChain matrix instructions (4 kChain
+// products), added as a tree.  A row with few keys has the error of its scores,
+// and in chains of 16 to 64 products it was up to 1.6 times that of the VALU
+// kernel's chains of 4 (fp32 caches) or 8 (16-bit ones) and trees over the lanes:
+// 2-norm against fp64, head dim 128, 17 keys, bf16, 1.79e-7, 1.12e-7 there, 1.07e-7
+// in chains of 8.  These cost head dim 64, bf16, 4% of its speed, chains of 4 22%.
+// kHold: the results of at most two groups of products at once, without which
+// an fp32 cache at head dim 64 takes 162 VGPRs and half the waves (15% slower;
+// with 16-bit caches, which fit either way, the barrier costs 3%).
+template <int N, int NT, int kChain, bool kHold>
 __device__ inline void dot_tree(const float* k, const float* q, int step, float4x (&s)[NT]) {
   if constexpr (N == 1) {
     const float4 kf = *reinterpret_cast<const float4*>(k);
@@ -141,10 +144,22 @@ __device__ inline void dot_tree(const float* k, const float* q, int step, float4
              (product4(kf.z, qf.z) + product4(kf.w, qf.w));
       if constexpr (kHold) __builtin_amdgcn_sched_barrier(kAllButProducts);
     }
+  } else if constexpr (N == kChain) {
+    const float4 k0 = *reinterpret_cast<const float4*>(k);
+    const float4 k1 = *reinterpret_cast<const float4*>(k + 4);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const float4 q0 = *reinterpret_cast<const float4*>(q + t * step);
+      const float4 q1 = *reinterpret_cast<const float4*>(q + t * step + 4);
+      s[t] = (product4(k1.x, q1.x, product4(k0.x, q0.x)) +
+              product4(k1.y, q1.y, product4(k0.y, q0.y))) +
+             (product4(k1.z, q1.z, product4(k0.z, q0.z)) +
+              product4(k1.w, q1.w, product4(k0.w, q0.w)));
+    }
   } else {
     float4x r[NT];
-    dot_tree<N / 2, NT, kHold>(k, q, step, s);
-    dot_tree<N / 2, NT, kHold>(k + 2 * N, q + 2 * N, step, r);
+    dot_tree<N / 2, NT, kChain, kHold>(k, q, step, s);
+    dot_tree<N / 2, NT, kChain, kHold>(k + 2 * N, q + 2 * N, step, r);
 #pragma unroll
     for (int t = 0; t < NT; ++t) s[t] += r[t];
   }
@@ -304,8 +319,8 @@ __device__ inline void rows_tile(const RowsArgs& ra, int b, int kvh, int tile, i
 
     // S^T: lane (j, g) gets keys 4 g + i of row j of each row tile.
     float4x s[NT];
-    dot_tree<D / 16, NT, sizeof(T) == 4 && D <= 64>(&ks[wv][j][g * (D / 4)], &qs[j][g * (D / 4)],
-                                                    kKeys * kRow, s);
+    dot_tree<D / 16, NT, (sizeof(T) == 2 && D > 32 ? 2 : 1), (sizeof(T) == 4 && D <= 64)>(
+        &ks[wv][j][g * (D / 4)], &qs[j][g * (D / 4)], kKeys * kRow, s);
     wave_lds_fence();
 
     const int t0 = lo + n * kKeys;
